@@ -1,0 +1,66 @@
+// Mixed-radix tile kernels for contiguous lines of 2^a 3^b 5^c 17^d points (mfft_mixed.hip).
+#pragma once
+#include "mfft_common.h"
+
+#include <vector>
+
+namespace mfft {
+
+constexpr int kMixThreads = 512;
+constexpr int kMixStages = 8;
+constexpr int kMixInline = 64;  // work-queue items that travel in the kernel's arguments
+
+// Stockham schedule of one line length, stage 0 first (the self-sorting order of the tile
+// kernels). cols = R / radix; s = product of the earlier radices; mul multiplies the stage's
+// outputs (scaling, and the 1/16 of the matrix-core operands).
+struct MixSched {
+    int R, nst;
+    int radix[kMixStages], cols[kMixStages], s[kMixStages];
+    float inv_cols[kMixStages], inv_s[kMixStages], mul[kMixStages];
+};
+
+// One launch of lines of one length: nlines dense lines of R points, T per tile.
+struct MixArgs {
+    const void *in;
+    void *out;
+    long long nlines;
+    const float2 *tw;      // W_R^e, e in [0, R), sign of the transform
+    const void *dft_ops;   // DftOps
+    int T, sign;
+    float w16[3];
+    MixSched sc;
+};
+
+// Work queue: an item is nlines dense lines of one registered length.
+struct MixLen {
+    const float2 *tw;
+    MixSched sc;
+};
+struct MixItem {
+    const void *in;
+    void *out;
+    long long nlines;
+    int len, T;            // index into the length table; lines per tile
+};
+struct MixQueueArgs {
+    const MixLen *lens;
+    const void *dft_ops;
+    const MixItem *items;      // more than kMixInline items: device arrays (else null)
+    const int *first;          // first tile of each item
+    unsigned *counter;         // {next tile, finished workgroups}, both 0 between launches
+    int nitems, total, sign, tw_at;  // tw_at: LDS word where a tile's twiddle table starts
+    float w16[3];
+    int first_in[kMixInline];
+    MixItem item_in[kMixInline];
+};
+
+// The radices of a length, stage order, as the kernels want them; false: not such a length.
+bool mix_radices(int n, std::vector<int> &out);
+// Schedule of a length for a precision (scale: every stage multiplies by 1/radix).
+bool mix_schedule(int n, int prec, bool scale, MixSched &sc);
+inline size_t mix_lds_bytes(int tile_points, int R) { return sizeof(float2) * ((size_t)tile_points + R); }
+
+const void *find_mixed_kernel(int prec, int in_fmt, int out_fmt);
+const void *find_mixed_queue_kernel(int prec, int in_fmt, int out_fmt);
+
+}  // namespace mfft

@@ -12,6 +12,7 @@
 #include "mfft_common.h"
 #include "mfft_fast.h"
 #include "mfft_internal.h"
+#include "mfft_mixed.h"
 #include "mfft_onchip.h"
 
 #include <hip/hip_ext.h>
@@ -203,7 +204,7 @@ struct PassSpec {
     bool small = false;   // streaming short-DFT kernel (R <= 16, one thread per line)
     float2 *stage_tw_s = nullptr, *tw_lo_s = nullptr;
     float last_mul = 1.f, tail_mul = 1.f;
-    long long max_grid = 0;  // persistent grid of the fast kernel
+    long long max_grid = 0;  // persistent grid of the fast kernel; tiles the mixed one wants
     int TL = 1, T = 1;
     int l0 = 0, l1 = -1, l2 = -1;  // indices into lines
     const void *fn = nullptr;
@@ -216,6 +217,8 @@ struct PassSpec {
     bool onchip = false;    // the whole 65536-point line in one pass (fft_onchip)
     bool onchip_cols = false;  // 2048-point lines, 32 per workgroup (fft_onchip_cols)
     bool onchip_rows = false;  // ... contiguous lines stored transposed (its rows kind)
+    bool mixed = false;     // dense contiguous lines on the mixed-radix kernel (fft_mixed)
+    MixSched mix{};
 };
 
 struct mfft_plan_s {
@@ -571,6 +574,30 @@ static int plan_reversed_1d(mfft_plan_s *p)
     return MFFT_OK;
 }
 
+// Whether a pass reads and writes whole contiguous lines that follow each other without gaps
+// (a level's stride is the extent of the levels below it), on both sides alike; the batch is
+// the outermost level, so that holds for any number of transforms.
+static bool dense_rows(const PassSpec &ps)
+{
+    if (ps.ps_in != 1 || ps.ps_out != 1) return false;
+    std::vector<Level> v = ps.lines;
+    std::sort(v.begin(), v.end(), [](const Level &a, const Level &b) { return a.in_stride < b.in_stride; });
+    long long stride = ps.R;
+    for (size_t i = 0; i < v.size(); ++i) {
+        if (v[i].in_stride != stride || v[i].out_stride != stride || (v[i].batch && i + 1 != v.size())) return false;
+        stride *= v[i].count;
+    }
+    return true;
+}
+
+// Lines per tile of the mixed-radix kernel: as many as kMaxTile points hold, fewer when the
+// launch would otherwise make fewer than `tiles` of them (two per compute unit).
+static int mixed_tile_lines(int R, long long nlines, long long tiles)
+{
+    const long long most = std::max(1, kMaxTile / R), want = nlines / tiles;
+    return (int)std::max(1LL, std::min(most, want));
+}
+
 // Choose tile geometry and kernel for every pass.
 static int finish_passes(mfft_plan_s *p)
 {
@@ -694,9 +721,24 @@ static int finish_passes(mfft_plan_s *p)
             }
         }
         if (ps.fast_kind < 0) ps.rev_fast = false;
+        if (ps.generic && !ps.small && ps.fast_kind < 0 && !rev && !ps.tw_N && dense_rows(ps)) {
+            const void *fn = find_mixed_kernel(p->d.precision, in_fmt, out_fmt);
+            if (fn && mix_schedule(ps.R, p->d.precision, p->d.scale == MFFT_SCALE_STAGE, ps.mix)) {
+                ps.mixed = true;
+                ps.fn = fn;
+                ps.radix.assign(ps.mix.radix, ps.mix.radix + ps.mix.nst);
+                long long nl = 1;
+                for (auto &l : ps.lines) nl *= l.count;
+                ps.max_grid = 2 * device_cus();
+                ps.T = mixed_tile_lines(ps.R, nl, ps.max_grid);
+                ps.TL = 1;
+                ps.l0 = 0;
+                HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix_lds_bytes(kMaxTile, kMaxTile)));
+            }
+        }
         if (rev && !ps.rev_fast && ps.perm_axis < 0)
             return fail(MFFT_ERR_UNSUPPORTED, "digit-reversed %d-point lines need the matrix-core kernels", ps.R);
-        if (ps.fast_kind >= 0 || ps.small) {
+        if (ps.fast_kind >= 0 || ps.small || ps.mixed) {
             // l0 chosen above
         } else if (!ps.generic) {
             ps.T = pow2_tile_lines(ps.R, ps.TL);
@@ -717,7 +759,7 @@ static int finish_passes(mfft_plan_s *p)
         ps.l2 = rest.size() > 1 ? rest[1] : -1;
         if (ps.tw_N && ps.tw_level != ps.l0 && ps.tw_level != ps.l1)
             return fail(MFFT_ERR_UNSUPPORTED, "twiddle level layout");
-        if (ps.fast_kind < 0 && !ps.small) {
+        if (ps.fast_kind < 0 && !ps.small && !ps.mixed) {
             ps.fn = (const void *)find_tile_kernel(p->d.precision, ps.R, ps.TL, ps.generic);
             if (!ps.fn) return fail(MFFT_ERR_UNSUPPORTED, "no kernel for R=%d TL=%d", ps.R, ps.TL);
         }
@@ -1020,6 +1062,27 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
                 HIP_TRY(hipExtLaunchKernel(ps.fn, grid, block, oargs, 0, s, kstart, kstop, 0));
             else
                 HIP_TRY(hipLaunchKernel(ps.fn, grid, block, oargs, 0, s));
+            continue;
+        }
+        if (ps.mixed) {
+            MixArgs m;
+            m.in = a.in;
+            m.out = a.out;
+            m.nlines = (long long)a.c0 * a.c1 * a.c2;
+            m.tw = ps.stage_tw;
+            m.dft_ops = p->ops;
+            m.T = mixed_tile_lines(ps.R, m.nlines, ps.max_grid);
+            m.sign = p->d.direction;
+            memcpy(m.w16, g_w16, sizeof m.w16);
+            m.sc = ps.mix;
+            const long long blocks = (m.nlines + m.T - 1) / m.T;
+            if (blocks >= (1LL << 31)) return fail(MFFT_ERR_UNSUPPORTED, "grid too large");
+            void *margs[] = {&m};
+            const size_t lds = mix_lds_bytes(m.T * ps.R, ps.R);
+            if (kstart || kstop)
+                HIP_TRY(hipExtLaunchKernel(ps.fn, dim3((unsigned)blocks), dim3(kMixThreads), margs, lds, s, kstart, kstop, 0));
+            else
+                HIP_TRY(hipLaunchKernel(ps.fn, dim3((unsigned)blocks), dim3(kMixThreads), margs, lds, s));
             continue;
         }
         if (ps.small) {
@@ -1384,11 +1447,18 @@ struct mfft_batcher_s {
     mfft_desc d{};
     int max_items = 0;
     DftOps *ops = nullptr;
-    std::vector<std::pair<int, float2 *>> tables;  // stage twiddles per length
+    std::vector<float2 *> tables;  // stage twiddles of the lengths seen so far
+    std::vector<float2 *> allocs;  // what holds them: one allocation per call that met new lengths
+    std::vector<short> index = std::vector<short>(kMaxTile + 1, -1);  // length -> tables
+    // the mixed-radix work-queue kernel, when it exists for the formats, and the schedules of
+    // the lengths (entry i belongs to tables[i])
+    const void *fn = nullptr;
+    MixLen *lens = nullptr;
     struct Slot {
         TileArgs *h_jobs = nullptr, *d_jobs = nullptr;
         long long *h_first = nullptr, *d_first = nullptr;
         unsigned long long *counter = nullptr;
+        MixItem *h_items = nullptr, *d_items = nullptr;  // max_items records, then their first tiles
         hipEvent_t done = nullptr;
         bool used = false;
     } slot[4];
@@ -1402,18 +1472,25 @@ int mfft_batcher_destroy(mfft_batcher b)
     if (!b) return MFFT_OK;
     (void)hipDeviceSynchronize();
     (void)hipFree(b->ops);
-    for (auto &t : b->tables) (void)hipFree(t.second);
+    (void)hipFree(b->lens);
+    for (float2 *t : b->allocs) (void)hipFree(t);
     for (auto &sl : b->slot) {
         (void)hipHostFree(sl.h_jobs);
         (void)hipHostFree(sl.h_first);
+        (void)hipHostFree(sl.h_items);
         (void)hipFree(sl.d_jobs);
         (void)hipFree(sl.d_first);
+        (void)hipFree(sl.d_items);
         (void)hipFree(sl.counter);
         if (sl.done) (void)hipEventDestroy(sl.done);
     }
     delete b;
     return MFFT_OK;
 }
+
+// Bytes of a slot's item records and first tiles; lengths 2^a 3^b 5^c 17^d up to kMaxTile: 195.
+static size_t mix_items_bytes(int max_items) { return (sizeof(MixItem) + sizeof(int)) * (size_t)max_items; }
+constexpr int kMixLengths = 256;
 
 int mfft_batcher_create(mfft_batcher *out, const mfft_desc *d, int max_items)
 {
@@ -1424,14 +1501,26 @@ int mfft_batcher_create(mfft_batcher *out, const mfft_desc *d, int max_items)
     mfft_batcher b = new mfft_batcher_s;
     b->d = *d;
     b->max_items = max_items;
+    b->fn = find_mixed_queue_kernel(d->precision, d->in_fmt, d->out_fmt);
     hipError_t e = hipMalloc((void **)&b->ops, sizeof(DftOps));
     if (e == hipSuccess) e = gen_dft_ops(b->ops, d->direction, 0);
+    if (b->fn) {
+        if (e == hipSuccess) e = hipMalloc((void **)&b->lens, sizeof(MixLen) * kMixLengths);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(b->fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix_lds_bytes(kMaxTile, kMaxTile));
+    }
     for (auto &sl : b->slot) {
-        if (e == hipSuccess) e = hipHostMalloc((void **)&sl.h_jobs, sizeof(TileArgs) * max_items, hipHostMallocDefault);
-        if (e == hipSuccess) e = hipHostMalloc((void **)&sl.h_first, sizeof(long long) * (max_items + 1), hipHostMallocDefault);
-        if (e == hipSuccess) e = hipMalloc((void **)&sl.d_jobs, sizeof(TileArgs) * max_items);
-        if (e == hipSuccess) e = hipMalloc((void **)&sl.d_first, sizeof(long long) * (max_items + 1));
+        if (b->fn) {
+            if (e == hipSuccess) e = hipHostMalloc((void **)&sl.h_items, mix_items_bytes(max_items), hipHostMallocDefault);
+            if (e == hipSuccess) e = hipMalloc((void **)&sl.d_items, mix_items_bytes(max_items));
+        } else {
+            if (e == hipSuccess) e = hipHostMalloc((void **)&sl.h_jobs, sizeof(TileArgs) * max_items, hipHostMallocDefault);
+            if (e == hipSuccess) e = hipHostMalloc((void **)&sl.h_first, sizeof(long long) * (max_items + 1), hipHostMallocDefault);
+            if (e == hipSuccess) e = hipMalloc((void **)&sl.d_jobs, sizeof(TileArgs) * max_items);
+            if (e == hipSuccess) e = hipMalloc((void **)&sl.d_first, sizeof(long long) * (max_items + 1));
+        }
         if (e == hipSuccess) e = hipMalloc((void **)&sl.counter, sizeof(unsigned long long));
+        if (e == hipSuccess) e = hipMemset(sl.counter, 0, sizeof(unsigned long long));
         if (e == hipSuccess) e = hipEventCreateWithFlags(&sl.done, hipEventDisableTiming);
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -1439,23 +1528,133 @@ int mfft_batcher_create(mfft_batcher *out, const mfft_desc *d, int max_items)
         mfft_batcher_destroy(b);
         return fail(MFFT_ERR_HIP, "batcher: %s", hipGetErrorString(e));
     }
-    b->grid = queue_grid(d->precision);
+    // the mixed-radix queue: up to four workgroups per compute unit take tiles from the counter
+    b->grid = b->fn ? (int)(4 * device_cus()) : queue_grid(d->precision);
     *out = b;
     return MFFT_OK;
 }
 
-static float2 *batch_table(mfft_batcher b, int n, hipStream_t s)
+// Makes the tables (and entries of b->lens) of the items' lengths that are new to the batcher:
+// generated together on the null stream and waited for once, so any stream may use them after.
+static int batch_tables(mfft_batcher b, const mfft_batch_item *items, int nitems)
 {
-    for (auto &t : b->tables)
-        if (t.first == n) return t.second;
+    std::vector<int> fresh;
+    size_t words = 0;
+    for (int i = 0; i < nitems; ++i)
+        if (b->index[items[i].n] == -1) {
+            b->index[items[i].n] = -2;  // seen in this call
+            fresh.push_back(items[i].n);
+            words += items[i].n;
+        }
+    if (fresh.empty()) return MFFT_OK;
+    auto undo = [&](int code, const char *what, hipError_t e) {
+        for (int n : fresh) b->index[n] = -1;
+        return fail(code, "%s: %s", what, hipGetErrorString(e));
+    };
+    std::vector<MixLen> len(fresh.size());
+    const size_t have = b->tables.size();
     float2 *tab = nullptr;
-    if (hipMalloc((void **)&tab, sizeof(float2) * n) != hipSuccess) return nullptr;
-    // generated once on the null stream and waited for, so any stream may use it after
-    (void)s;
-    if (gen_twiddle(tab, n, n, 1, b->d.direction, 0) != hipSuccess) return nullptr;
-    if (hipStreamSynchronize(0) != hipSuccess) return nullptr;
-    b->tables.push_back({n, tab});
-    return tab;
+    hipError_t e = hipMalloc((void **)&tab, sizeof(float2) * words);
+    if (e != hipSuccess) return undo(MFFT_ERR_NOMEM, "twiddle tables", e);
+    float2 *t = tab;
+    for (size_t i = 0; i < fresh.size() && e == hipSuccess; ++i) {
+        len[i].tw = t;
+        if (b->fn && (have + i >= kMixLengths ||
+                      !mix_schedule(fresh[i], b->d.precision, b->d.scale == MFFT_SCALE_STAGE, len[i].sc)))
+            e = hipErrorInvalidValue;
+        else
+            e = gen_twiddle(t, fresh[i], fresh[i], 1, b->d.direction, 0);
+        t += fresh[i];
+    }
+    if (e == hipSuccess && b->fn)
+        e = hipMemcpyAsync(b->lens + have, len.data(), sizeof(MixLen) * len.size(), hipMemcpyHostToDevice, 0);
+    const hipError_t e2 = hipStreamSynchronize(0);
+    if (e == hipSuccess) e = e2;
+    if (e != hipSuccess) {
+        (void)hipFree(tab);
+        return undo(MFFT_ERR_HIP, "twiddle tables", e);
+    }
+    b->allocs.push_back(tab);
+    for (size_t i = 0; i < fresh.size(); ++i) {
+        b->index[fresh[i]] = (short)b->tables.size();
+        b->tables.push_back(const_cast<float2 *>(len[i].tw));
+    }
+    return MFFT_OK;
+}
+
+// The next slot, once its previous launch has read its records.
+static int batch_slot(mfft_batcher b, mfft_batcher_s::Slot **out)
+{
+    auto &sl = b->slot[b->next];
+    if (sl.used) HIP_TRY(hipEventSynchronize(sl.done));
+    b->next = (b->next + 1) % 4;
+    *out = &sl;
+    return MFFT_OK;
+}
+
+// The mixed-radix work queue. Up to kMixInline items travel in the kernel's arguments, and a
+// launch whose tiles fit the grid hands out no further ones: such a call is one launch, with no
+// copy, counter or slot.
+static int batch_exec_mixed(mfft_batcher b, const mfft_batch_item *items, int nitems, hipStream_t s)
+{
+    long long points = 0;
+    for (int i = 0; i < nitems; ++i) points += items[i].count * items[i].n;
+    // points per tile: kMaxTile, less when that would leave compute units without a tile
+    const long long cap = std::min<long long>(kMaxTile, std::max<long long>(kMixThreads, points / (2 * device_cus())));
+    MixQueueArgs q;
+    q.lens = b->lens;
+    q.dft_ops = b->ops;
+    q.items = nullptr;
+    q.first = nullptr;
+    q.counter = nullptr;
+    q.nitems = nitems;
+    q.sign = b->d.direction;
+    memcpy(q.w16, g_w16, sizeof q.w16);
+    mfft_batcher_s::Slot *sl = nullptr;
+    MixItem *rec = q.item_in;
+    int *first = q.first_in;
+    if (nitems > kMixInline) {
+        int rc = batch_slot(b, &sl);
+        if (rc) return rc;
+        rec = sl->h_items;
+        first = (int *)(sl->h_items + b->max_items);
+    }
+    long long total = 0;
+    int most = 0, longest = 0;
+    for (int i = 0; i < nitems; ++i) {
+        const mfft_batch_item &it = items[i];
+        MixItem &m = rec[i];
+        m.in = it.in;
+        m.out = it.out;
+        m.nlines = it.count;
+        m.len = b->index[it.n];
+        m.T = (int)std::max<long long>(1, std::min<long long>(it.count, cap / it.n));
+        first[i] = (int)total;
+        total += (it.count + m.T - 1) / m.T;
+        if (total >= (1LL << 31)) return fail(MFFT_ERR_UNSUPPORTED, "%lld tiles in one launch", total);
+        most = std::max(most, m.T * it.n);
+        longest = std::max(longest, it.n);
+    }
+    q.total = (int)total;
+    q.tw_at = (most + 1) & ~1;
+    const int grid = (int)std::min<long long>(b->grid, total);
+    if (total > grid && !sl) {
+        int rc = batch_slot(b, &sl);
+        if (rc) return rc;
+    }
+    if (sl) q.counter = (unsigned *)sl->counter;
+    if (nitems > kMixInline) {
+        HIP_TRY(hipMemcpyAsync(sl->d_items, sl->h_items, mix_items_bytes(b->max_items), hipMemcpyHostToDevice, s));
+        q.items = sl->d_items;
+        q.first = (const int *)(sl->d_items + b->max_items);
+    }
+    void *args[] = {&q};
+    HIP_TRY(hipLaunchKernel(b->fn, dim3((unsigned)grid), dim3(kMixThreads), args, mix_lds_bytes(q.tw_at, longest), s));
+    if (sl) {
+        HIP_TRY(hipEventRecord(sl->done, s));
+        sl->used = true;
+    }
+    return MFFT_OK;
 }
 
 int mfft_batcher_exec(mfft_batcher b, const mfft_batch_item *items, int nitems, void *stream)
@@ -1465,17 +1664,35 @@ int mfft_batcher_exec(mfft_batcher b, const mfft_batch_item *items, int nitems, 
     if (nitems == 0) return MFFT_OK;
     std::lock_guard<std::mutex> lk(b->mu);
     hipStream_t s = (hipStream_t)stream;
-    auto &sl = b->slot[b->next];
-    b->next = (b->next + 1) % 4;
-    if (sl.used) HIP_TRY(hipEventSynchronize(sl.done));  // the slot's previous launch has read its jobs
-    long long total = 0;
     for (int i = 0; i < nitems; ++i) {
         const mfft_batch_item &it = items[i];
         std::vector<int> rad;
         if (it.n < 2 || it.n > kMaxTile || !line_radices(it.n, rad) || it.count < 1 || !it.in || !it.out)
             return fail(MFFT_ERR_INVALID, "item %d: n=%d count=%lld", i, it.n, (long long)it.count);
-        float2 *tab = batch_table(b, it.n, s);
-        if (!tab) return fail(MFFT_ERR_NOMEM, "twiddle table");
+    }
+    int rc = batch_tables(b, items, nitems);
+    if (rc) return rc;
+    if (trace_active()) {
+        // one record for the call
+        long long rd = 0, wr = 0;
+        for (int i = 0; i < nitems; ++i) {
+            rd += items[i].count * items[i].n * (long long)fmt_bytes(b->d.in_fmt);
+            wr += items[i].count * items[i].n * (long long)fmt_bytes(b->d.out_fmt);
+        }
+        char name[64];
+        snprintf(name, sizeof name, "queue %d items %s>%s", nitems, fmt_name(b->d.in_fmt), fmt_name(b->d.out_fmt));
+        trace_launch(s, name, rd, wr);
+    }
+    if (b->fn) return batch_exec_mixed(b, items, nitems, s);
+    mfft_batcher_s::Slot *slp = nullptr;
+    rc = batch_slot(b, &slp);
+    if (rc) return rc;
+    auto &sl = *slp;
+    long long total = 0;
+    for (int i = 0; i < nitems; ++i) {
+        const mfft_batch_item &it = items[i];
+        std::vector<int> rad;
+        line_radices(it.n, rad);
         TileArgs &a = sl.h_jobs[i];
         memset(&a, 0, sizeof a);
         a.in = it.in;
@@ -1494,7 +1711,7 @@ int mfft_batcher_exec(mfft_batcher b, const mfft_batch_item *items, int nitems, 
         a.c1 = a.c2 = 1;
         a.in_s0 = a.out_s0 = it.n;
         a.in_ps = a.out_ps = 1;
-        a.stage_tw = tab;
+        a.stage_tw = b->tables[b->index[it.n]];
         a.dft_ops = b->ops;
         a.out_mul = 1.0f;
         a.sign = b->d.direction;
@@ -1508,17 +1725,6 @@ int mfft_batcher_exec(mfft_batcher b, const mfft_batch_item *items, int nitems, 
     HIP_TRY(hipMemcpyAsync(sl.d_jobs, sl.h_jobs, sizeof(TileArgs) * nitems, hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(sl.d_first, sl.h_first, sizeof(long long) * (nitems + 1), hipMemcpyHostToDevice, s));
     int grid = (int)std::min<long long>(b->grid, total);
-    if (trace_active()) {
-        // one record for the counter reset and the work-queue kernel
-        long long rd = 0, wr = 0;
-        for (int i = 0; i < nitems; ++i) {
-            rd += items[i].count * items[i].n * (long long)fmt_bytes(b->d.in_fmt);
-            wr += items[i].count * items[i].n * (long long)fmt_bytes(b->d.out_fmt);
-        }
-        char name[64];
-        snprintf(name, sizeof name, "queue %d items %s>%s", nitems, fmt_name(b->d.in_fmt), fmt_name(b->d.out_fmt));
-        trace_launch(s, name, rd, wr);
-    }
     HIP_TRY(launch_queue(b->d.precision, sl.d_jobs, sl.d_first, nitems, total, sl.counter, grid, s));
     HIP_TRY(hipEventRecord(sl.done, s));
     sl.used = true;

@@ -6,7 +6,7 @@
 // every load is coalesced), transforms them in fp32 registers, applies the four-step
 // twiddle and the stage scale, and stores -- no LDS, one HBM pass. A thread reads and
 // writes the same R positions, so the pass may run in place.
-#include "mfft_common.h"
+#include "mfft_butterfly.h"
 
 namespace mfft {
 namespace small {
@@ -140,42 +140,14 @@ __device__ __forceinline__ void dft(float2 *v, int sg, const float *w16)
     }
 }
 
-// Odd R: y_k = x_0 + sum_j S_j c_jk + i sum_j D_j t_jk and y_{R-k} = x_0 + sum_j S_j c_jk -
-// i sum_j D_j t_jk (j, k = 1..(R-1)/2), with S_j = x_j + x_{R-j}, D_j = x_j - x_{R-j} and
-// W_R^m = c_m + i t_m from the pass table (FP64-generated, carries the transform's sign):
-// (R-1)^2 real multiply-adds per line instead of 4 (R-1)^2.
+// Odd R, W_R^m from the pass table.
 template <int R>
 __device__ __forceinline__ void dft_odd(float2 *v, const float2 *__restrict__ tab)
 {
-    constexpr int H = (R - 1) / 2;
     float2 w[R];
 #pragma unroll
     for (int m = 0; m < R; ++m) w[m] = tab[m];
-    float2 S[H + 1], D[H + 1];
-#pragma unroll
-    for (int j = 1; j <= H; ++j) {
-        S[j] = make_float2(v[j].x + v[R - j].x, v[j].y + v[R - j].y);
-        D[j] = make_float2(v[j].x - v[R - j].x, v[j].y - v[R - j].y);
-    }
-    float2 y0 = v[0];
-#pragma unroll
-    for (int j = 1; j <= H; ++j) y0 = make_float2(y0.x + S[j].x, y0.y + S[j].y);
-#pragma unroll
-    for (int k = 1; k <= H; ++k) {
-        float2 a = v[0], b = make_float2(0.f, 0.f);
-#pragma unroll
-        for (int j = 1; j <= H; ++j) {
-            const float2 t = w[(j * k) % R];
-            a.x += S[j].x * t.x;
-            a.y += S[j].y * t.x;
-            b.x += D[j].x * t.y;
-            b.y += D[j].y * t.y;
-        }
-        // i * b = (-b.y, b.x)
-        v[k] = make_float2(a.x - b.y, a.y + b.x);
-        v[R - k] = make_float2(a.x + b.y, a.y - b.x);
-    }
-    v[0] = y0;
+    dft_odd_w<R>(v, w);
 }
 
 // Stage scale, four-step twiddle W_N^(mult k) and store of one line. W_N^mult comes from
