@@ -224,8 +224,7 @@ int mfft_conv2d_create(mfft_conv2d *out, const mfft_conv2d_desc *d)
     // fp16 pass boundaries with fp32 ends: the intermediates the passes keep in the output
     // buffer are fp16 as well (the image transforms then never run in place)
     auto create = [&](mfft_plan *pl, int64_t b) {
-        return op->mid16 ? mfft::plan_create_2d_out_mid(pl, op->Ph, op->Pw, b, &fd)
-                         : mfft_plan_create_2d(pl, op->Ph, op->Pw, b, &fd);
+        return mfft::plan_create_2d_conv(pl, op->Ph, op->Pw, b, &fd, op->mid16);
     };
     int rc = create(&op->fwd_img, op->pairs * d->channels);
     if (!rc) {
@@ -243,7 +242,7 @@ int mfft_conv2d_create(mfft_conv2d *out, const mfft_conv2d_desc *d)
         fd.direction = MFFT_FORWARD;
         fd.in_fmt = fd.out_fmt = MFFT_FMT_C32;
         fd.mid_fmt = -1;
-        rc = mfft_plan_create_2d(&op->fwd_filt, op->Ph, op->Pw, (int64_t)d->filters * d->channels, &fd);
+        rc = mfft::plan_create_2d_conv(&op->fwd_filt, op->Ph, op->Pw, (int64_t)d->filters * d->channels, &fd);
     }
     if (rc) {
         std::string m = mfft_last_error();
@@ -454,11 +453,11 @@ static int backward_setup(mfft_conv2d op)
     fd.in_fmt = fd.out_fmt = MFFT_FMT_C32;
     fd.workspace_limit = d.workspace_limit;
     fd.scale = MFFT_SCALE_STAGE;
-    int rc = mfft_plan_create_2d(&op->fwd_delta, op->Ph, op->Pw, op->pairs * d.filters, &fd);
+    int rc = mfft::plan_create_2d_conv(&op->fwd_delta, op->Ph, op->Pw, op->pairs * d.filters, &fd);
     fd.scale = MFFT_SCALE_NONE;
     fd.direction = MFFT_INVERSE;
-    if (!rc) rc = mfft_plan_create_2d(&op->inv_fc, op->Ph, op->Pw, (int64_t)d.filters * d.channels, &fd);
-    if (!rc) rc = mfft_plan_create_2d(&op->inv_pc, op->Ph, op->Pw, op->pairs * d.channels, &fd);
+    if (!rc) rc = mfft::plan_create_2d_conv(&op->inv_fc, op->Ph, op->Pw, (int64_t)d.filters * d.channels, &fd);
+    if (!rc) rc = mfft::plan_create_2d_conv(&op->inv_pc, op->Ph, op->Pw, op->pairs * d.channels, &fd);
     if (!rc && hipMalloc(&op->G, (size_t)d.filters * d.channels * op->Ph * op->Pw * 8) != hipSuccess) rc = MFFT_ERR_NOMEM;
     if (rc) {
         std::string m = mfft_last_error();

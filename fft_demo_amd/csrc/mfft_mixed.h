@@ -7,6 +7,8 @@
 namespace mfft {
 
 constexpr int kMixThreads = 512;
+constexpr int kMixColSmall = 8192, kMixColLarge = 17408;  // points per tile of the strided kernels
+constexpr int mix_col_threads(int cap) { return cap == kMixColSmall ? 512 : 1024; }
 constexpr int kMixStages = 8;
 constexpr int kMixInline = 64;  // work-queue items that travel in the kernel's arguments
 
@@ -16,7 +18,7 @@ constexpr int kMixInline = 64;  // work-queue items that travel in the kernel's 
 struct MixSched {
     int R, nst;
     int radix[kMixStages], cols[kMixStages], s[kMixStages];
-    float inv_cols[kMixStages], inv_s[kMixStages], mul[kMixStages];
+    float mul[kMixStages];
 };
 
 // One launch of lines of one length: nlines dense lines of R points, T per tile.
@@ -27,6 +29,20 @@ struct MixArgs {
     const float2 *tw;      // W_R^e, e in [0, R), sign of the transform
     const void *dft_ops;   // DftOps
     int T, sign;
+    float w16[3];
+    MixSched sc;
+};
+
+// One launch of strided lines of one length (the columns of 2D transforms): transforms of c0
+// adjacent lines each, T lines per tile (tiles0 tiles per transform).
+struct MixColArgs {
+    const void *in;
+    void *out;
+    const float2 *tw;
+    const void *dft_ops;
+    int T, sign, c0, tiles0;
+    int ps_in, ps_out;           // elements between a line's points
+    long long in_dist, out_dist; // elements between transforms
     float w16[3];
     MixSched sc;
 };
@@ -60,7 +76,8 @@ bool mix_radices(int n, std::vector<int> &out);
 bool mix_schedule(int n, int prec, bool scale, MixSched &sc);
 inline size_t mix_lds_bytes(int tile_points, int R) { return sizeof(float2) * ((size_t)tile_points + R); }
 
-const void *find_mixed_kernel(int prec, int in_fmt, int out_fmt);
+// cap: 0 = contiguous lines, kMixColSmall or kMixColLarge = strided lines
+const void *find_mixed_kernel(int prec, int in_fmt, int out_fmt, int cap = 0);
 const void *find_mixed_queue_kernel(int prec, int in_fmt, int out_fmt);
 
 }  // namespace mfft

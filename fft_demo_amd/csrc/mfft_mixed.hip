@@ -12,42 +12,50 @@
 
 namespace mfft {
 
+constexpr int kMixQueue = -1;
+
 template <int PREC, int INF, int OUTF>
-static const void *pick_mixed(bool queue)
+static const void *pick_mixed(int what)
 {
-    return queue ? (const void *)mixed::fft_mixed_queue<PREC, INF, OUTF> : (const void *)mixed::fft_mixed<PREC, INF, OUTF>;
+    switch (what) {
+    case 0: return (const void *)mixed::fft_mixed<PREC, INF, OUTF>;
+    case kMixQueue: return (const void *)mixed::fft_mixed_queue<PREC, INF, OUTF>;
+    case kMixColSmall: return (const void *)mixed::fft_mixed_cols<kMixColSmall, PREC, INF, OUTF>;
+    case kMixColLarge: return (const void *)mixed::fft_mixed_cols<kMixColLarge, PREC, INF, OUTF>;
+    default: return nullptr;
+    }
 }
 
 #if MFFT_PART == 1
-const void *find_mixed_split32(int inf, int outf, bool queue)
+const void *find_mixed_split32(int inf, int outf, int what)
 {
-    if (inf == FMT_C16 && outf == FMT_C32) return pick_mixed<PREC_SPLIT, FMT_C16, FMT_C32>(queue);
-    if (inf == FMT_C32 && outf == FMT_C16) return pick_mixed<PREC_SPLIT, FMT_C32, FMT_C16>(queue);
-    if (inf == FMT_C32 && outf == FMT_C32) return pick_mixed<PREC_SPLIT, FMT_C32, FMT_C32>(queue);
+    if (inf == FMT_C16 && outf == FMT_C32) return pick_mixed<PREC_SPLIT, FMT_C16, FMT_C32>(what);
+    if (inf == FMT_C32 && outf == FMT_C16) return pick_mixed<PREC_SPLIT, FMT_C32, FMT_C16>(what);
+    if (inf == FMT_C32 && outf == FMT_C32) return pick_mixed<PREC_SPLIT, FMT_C32, FMT_C32>(what);
     return nullptr;
 }
 #elif MFFT_PART == 2
-const void *find_mixed_plain(int prec, int inf, int outf, bool queue)
+const void *find_mixed_plain(int prec, int inf, int outf, int what)
 {
-    if (prec == PREC_FP16 && inf == FMT_C16 && outf == FMT_C16) return pick_mixed<PREC_FP16, FMT_C16, FMT_C16>(queue);
+    if (prec == PREC_FP16 && inf == FMT_C16 && outf == FMT_C16) return pick_mixed<PREC_FP16, FMT_C16, FMT_C16>(what);
     if (prec == PREC_BF16 && inf == FMT_CBF16 && outf == FMT_CBF16)
-        return pick_mixed<PREC_BF16, FMT_CBF16, FMT_CBF16>(queue);
-    if (prec == PREC_FP32 && inf == FMT_C32 && outf == FMT_C32) return pick_mixed<PREC_FP32, FMT_C32, FMT_C32>(queue);
+        return pick_mixed<PREC_BF16, FMT_CBF16, FMT_CBF16>(what);
+    if (prec == PREC_FP32 && inf == FMT_C32 && outf == FMT_C32) return pick_mixed<PREC_FP32, FMT_C32, FMT_C32>(what);
     return nullptr;
 }
 #else
-const void *find_mixed_split32(int inf, int outf, bool queue);
-const void *find_mixed_plain(int prec, int inf, int outf, bool queue);
+const void *find_mixed_split32(int inf, int outf, int what);
+const void *find_mixed_plain(int prec, int inf, int outf, int what);
 
-static const void *find_mixed(int prec, int inf, int outf, bool queue)
+static const void *find_mixed(int prec, int inf, int outf, int what)
 {
-    if (prec != PREC_SPLIT) return find_mixed_plain(prec, inf, outf, queue);
-    if (inf == FMT_C16 && outf == FMT_C16) return pick_mixed<PREC_SPLIT, FMT_C16, FMT_C16>(queue);
-    return find_mixed_split32(inf, outf, queue);
+    if (prec != PREC_SPLIT) return find_mixed_plain(prec, inf, outf, what);
+    if (inf == FMT_C16 && outf == FMT_C16) return pick_mixed<PREC_SPLIT, FMT_C16, FMT_C16>(what);
+    return find_mixed_split32(inf, outf, what);
 }
 
-const void *find_mixed_kernel(int prec, int inf, int outf) { return find_mixed(prec, inf, outf, false); }
-const void *find_mixed_queue_kernel(int prec, int inf, int outf) { return find_mixed(prec, inf, outf, true); }
+const void *find_mixed_kernel(int prec, int inf, int outf, int cap) { return find_mixed(prec, inf, outf, cap); }
+const void *find_mixed_queue_kernel(int prec, int inf, int outf) { return find_mixed(prec, inf, outf, kMixQueue); }
 
 // Radices of n with the least sum of stage costs: a stage costs an LDS round trip of every
 // point (about 20 issue slots a point) plus its butterfly. 16 is the matrix-core stage; 6, 10,
@@ -113,8 +121,6 @@ bool mix_schedule(int n, int prec, bool scale, MixSched &sc)
         sc.radix[i] = r[i];
         sc.cols[i] = n / r[i];
         sc.s[i] = s;
-        sc.inv_cols[i] = 1.0f / sc.cols[i];
-        sc.inv_s[i] = 1.0f / s;
         sc.mul[i] = mfma ? (scale ? 1.f / 256 : 1.f / 16) : 1.f;  // the operands carry a factor 16
         if (scale && !mfma) valu /= r[i];
         s *= r[i];

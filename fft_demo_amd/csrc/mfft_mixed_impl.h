@@ -28,25 +28,37 @@ using fast::b8;
 using fast::u4;
 
 enum Role { FIRST = 0, MID = 1, LAST = 2 };
-constexpr int NT = kMixThreads;
 
-// What the stages of one tile share. data: nl lines of R points (dense); tw: the stage
-// twiddles, both in LDS; gtw: the same table in global memory (uniform reads: the constants
-// of the odd butterflies, which then sit in scalar registers).
+// Geometry of a kernel: threads per workgroup and the points its tiles hold at most.
+// Contiguous lines lie one after the other in LDS. Strided lines (columns) lie interleaved,
+// point by point: the tile is then one Stockham array whose innermost factor is the line.
+template <bool COLS_, int NT_, int CAP_>
+struct Geo {
+    static constexpr bool COLS = COLS_;
+    static constexpr int NT = NT_, CAP = CAP_;
+};
+
+// What the stages of one tile share. data: nl lines of R points; tw: the stage twiddles, both
+// in LDS; gtw: the same table in global memory (uniform reads: the constants of the odd
+// butterflies, which then sit in scalar registers). in, out: the tile's first element;
+// ps_in, ps_out: bytes between a strided line's points.
 struct Ctx {
     float2 *data;
     const float2 *tw;
     const float2 *gtw;
-    const void *in;
-    void *out;
+    const void *dft_ops;
+    const char *in;
+    char *out;
     int R, nl, sign;
+    unsigned ps_in, ps_out;
     const float *w16;
     int tid;
 };
 
-// x / d for 0 <= x < 2^20 with inv = 1.0f / d: x + 0.5 is at least 0.5 / d away from the next
-// integer multiple, more than the product's rounding.
+// x / d for 0 <= x < 2^17 with inv = 1 / d to an ulp or two: x + 0.5 is at least 0.5 / d away
+// from the next multiple, more than the product's error.
 __device__ __forceinline__ int fdiv(int x, float inv) { return (int)(((float)x + 0.5f) * inv); }
+__device__ __forceinline__ float recip(int d) { return __builtin_amdgcn_rcpf((float)d); }
 
 // W_N^m, m < N, from the table of W_R (N divides R): one scalar load each.
 template <int N>
@@ -108,15 +120,57 @@ struct Split {
     static constexpr int B = r / A;
 };
 
-// One radix-r stage on the vector ALUs. An item is one r-point butterfly: line t, column col.
-template <int r, int ROLE, int INF, int OUTF>
-__device__ __forceinline__ void vstage(const Ctx &c, int cols, int s, float inv_cols, float inv_s, float mul)
+// Where the columns of a stage lie. A column is r points, the stage's butterfly; item I is a
+// (line, column) pair, columns fastest for contiguous lines, lines fastest for strided ones.
+// In LDS point j of item I is at lds(I) + j * pitch.
+template <class G>
+struct Cols {
+    int n, pitch, mul;   // items; elements between a column's points; elements per point step
+    int cols;
+    float inv;
+    __device__ __forceinline__ Cols(const Ctx &c, int cols_)
+    {
+        cols = cols_;
+        n = c.nl * cols;
+        mul = G::COLS ? c.nl : 1;
+        pitch = cols * mul;
+        inv = recip(G::COLS ? c.nl : cols);
+    }
+    // item -> first point's LDS element and column
+    __device__ __forceinline__ void at(const Ctx &c, int I, int &e, int &col, int &t) const
+    {
+        if constexpr (G::COLS) {
+            col = fdiv(I, inv);
+            t = I - col * c.nl;
+            e = I;
+        } else {
+            t = fdiv(I, inv);
+            col = I - t * cols;
+            e = t * c.R + col;
+        }
+    }
+    // byte offset of an item's point 0 on the input or output side, and the step between points
+    template <int EB>
+    __device__ __forceinline__ unsigned goff(int e, int col, int t, unsigned ps) const
+    {
+        return G::COLS ? (unsigned)t * EB + (unsigned)col * ps : (unsigned)e * EB;
+    }
+    template <int EB>
+    __device__ __forceinline__ unsigned gstep(unsigned ps) const
+    {
+        return G::COLS ? (unsigned)cols * ps : (unsigned)cols * EB;
+    }
+};
+
+// One radix-r stage on the vector ALUs.
+template <class G, int r, int ROLE, int INF, int OUTF>
+__device__ __forceinline__ void vstage(const Ctx &c, int ncols, int s, float mul)
 {
     typedef typename Elem<INF>::raw iraw;
     typedef typename Elem<OUTF>::raw oraw;
-    constexpr int MAXI = (kMaxTile + r * NT - 1) / (r * NT);
+    constexpr int NT = G::NT, MAXI = (G::CAP + r * NT - 1) / (r * NT);
     constexpr int A = Split<r>::A, B = Split<r>::B;
-    const int items = c.nl * cols;
+    const Cols<G> K(c, ncols);
     float2 w1[A > 1 ? A : 1], w2[B];
     if constexpr (r > 1) {
         if constexpr (A == 3) root_table<A>(c, w1);
@@ -124,28 +178,29 @@ __device__ __forceinline__ void vstage(const Ctx &c, int cols, int s, float inv_
     }
     iraw rw[ROLE == FIRST ? MAXI : 1][r];
     float2 v[MAXI][r];
-    int at[MAXI], p[MAXI];  // element of the item's first point, line * R + col; column
+    int e[MAXI], col[MAXI], t[MAXI];
 #pragma unroll
     for (int k = 0; k < MAXI; ++k) {
         const int I = c.tid + k * NT;
-        const int t = fdiv(I, inv_cols);
-        p[k] = I - t * cols;
-        at[k] = t * c.R + p[k];
-        if (I < items) {
+        K.at(c, I, e[k], col[k], t[k]);
+        if (I < K.n) {
             if constexpr (ROLE == FIRST) {
+                const unsigned o = K.template goff<sizeof(iraw)>(e[k], col[k], t[k], c.ps_in);
+                const unsigned st = K.template gstep<sizeof(iraw)>(c.ps_in);
 #pragma unroll
-                for (int j = 0; j < r; ++j) rw[k][j] = reinterpret_cast<const iraw *>(c.in)[(unsigned)(at[k] + j * cols)];
+                for (int j = 0; j < r; ++j) rw[k][j] = *reinterpret_cast<const iraw *>(c.in + (o + j * st));
             } else {
 #pragma unroll
-                for (int j = 0; j < r; ++j) v[k][j] = c.data[at[k] + j * cols];
+                for (int j = 0; j < r; ++j) v[k][j] = c.data[e[k] + j * K.pitch];
             }
         }
     }
     if constexpr (ROLE == MID) __syncthreads();  // every read of the tile precedes its writes
+    const int sm = s * K.mul;
+    const float inv_s = ROLE == MID ? recip(sm) : 0.f;
 #pragma unroll
     for (int k = 0; k < MAXI; ++k) {
-        const int I = c.tid + k * NT;
-        if (I >= items) continue;
+        if (c.tid + k * NT >= K.n) continue;
         if constexpr (ROLE == FIRST) {
 #pragma unroll
             for (int j = 0; j < r; ++j) v[k][j] = Elem<INF>::f(rw[k][j]);
@@ -157,82 +212,78 @@ __device__ __forceinline__ void vstage(const Ctx &c, int cols, int s, float inv_
                 dft_n<r>(v[k], w2, c.sign, c.w16);
         }
         if constexpr (ROLE == LAST) {
-            oraw *dst = reinterpret_cast<oraw *>(c.out);
+            const unsigned o = K.template goff<sizeof(oraw)>(e[k], col[k], t[k], c.ps_out);
+            const unsigned st = K.template gstep<sizeof(oraw)>(c.ps_out);
 #pragma unroll
             for (int j = 0; j < r; ++j)
-                dst[(unsigned)(at[k] + j * cols)] = Elem<OUTF>::pack(make_float2(v[k][j].x * mul, v[k][j].y * mul));
+                *reinterpret_cast<oraw *>(c.out + (o + j * st)) =
+                    Elem<OUTF>::pack(make_float2(v[k][j].x * mul, v[k][j].y * mul));
         } else {
             // output j of column q + s p goes to q + s (r p + j), times W_R^(s p j)
-            int ps, base, step;
-            if constexpr (ROLE == FIRST) {
-                ps = p[k];
-                base = at[k] + p[k] * (r - 1);
-                step = 1;
-            } else {
-                ps = fdiv(p[k], inv_s) * s;
-                base = at[k] + ps * (r - 1);
-                step = s;
-            }
+            const int p = ROLE == FIRST ? col[k] : fdiv(G::COLS ? e[k] : col[k], inv_s);
+            const int ps = p * s, base = e[k] + p * sm * (r - 1);
             if constexpr (ROLE == FIRST) {
 #pragma unroll
                 for (int j = 0; j < r; ++j) v[k][j] = make_float2(v[k][j].x * mul, v[k][j].y * mul);
             }
 #pragma unroll
             for (int j = 1; j < r; ++j) v[k][j] = cmulf(v[k][j], c.tw[j * ps]);
-            if constexpr (ROLE == FIRST && r % 2 == 0) {
+            if constexpr (ROLE == FIRST && !G::COLS && r % 2 == 0) {
                 // r consecutive words per lane: 16-byte writes (8-byte ones at this stride share banks)
 #pragma unroll
                 for (int j = 0; j < r; j += 2)
                     *reinterpret_cast<f4 *>(c.data + base + j) = f4{v[k][j].x, v[k][j].y, v[k][j + 1].x, v[k][j + 1].y};
             } else {
 #pragma unroll
-                for (int j = 0; j < r; ++j) c.data[base + j * step] = v[k][j];
+                for (int j = 0; j < r; ++j) c.data[base + j * sm] = v[k][j];
             }
         }
     }
     if constexpr (ROLE != LAST) __syncthreads();
 }
 
-// One radix-16 stage on the matrix cores: 16 columns per group, lane (g, col) feeds points
+// One radix-16 stage on the matrix cores: 16 columns per group, lane (g, column) feeds points
 // 4g..4g+3 of its column and receives outputs 4g..4g+3 of it.
-template <int PREC, int ROLE, int INF, int OUTF>
-__device__ __forceinline__ void mstage(const Ctx &c, const fast::Ops<PREC> &op, int cols, int s, float inv_cols,
-                                       float inv_s, float mul)
+template <class G, int PREC, int ROLE, int INF, int OUTF>
+__device__ __forceinline__ void mstage(const Ctx &c, int ncols, int s, float mul)
 {
     typedef typename Elem<INF>::raw iraw;
     typedef typename Elem<OUTF>::raw oraw;
-    constexpr int NW = NT / 64;
-    constexpr int MAXP = kMaxTile / 256 / NW;
+    constexpr int NW = G::NT / 64;
+    constexpr int MAXP = (G::CAP / 16 + 16 * NW - 1) / (16 * NW);
     constexpr bool EXACT =
         ROLE == FIRST && ((INF == FMT_C16 && PREC != PREC_BF16) || (INF == FMT_CBF16 && PREC == PREC_BF16));
-    const int lane = c.tid & 63, wave = c.tid >> 6;
-    const int g = lane >> 4;
-    const int slots = c.nl * cols;
+    // the operands are loaded by the stage that needs them: held through the vector-ALU stages
+    // they would cost the kernel a wave per SIMD
+    fast::Ops<PREC> op;
+    op.load(reinterpret_cast<const DftOps *>(c.dft_ops), c.tid & 63);
+    const Cols<G> K(c, ncols);
+    const int wave = c.tid >> 6, l15 = c.tid & 15;
+    const int g = (c.tid & 63) >> 4;
     f4 yr[MAXP], yi[MAXP];
-    int at[MAXP], col[MAXP];
+    int e[MAXP], col[MAXP], t[MAXP];
     iraw rw[ROLE == FIRST ? MAXP : 1][4];
     float2 x[MAXP][4];
 #pragma unroll
     for (int u = 0; u < MAXP; ++u) {
         // lanes past the last column repeat it (their outputs are dropped): the matrix
         // instruction takes all 64 lanes
-        const int slot = min((wave + u * NW) * 16 + (lane & 15), slots - 1);
-        const int t = fdiv(slot, inv_cols);
-        col[u] = slot - t * cols;
-        at[u] = t * c.R + col[u];
-        if ((wave + u * NW) * 16 < slots) {
+        K.at(c, min((wave + u * NW) * 16 + l15, K.n - 1), e[u], col[u], t[u]);
+        if ((wave + u * NW) * 16 < K.n) {
+            if constexpr (ROLE == FIRST) {
+                const unsigned st = K.template gstep<sizeof(iraw)>(c.ps_in);
+                const unsigned o = K.template goff<sizeof(iraw)>(e[u], col[u], t[u], c.ps_in) + 4 * g * st;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if constexpr (ROLE == FIRST)
-                    rw[u][i] = reinterpret_cast<const iraw *>(c.in)[(unsigned)(at[u] + (4 * g + i) * cols)];
-                else
-                    x[u][i] = c.data[at[u] + (4 * g + i) * cols];
+                for (int i = 0; i < 4; ++i) rw[u][i] = *reinterpret_cast<const iraw *>(c.in + (o + i * st));
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[u][i] = c.data[e[u] + (4 * g + i) * K.pitch];
             }
         }
     }
 #pragma unroll
     for (int u = 0; u < MAXP; ++u) {
-        if ((wave + u * NW) * 16 >= slots) continue;  // the same for the whole wave
+        if ((wave + u * NW) * 16 >= K.n) continue;  // the same for the whole wave
         h8 r16;
         b8 rb;
         if constexpr (ROLE == FIRST) {
@@ -248,46 +299,51 @@ __device__ __forceinline__ void mstage(const Ctx &c, const fast::Ops<PREC> &op, 
         fast::dft16<PREC, EXACT>(x[u], r16, rb, op, yr[u], yi[u]);
     }
     if constexpr (ROLE == MID) __syncthreads();
+    const int sm = s * K.mul;
+    const float inv_s = ROLE == MID ? recip(sm) : 0.f;
 #pragma unroll
     for (int u = 0; u < MAXP; ++u) {
-        if ((wave + u * NW) * 16 + (lane & 15) >= slots) continue;
+        if ((wave + u * NW) * 16 + l15 >= K.n) continue;
         if constexpr (ROLE == LAST) {
-            oraw *dst = reinterpret_cast<oraw *>(c.out);
+            const unsigned st = K.template gstep<sizeof(oraw)>(c.ps_out);
+            const unsigned o = K.template goff<sizeof(oraw)>(e[u], col[u], t[u], c.ps_out) + 4 * g * st;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                dst[(unsigned)(at[u] + (4 * g + i) * cols)] = Elem<OUTF>::pack(make_float2(yr[u][i] * mul, yi[u][i] * mul));
+                *reinterpret_cast<oraw *>(c.out + (o + i * st)) =
+                    Elem<OUTF>::pack(make_float2(yr[u][i] * mul, yi[u][i] * mul));
         } else {
-            const int ps = ROLE == FIRST ? col[u] : fdiv(col[u], inv_s) * s;
+            const int p = ROLE == FIRST ? col[u] : fdiv(G::COLS ? e[u] : col[u], inv_s);
+            const int ps = p * s;
             float2 y[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 y[i] = cmulf(make_float2(yr[u][i] * mul, yi[u][i] * mul), c.tw[(4 * g + i) * ps]);
-            float2 *d = c.data + at[u] + ps * 15;
-            if constexpr (ROLE == FIRST) {
+            float2 *d = c.data + e[u] + p * sm * 15;
+            if constexpr (ROLE == FIRST && !G::COLS) {
                 *reinterpret_cast<f4 *>(d + 4 * g) = f4{y[0].x, y[0].y, y[1].x, y[1].y};
                 *reinterpret_cast<f4 *>(d + 4 * g + 2) = f4{y[2].x, y[2].y, y[3].x, y[3].y};
             } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) d[(4 * g + i) * s] = y[i];
+                for (int i = 0; i < 4; ++i) d[(4 * g + i) * sm] = y[i];
             }
         }
     }
     if constexpr (ROLE != LAST) __syncthreads();
 }
 
-template <int PREC, int ROLE, int INF, int OUTF>
-__device__ __forceinline__ void stage(const Ctx &c, const fast::Ops<PREC> &op, const MixSched &sc, int st)
+template <class G, int PREC, int ROLE, int INF, int OUTF>
+__device__ __forceinline__ void stage(const Ctx &c, const MixSched &sc, int st)
 {
     const int cols = sc.cols[st], s = sc.s[st];
-    const float ic = sc.inv_cols[st], is = sc.inv_s[st], mul = sc.mul[st];
+    const float mul = sc.mul[st];
 #define MFFT_MIX_CASE(r) \
-    case r: vstage<r, ROLE, INF, OUTF>(c, cols, s, ic, is, mul); break
+    case r: vstage<G, r, ROLE, INF, OUTF>(c, cols, s, mul); break
     switch (sc.radix[st]) {
     case 16:
         if constexpr (PREC == PREC_FP32)
-            vstage<16, ROLE, INF, OUTF>(c, cols, s, ic, is, mul);
+            vstage<G, 16, ROLE, INF, OUTF>(c, cols, s, mul);
         else
-            mstage<PREC, ROLE, INF, OUTF>(c, op, cols, s, ic, is, mul);
+            mstage<G, PREC, ROLE, INF, OUTF>(c, cols, s, mul);
         break;
     MFFT_MIX_CASE(3);
     MFFT_MIX_CASE(5);
@@ -299,12 +355,12 @@ __device__ __forceinline__ void stage(const Ctx &c, const fast::Ops<PREC> &op, c
     MFFT_MIX_CASE(17);
     default:
         if constexpr (ROLE == FIRST) {
-            vstage<1, ROLE, INF, OUTF>(c, cols, s, ic, is, mul);  // a length of one stage: a copy first
+            vstage<G, 1, ROLE, INF, OUTF>(c, cols, s, mul);  // a length of one stage: a copy first
         } else {
             switch (sc.radix[st]) {
             MFFT_MIX_CASE(2);
             MFFT_MIX_CASE(4);
-            default: vstage<8, ROLE, INF, OUTF>(c, cols, s, ic, is, mul); break;
+            default: vstage<G, 8, ROLE, INF, OUTF>(c, cols, s, mul); break;
             }
         }
         break;
@@ -312,36 +368,75 @@ __device__ __forceinline__ void stage(const Ctx &c, const fast::Ops<PREC> &op, c
 #undef MFFT_MIX_CASE
 }
 
-template <int PREC, int INF, int OUTF>
-__device__ __forceinline__ void tile(const Ctx &c, const fast::Ops<PREC> &op, const MixSched &sc)
+template <class G, int PREC, int INF, int OUTF>
+__device__ __forceinline__ void tile(const Ctx &c, const MixSched &sc)
 {
-    stage<PREC, FIRST, INF, OUTF>(c, op, sc, 0);
-    for (int st = 1; st < sc.nst - 1; ++st) stage<PREC, MID, INF, OUTF>(c, op, sc, st);
-    stage<PREC, LAST, INF, OUTF>(c, op, sc, sc.nst - 1);
+    stage<G, PREC, FIRST, INF, OUTF>(c, sc, 0);
+    for (int st = 1; st < sc.nst - 1; ++st) stage<G, PREC, MID, INF, OUTF>(c, sc, st);
+    stage<G, PREC, LAST, INF, OUTF>(c, sc, sc.nst - 1);
 }
 
+template <int NT>
 __device__ __forceinline__ void load_table(float2 *dst, const float2 *src, int R)
 {
     for (int i = threadIdx.x; i < R; i += NT) dst[i] = src[i];
 }
 
+// Waves per SIMD the registers are held to. Contiguous lines, 1200 x 3001 in us at 4 / 5 / 6 / 8:
+// fp32 15.5 / 15.6 / 14.8 / 13.2; split fp16 spills from 6 on.
+template <int PREC>
+constexpr int row_waves() { return PREC == PREC_FP32 ? 8 : PREC == PREC_SPLIT ? 5 : 6; }
+
 // One workgroup per tile: in a loop over tiles the lane addresses of every stage are loop
 // invariants, which the compiler keeps in registers until they spill.
 template <int PREC, int INF, int OUTF>
-__global__ void __launch_bounds__(kMixThreads, 4) fft_mixed(MixArgs a)
+__global__ void __launch_bounds__(kMixThreads, row_waves<PREC>()) fft_mixed(MixArgs a)
 {
+    typedef Geo<false, kMixThreads, kMaxTile> G;
     extern __shared__ __attribute__((aligned(16))) float2 sm[];
     const int R = a.sc.R;
-    fast::Ops<PREC> op;
-    if constexpr (PREC != PREC_FP32) op.load(reinterpret_cast<const DftOps *>(a.dft_ops), threadIdx.x & 63);
     float2 *tw = sm + a.T * R;
-    load_table(tw, a.tw, R);
+    load_table<G::NT>(tw, a.tw, R);
     __syncthreads();
     const long long l0 = (long long)blockIdx.x * a.T, left = a.nlines - l0;
-    const Ctx c{sm, tw, a.tw, reinterpret_cast<const typename Elem<INF>::raw *>(a.in) + l0 * R,
-                reinterpret_cast<typename Elem<OUTF>::raw *>(a.out) + l0 * R, R, (int)(left < a.T ? left : a.T), a.sign,
+    const Ctx c{sm, tw, a.tw, a.dft_ops,
+                reinterpret_cast<const char *>(a.in) + l0 * R * (long long)sizeof(typename Elem<INF>::raw),
+                reinterpret_cast<char *>(a.out) + l0 * R * (long long)sizeof(typename Elem<OUTF>::raw),
+                R, (int)(left < a.T ? left : a.T), a.sign, 0u, 0u, a.w16, (int)threadIdx.x};
+    tile<G, PREC, INF, OUTF>(c, a.sc);
+}
+
+// Strided lines: the lines of a transform are adjacent (a point of T lines is one segment of
+// memory), c0 of them, transforms in_dist / out_dist elements apart. CAP: points per tile.
+// Bound: instruction issue, and segment length (16 lines of 16-bit words are 64 bytes). Tiles
+// of up to 8192 points run 512 threads at 16 points each, two workgroups per compute unit (480
+// x 640 x 18 2D split fp16 39.9 us; 256 threads 44.4, 1024 threads 42.1); longer lines fill the
+// LDS with one workgroup of 1024. 2D execs with both axes on the mixed-radix kernels against an
+// odd pass and a power-of-two pass per axis (us): 480 x 640 x 18 fp32 90 -> 41, split fp16 86 ->
+// 40, 960 x 960 x 16 fp32 177 -> 100, 96 x 96 x 100 split fp16 90 -> 15.
+template <int CAP, int PREC, int INF, int OUTF>
+__global__ void __launch_bounds__(mix_col_threads(CAP), 4) fft_mixed_cols(MixColArgs a)
+{
+    typedef Geo<true, mix_col_threads(CAP), CAP> G;
+    typedef typename Elem<INF>::raw iraw;
+    typedef typename Elem<OUTF>::raw oraw;
+    extern __shared__ __attribute__((aligned(16))) float2 sm[];
+    const int R = a.sc.R;
+    float2 *tw = sm + a.T * R;
+    load_table<G::NT>(tw, a.tw, R);
+    __syncthreads();
+    // each XCD (workgroups are dealt to the 8 of them in turn) takes a run of tiles, so that
+    // neighbouring tiles, which share cache lines, meet in one L2
+    unsigned b = blockIdx.x;
+    const unsigned nb = gridDim.x;
+    if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
+    const unsigned tr = b / (unsigned)a.tiles0, t0 = b - tr * (unsigned)a.tiles0;
+    const int l0 = (int)t0 * a.T;
+    const Ctx c{sm, tw, a.tw, a.dft_ops, reinterpret_cast<const char *>(reinterpret_cast<const iraw *>(a.in) + tr * a.in_dist + l0),
+                reinterpret_cast<char *>(reinterpret_cast<oraw *>(a.out) + tr * a.out_dist + l0),
+                R, min(a.c0 - l0, a.T), a.sign, (unsigned)(a.ps_in * (int)sizeof(iraw)), (unsigned)(a.ps_out * (int)sizeof(oraw)),
                 a.w16, (int)threadIdx.x};
-    tile<PREC, INF, OUTF>(c, op, a.sc);
+    tile<G, PREC, INF, OUTF>(c, a.sc);
 }
 
 // Many transforms of uneven length and count in one launch: workgroup b takes tile b, then
@@ -352,11 +447,10 @@ __global__ void __launch_bounds__(kMixThreads, 4) fft_mixed(MixArgs a)
 template <int PREC, int INF, int OUTF>
 __global__ void __launch_bounds__(kMixThreads, 4) fft_mixed_queue(MixQueueArgs a)
 {
+    typedef Geo<false, kMixThreads, kMaxTile> G;
     extern __shared__ __attribute__((aligned(16))) float2 sm[];
     __shared__ unsigned s_next;
     const int lane = threadIdx.x & 63;
-    fast::Ops<PREC> op;
-    if constexpr (PREC != PREC_FP32) op.load(reinterpret_cast<const DftOps *>(a.dft_ops), lane);
     int t = blockIdx.x, have = -1;  // have: the length whose table is in LDS
     float2 *tw = sm + a.tw_at;
     while (t < a.total) {
@@ -376,17 +470,18 @@ __global__ void __launch_bounds__(kMixThreads, 4) fft_mixed_queue(MixQueueArgs a
         const MixLen &len = a.lens[li];
         const int R = len.sc.R;
         if (have != li) {
-            load_table(tw, len.tw, R);
+            load_table<G::NT>(tw, len.tw, R);
             have = li;
         }
         __syncthreads();
         int tid = threadIdx.x;
         __asm__("" : "+v"(tid));  // not a loop invariant: see fft_mixed
         const long long l0 = (long long)(t - first) * it.T, left = it.nlines - l0;
-        const Ctx c{sm, tw, len.tw, reinterpret_cast<const typename Elem<INF>::raw *>(it.in) + l0 * R,
-                    reinterpret_cast<typename Elem<OUTF>::raw *>(it.out) + l0 * R, R, (int)(left < it.T ? left : it.T),
-                    a.sign, a.w16, tid};
-        tile<PREC, INF, OUTF>(c, op, len.sc);
+        const Ctx c{sm, tw, len.tw, a.dft_ops,
+                    reinterpret_cast<const char *>(it.in) + l0 * R * (long long)sizeof(typename Elem<INF>::raw),
+                    reinterpret_cast<char *>(it.out) + l0 * R * (long long)sizeof(typename Elem<OUTF>::raw),
+                    R, (int)(left < it.T ? left : it.T), a.sign, 0u, 0u, a.w16, tid};
+        tile<G, PREC, INF, OUTF>(c, len.sc);
         if (a.total <= (int)gridDim.x) return;  // one tile per workgroup: no queue
         if (threadIdx.x == 0) s_next = gridDim.x + atomicAdd(a.counter, 1u);
         __syncthreads();

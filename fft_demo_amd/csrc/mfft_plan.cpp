@@ -217,7 +217,8 @@ struct PassSpec {
     bool onchip = false;    // the whole 65536-point line in one pass (fft_onchip)
     bool onchip_cols = false;  // 2048-point lines, 32 per workgroup (fft_onchip_cols)
     bool onchip_rows = false;  // ... contiguous lines stored transposed (its rows kind)
-    bool mixed = false;     // dense contiguous lines on the mixed-radix kernel (fft_mixed)
+    bool mixed = false;     // lines on the mixed-radix kernels (fft_mixed, fft_mixed_cols)
+    int mixed_cap = 0;      // strided lines: points per tile at most; 0 = dense contiguous lines
     MixSched mix{};
 };
 
@@ -315,8 +316,6 @@ static bool factorable(long long n)
     return n <= kMaxTile && line_radices((int)n, r);
 }
 
-// Append the passes of a length-L DFT along an axis. Input element (line, j) is at
-// line_in + j*ps_in, output element (line, k) at line_out + k*ps_out.
 static long long odd_part(long long L)
 {
     while (L > 0 && L % 2 == 0) L /= 2;
@@ -326,6 +325,32 @@ static long long odd_part(long long L)
 // Odd factors the streaming kernel takes as a pass of its own.
 static bool small_odd(long long o) { return o == 3 || o == 5 || o == 9 || o == 15 || o == 17; }
 
+// Lines per tile of the strided mixed-radix kernels at most: 32 up to 256 points (a point of a
+// tile is then a segment of 128 bytes of 16-bit words), 16 up to 1088, 8 up to 2176.
+static int mixed_col_lines(long long R)
+{
+    return R * 32 <= kMixColSmall ? 32 : R * 16 <= kMixColLarge ? 16 : R * 8 <= kMixColLarge ? 8 : 0;
+}
+
+// An axis with odd factors that runs in one pass of the mixed-radix kernels instead of an odd
+// pass and a power-of-two pass. Where the two passes stay (us, two passes / one): contiguous
+// lines above 2048 points with a factor 17 on the matrix cores, one line a tile, whose radix-17
+// stage then keeps a quarter of the threads busy (2176 x 4000 split fp16: 39 / 43, with 16-bit
+// intermediates 33 / 43; plain fp32 45 / 36, 3072 x 4000 split fp16 60 / 42); strided lines
+// above 1088 points with 16-bit words, 8 lines a tile, segments of 32 bytes (2176 x 2176 x 4
+// split fp16 110 / 151, plain fp32 209 / 185; 1088 x 1088 x 16 split fp16 129 / 119).
+static bool mixed_one_pass(int prec, long long L, long long ps_in, long long ps_out, const std::vector<Level> &lines)
+{
+    std::vector<int> r;
+    if (is_pow2(L) || L > kMaxTile || !mix_radices((int)L, r)) return false;
+    if (ps_in == 1 && ps_out == 1) return prec == PREC_FP32 || L <= kMaxTile / 2 || L % 17 || !small_odd(odd_part(L));
+    const long long T = mixed_col_lines(L);
+    if (ps_in == 1 || T < (prec == PREC_FP32 ? 8 : 16) || std::max(ps_in, ps_out) * L >= (1LL << 29)) return false;
+    for (auto &l : lines)
+        if (l.in_stride == 1 && l.out_stride == 1 && !l.batch) return lines.size() <= 2;
+    return false;
+}
+
 // Whether a plan's intermediates between passes are 16-bit (the rule finalize_plan applies).
 static bool narrow_mid(const mfft_desc *d)
 {
@@ -333,12 +358,15 @@ static bool narrow_mid(const mfft_desc *d)
     return d->precision == MFFT_PREC_FP16 || d->precision == MFFT_PREC_BF16;
 }
 
+// Append the passes of a length-L DFT along an axis. Input element (line, j) is at
+// line_in + j*ps_in, output element (line, k) at line_out + k*ps_out.
 // narrow: the intermediates between passes are 16-bit (an extra pass costs 8 bytes a point)
 // rev_cols: a digit-reversed strided axis may still run in one pass of the strided
 // matrix-core kernel (it reads the reversed order itself)
+// mixed: the precision whose mixed-radix kernels exist for the axis's formats, -1 = none
 static int plan_axis(std::vector<PassSpec> &out, long long L, long long ps_in, long long ps_out,
                      std::vector<Level> lines, int src, int dst, int perm_axis, int split_hint, bool narrow,
-                     bool rev_cols = false)
+                     bool rev_cols = false, int mixed = -1)
 {
     // odd * 2^a (2176 = 17 x 128): the odd factor in a streaming pass, the power of two on
     // the matrix-core kernels, instead of one generic mixed-radix tile pass.
@@ -347,7 +375,9 @@ static int plan_axis(std::vector<PassSpec> &out, long long L, long long ps_in, l
     const bool odd_split = perm_axis < 0 && split_hint != 1 && odd > 1 && small_odd(odd) && L / odd >= 16 &&
                            L / odd <= kMaxTile;
     const bool fast_cols = (perm_axis < 0 || rev_cols) && split_hint <= 1;  // no split asked for
-    if (!odd_split && single_pass_ok((int)std::min<long long>(L, 1 << 30), ps_in, lines, fast_cols)) {
+    const bool one_mixed =
+        mixed >= 0 && perm_axis < 0 && split_hint <= 1 && mixed_one_pass(mixed, L, ps_in, ps_out, lines);
+    if (one_mixed || (!odd_split && single_pass_ok((int)std::min<long long>(L, 1 << 30), ps_in, lines, fast_cols))) {
         PassSpec p;
         p.R = (int)L;
         p.ps_in = ps_in;
@@ -721,8 +751,11 @@ static int finish_passes(mfft_plan_s *p)
             }
         }
         if (ps.fast_kind < 0) ps.rev_fast = false;
-        if (ps.generic && !ps.small && ps.fast_kind < 0 && !rev && !ps.tw_N && dense_rows(ps)) {
-            const void *fn = find_mixed_kernel(p->d.precision, in_fmt, out_fmt);
+        const bool mixed_cols = !is_pow2(ps.R) && ps.ps_in != 1 && mixed_one_pass(p->d.precision, ps.R, ps.ps_in, ps.ps_out, ps.lines);
+        if (!ps.small && ps.fast_kind < 0 && !rev && !ps.tw_N && (mixed_cols || (ps.generic && dense_rows(ps)))) {
+            const int T = mixed_cols ? mixed_col_lines(ps.R) : 0;
+            ps.mixed_cap = !mixed_cols ? 0 : ps.R * T <= kMixColSmall ? kMixColSmall : kMixColLarge;
+            const void *fn = find_mixed_kernel(p->d.precision, in_fmt, out_fmt, ps.mixed_cap);
             if (fn && mix_schedule(ps.R, p->d.precision, p->d.scale == MFFT_SCALE_STAGE, ps.mix)) {
                 ps.mixed = true;
                 ps.fn = fn;
@@ -730,10 +763,18 @@ static int finish_passes(mfft_plan_s *p)
                 long long nl = 1;
                 for (auto &l : ps.lines) nl *= l.count;
                 ps.max_grid = 2 * device_cus();
-                ps.T = mixed_tile_lines(ps.R, nl, ps.max_grid);
                 ps.TL = 1;
                 ps.l0 = 0;
-                HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix_lds_bytes(kMaxTile, kMaxTile)));
+                int lds = (int)mix_lds_bytes(kMaxTile, kMaxTile);
+                if (mixed_cols) {
+                    for (int i = 0; i < (int)ps.lines.size(); ++i)
+                        if (ps.lines[i].in_stride == 1 && ps.lines[i].out_stride == 1 && !ps.lines[i].batch) ps.l0 = i;
+                    ps.T = (int)std::min<long long>(T, ps.lines[ps.l0].count);
+                    lds = (int)mix_lds_bytes(ps.mixed_cap, ps.R);
+                } else {
+                    ps.T = mixed_tile_lines(ps.R, nl, ps.max_grid);
+                }
+                HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, std::max(lds, 65536)));
             }
         }
         if (rev && !ps.rev_fast && ps.perm_axis < 0)
@@ -1064,6 +1105,34 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
                 HIP_TRY(hipLaunchKernel(ps.fn, grid, block, oargs, 0, s));
             continue;
         }
+        if (ps.mixed && ps.mixed_cap) {
+            MixColArgs m;
+            m.in = a.in;
+            m.out = a.out;
+            m.tw = ps.stage_tw;
+            m.dft_ops = p->ops;
+            m.sign = p->d.direction;
+            m.c0 = a.c0;
+            // fewer lines per tile when the launch would leave compute units without one
+            m.T = ps.T;
+            while (m.T > 8 && (long long)((a.c0 + m.T - 1) / m.T) * a.c1 < ps.max_grid / 2) m.T /= 2;
+            m.tiles0 = (a.c0 + m.T - 1) / m.T;
+            m.ps_in = (int)a.in_ps;
+            m.ps_out = (int)a.out_ps;
+            m.in_dist = a.in_s1;
+            m.out_dist = a.out_s1;
+            memcpy(m.w16, g_w16, sizeof m.w16);
+            m.sc = ps.mix;
+            const long long blocks = (long long)m.tiles0 * a.c1;
+            if (blocks >= (1LL << 31)) return fail(MFFT_ERR_UNSUPPORTED, "grid too large");
+            void *margs[] = {&m};
+            const size_t lds = mix_lds_bytes(m.T * ps.R, ps.R);
+            if (kstart || kstop)
+                HIP_TRY(hipExtLaunchKernel(ps.fn, dim3((unsigned)blocks), dim3(mix_col_threads(ps.mixed_cap)), margs, lds, s, kstart, kstop, 0));
+            else
+                HIP_TRY(hipLaunchKernel(ps.fn, dim3((unsigned)blocks), dim3(mix_col_threads(ps.mixed_cap)), margs, lds, s));
+            continue;
+        }
         if (ps.mixed) {
             MixArgs m;
             m.in = a.in;
@@ -1192,7 +1261,8 @@ static int create_1d(mfft_plan *plan, int n, int64_t batch, const mfft_desc *d_i
         rc = plan_reversed_1d(p);
     } else {
         std::vector<Level> lines{Level{batch, n, n, true}};
-        rc = plan_axis(p->passes, n, 1, 1, lines, BUF_IN, BUF_OUT, rev ? 0 : -1, d->split_hint, narrow_mid(d));
+        rc = plan_axis(p->passes, n, 1, 1, lines, BUF_IN, BUF_OUT, rev ? 0 : -1, d->split_hint, narrow_mid(d), false,
+                       find_mixed_kernel(d->precision, d->in_fmt, d->out_fmt) ? d->precision : -1);
     }
     if (!rc) rc = finalize_plan(p);
     if (rc) {
@@ -1232,8 +1302,10 @@ int mfft_plan_create_1d(mfft_plan *plan, int n, int64_t batch, const mfft_desc *
     return MFFT_OK;
 }
 
+// conv: a transform of the conv operator, whose odd axes keep a streaming pass of their own (it
+// takes the fused image load and filter product)
 static int create_2d(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_desc *d_in, bool allow_onchip,
-                     bool out_mid = false)
+                     bool out_mid, bool conv)
 {
     if (!plan || !d_in) return fail(MFFT_ERR_INVALID, "null argument");
     *plan = nullptr;
@@ -1269,7 +1341,8 @@ static int create_2d(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_
     // rows (y axis, contiguous): lines = (x, b)
     std::vector<Level> rows{Level{nx, ny, ny, false}, Level{batch, NN, NN, true}};
     const int odd_hint = d->split_hint == 1 ? 1 : 0;  // 1 keeps odd * 2^a axes in one pass
-    rc = plan_axis(p->passes, ny, 1, 1, rows, BUF_IN, BUF_WORK, rev ? 1 : -1, odd_hint, narrow_mid(d));
+    rc = plan_axis(p->passes, ny, 1, 1, rows, BUF_IN, BUF_WORK, rev ? 1 : -1, odd_hint, narrow_mid(d), false,
+                   !conv && find_mixed_kernel(d->precision, d->in_fmt, col_in_fmt) ? d->precision : -1);
     // columns (x axis, stride ny): lines = (y, b)
     if (!rc) {
         // split_hint > 1: the first-pass length of the column axis when it is split
@@ -1292,7 +1365,8 @@ static int create_2d(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_
             p->passes.push_back(ps);
         } else {
             rc = plan_axis(p->passes, nx, ny, ny, cols, BUF_WORK, BUF_OUT, rev ? 0 : -1, col_hint, narrow_mid(d),
-                           rev_cols);
+                           rev_cols,
+                           !conv && find_mixed_kernel(d->precision, col_in_fmt, d->out_fmt) ? d->precision : -1);
         }
     }
     p->out_mid = out_mid;
@@ -1308,13 +1382,14 @@ static int create_2d(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_
     return MFFT_OK;
 }
 
-static int create_2d_all(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_desc *d_in, bool out_mid)
+static int create_2d_all(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_desc *d_in, bool out_mid,
+                         bool conv)
 {
-    int rc = create_2d(plan, nx, ny, batch, d_in, true, out_mid);
+    int rc = create_2d(plan, nx, ny, batch, d_in, true, out_mid, conv);
     if (rc || !has_onchip(*plan)) return rc;
     mfft_plan p = *plan, q = nullptr;
     const long long below = onchip_cols_min_images(ny);
-    rc = create_2d(&q, nx, ny, below - 1, d_in, false, out_mid);
+    rc = create_2d(&q, nx, ny, below - 1, d_in, false, out_mid, conv);
     if (rc) {
         std::string msg = g_err;
         mfft_plan_destroy(p);
@@ -1329,7 +1404,7 @@ static int create_2d_all(mfft_plan *plan, int nx, int ny, int64_t batch, const m
 
 int mfft_plan_create_2d(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_desc *d_in)
 {
-    return create_2d_all(plan, nx, ny, batch, d_in, false);
+    return create_2d_all(plan, nx, ny, batch, d_in, false, false);
 }
 
 int mfft_plan_destroy(mfft_plan plan)
@@ -1949,9 +2024,9 @@ void StreamOrder::destroy()
     ev = nullptr;
 }
 
-int plan_create_2d_out_mid(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_desc *d)
+int plan_create_2d_conv(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_desc *d, bool out_mid)
 {
-    return create_2d_all(plan, nx, ny, batch, d, true);
+    return create_2d_all(plan, nx, ny, batch, d, out_mid, true);
 }
 
 bool plan_first_pass_fusable(mfft_plan p)

@@ -102,3 +102,25 @@ def test_queue(dev, prec, what):
         l2, mx = rel_errors(y, oracle.fft(x))
         assert l2 <= TOL[prec][0] and mx <= TOL[prec][1], (n, c, l2, mx)
     lib.mfft_batcher_destroy(bh)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", list(TOL))
+@pytest.mark.parametrize("nx,ny,b", [(96, 80, 3),       # 32 lines a tile, partial last tile
+                                     (480, 100, 2),     # 16 lines a tile, 4 in the last
+                                     (1088, 64, 2),     # the large tile, full
+                                     (2176, 72, 1),     # 8 lines a tile
+                                     (272, 5, 2)])      # fewer lines than a tile
+def test_mixed_columns(dev, prec, nx, ny, b):
+    import fft_demo_amd as F
+
+    fmt = {"bf16": "cbf16", "fp32": "c32"}.get(prec, "c16")
+    x = complex_input((b, nx, ny), nx + ny, fmt)
+    for inverse in (False, True):
+        with F.Plan((nx, ny), b, precision=prec, direction=F.INVERSE if inverse else F.FORWARD) as plan:
+            assert len(plan.info["passes"]) == 2 or (nx > 1088 and prec != "fp32")
+            xd = to_device(x, _dtype(prec), dev)
+            y = from_device(plan.exec(xd, out=xd)) / plan.out_scale  # in place
+        ref = oracle.fft2d(x.conj()).conj() if inverse else oracle.fft2d(x)
+        l2, mx = rel_errors(y, ref)
+        assert l2 <= TOL[prec][0] and mx <= TOL[prec][1], (inverse, l2, mx)
