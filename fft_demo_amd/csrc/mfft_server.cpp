@@ -91,7 +91,8 @@ struct mfft_server_s {
     std::vector<std::pair<int, int>> stale_classes;  // (fh & 1, fw & 1) changed since their operators were built; under mu
     struct mfft_server_convs *conv = nullptr;
     std::mutex mu;
-    std::condition_variable cv;
+    std::condition_variable cv;       // submissions, for the scheduler
+    std::condition_variable idle_cv;  // the last outstanding request completed
     std::deque<Req *> incoming;
     std::deque<Req *> pending;
     std::vector<Req *> inflight;
@@ -383,6 +384,7 @@ void complete(mfft_server_s *S, Req *q, int status)
         std::lock_guard<std::mutex> lk(S->mu);
         S->done.push_back(c);
         S->completed++;
+        if (S->submitted == S->completed) S->idle_cv.notify_all();
     }
     if (q->admitted) S->used -= q->need;
     if (q->stream >= 0) {
@@ -692,15 +694,17 @@ int mfft_server_poll(mfft_server S, mfft_completion *out, int max, int *n)
 int mfft_server_wait_idle(mfft_server S, double timeout_s)
 {
     if (!S) return sfail(MFFT_ERR_INVALID, "null server");
-    double t0 = now_us();
-    while (true) {
-        {
-            std::lock_guard<std::mutex> lk(S->mu);
-            if (S->submitted == S->completed) return MFFT_OK;
-        }
-        if (timeout_s > 0 && now_us() - t0 > timeout_s * 1e6) return sfail(MFFT_ERR_INVALID, "timeout");
-        std::this_thread::sleep_for(std::chrono::microseconds(100));
+    // woken by the completion that leaves nothing outstanding
+    std::unique_lock<std::mutex> lk(S->mu);
+    auto idle = [&] { return S->submitted == S->completed; };
+    if (timeout_s > 0) {
+        // bounded: a longer wait would overflow the clock
+        const double t = std::min(timeout_s, 1e9);
+        if (!S->idle_cv.wait_for(lk, std::chrono::duration<double>(t), idle)) return sfail(MFFT_ERR_INVALID, "timeout");
+    } else {
+        S->idle_cv.wait(lk, idle);
     }
+    return MFFT_OK;
 }
 
 int mfft_server_get_stats(mfft_server S, mfft_server_stats *st)

@@ -71,6 +71,9 @@ class Plan:
             raise ValueError("shape must have 1 or 2 dimensions")
         L.check(rc, "mfft_plan_create")
         self._h = h
+        # what exec compares its buffers with, so that a call costs little more than its launch
+        self._values = self.batch * int(np.prod(self.shape)) * 2
+        self._dtypes = None  # (input, output), set by the first exec: torch is loaded on demand
         inf = L.Info()
         L.check(lib.mfft_plan_info(self._h, ctypes.byref(inf)), "mfft_plan_info")
         self.info = inf.as_dict()
@@ -101,20 +104,25 @@ class Plan:
             raise ValueError(f"{what} must be a device tensor")
         if not t.is_contiguous():
             raise ValueError(f"{what} must be contiguous")
-        if t.numel() != self.batch * self.n * 2:
-            raise ValueError(f"{what} has {t.numel()} values, expected {self.batch * self.n * 2}")
+        if t.numel() != self._values:
+            raise ValueError(f"{what} has {t.numel()} values, expected {self._values}")
 
     def exec(self, x, out=None, stream=None):
         """Run the transform on device tensors; returns `out`."""
-        torch = _torch()
-        self._check_buf(x, self.in_dtype(), "input")
+        if self._dtypes is None:
+            self._dtypes = (self.in_dtype(), self.out_dtype())
+        in_dtype, out_dtype = self._dtypes
+        self._check_buf(x, in_dtype, "input")
         if out is None:
             out = self.empty_out(device=x.device)
-        self._check_buf(out, self.out_dtype(), "output")
-        s = stream if stream is not None else torch.cuda.current_stream(x.device)
-        rc = L.load().mfft_exec(self._h, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(out.data_ptr()),
-                                ctypes.c_void_p(s.cuda_stream))
-        L.check(rc, "mfft_exec")
+        self._check_buf(out, out_dtype, "output")
+        if stream is None:
+            handle = _torch()._C._cuda_getCurrentRawStream(x.get_device())
+        else:
+            handle = stream.cuda_stream
+        rc = L.load().mfft_exec(self._h, x.data_ptr(), out.data_ptr(), handle)
+        if rc:
+            L.check(rc, "mfft_exec")
         return out
 
     def exec_ptr(self, in_ptr: int, out_ptr: int, stream_handle: int = 0) -> None:
