@@ -133,17 +133,20 @@ struct TileWalk {
     long long in_base, out_base;
     long long in_a, in_b, in_c, out_a, out_b, out_c;
 
-    __device__ __forceinline__ void init(const TileArgs &a, int T, long long tile, long long step)
+    // tile and step are below 2^31 (checked on the host): 32-bit divisions. 64-bit ones took
+    // hundreds of scalar instructions at the start of every workgroup, as long as a small
+    // launch's transforms (1024 x 4 5.3 -> 4.8 us without them, 16384 x 96 bf16 12.7 -> 11.0).
+    __device__ __forceinline__ void init(const TileArgs &a, int T, int tile, int step)
     {
         tiles0 = (a.c0 + T - 1) / T;
-        long long r = tile / tiles0;
-        t0 = (int)(tile - r * tiles0);
-        l1 = (int)(r % a.c1);
-        l2 = r / a.c1;
-        r = step / tiles0;
-        s0 = (int)(step - r * tiles0);
-        s1 = (int)(r % a.c1);
-        s2 = r / a.c1;
+        unsigned r = (unsigned)tile / (unsigned)tiles0;
+        t0 = tile - (int)r * tiles0;
+        l2 = r / (unsigned)a.c1;
+        l1 = (int)(r - (unsigned)l2 * (unsigned)a.c1);
+        r = (unsigned)step / (unsigned)tiles0;
+        s0 = step - (int)r * tiles0;
+        s2 = r / (unsigned)a.c1;
+        s1 = (int)(r - (unsigned)s2 * (unsigned)a.c1);
         const long long ti = (long long)T * a.in_s0, to = (long long)T * a.out_s0;
         in_base = t0 * ti + l1 * a.in_s1 + l2 * a.in_s2;
         out_base = t0 * to + l1 * a.out_s1 + l2 * a.out_s2;
@@ -810,14 +813,14 @@ __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float
     constexpr int MAP_OUT = KIND == KIND_ROWS ? MAP_POINTS : MAP_LINES;
     // Each of the 8 XCDs (workgroups are dealt to them round-robin) walks a contiguous
     // range of tiles, so tiles that share cache lines meet in the same L2.
-    const long long ntiles = (long long)((a.c0 + G::T - 1) / G::T) * a.c1 * a.c2;
-    long long tile, step, end;
+    const int ntiles = (a.c0 + G::T - 1) / G::T * a.c1 * a.c2;  // below 2^31 (checked on the host)
+    int tile, step, end;
     if ((gridDim.x & 7) == 0) {
-        const long long per = (ntiles + 7) >> 3;
+        const int per = (int)(((unsigned)ntiles + 7u) >> 3);
         const int xcd = blockIdx.x & 7;
-        tile = xcd * per + (blockIdx.x >> 3);
-        step = gridDim.x >> 3;
-        end = min(ntiles, (xcd + 1) * per);
+        tile = xcd * per + (int)(blockIdx.x >> 3);
+        step = (int)(gridDim.x >> 3);
+        end = xcd == 7 ? ntiles : min(ntiles, (xcd + 1) * per);
     } else {
         tile = blockIdx.x;
         step = gridDim.x;
@@ -838,7 +841,7 @@ __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float
     // first product
     wait_prefetch();
     while (tile < end) {
-        const long long next = tile + step;
+        const int next = (int)min((unsigned)tile + (unsigned)step, 0x7fffffffu);
         Origin on = o;
         if (next < end) {
             walk.advance(a);
