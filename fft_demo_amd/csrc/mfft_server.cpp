@@ -458,53 +458,66 @@ void scheduler(mfft_server_s *S)
         items.clear();
         convq.clear();
         const long long budget = S->d.hbm_budget;
-        for (auto it = S->pending.begin(); it != S->pending.end();) {
-            if (plain && !S->inflight.empty()) break;
-            Req *q = *it;
-            q->need = io_bytes(S, q->r);
-            if (S->static_bytes + S->used + q->need > budget) {
-                if (q->need + S->static_bytes > budget) {  // can never fit: reject
+        // Requests that arrive while a pass over the queue runs (it may build plans or a conv
+        // operator) are admitted in another one, while requests are held back (at most four
+        // passes): they can then pair or coalesce with those. Not past a filter registered
+        // meanwhile: its class's operators are dropped above, before requests that may use it.
+        for (int pass = 0; pass < 4; ++pass) {
+            if (pass) {
+                if (plain || (small.empty() && convq.empty())) break;
+                std::lock_guard<std::mutex> lk(S->mu);
+                if (S->incoming.empty() || !S->stale_classes.empty()) break;
+                S->pending.insert(S->pending.end(), S->incoming.begin(), S->incoming.end());
+                S->incoming.clear();
+            }
+            for (auto it = S->pending.begin(); it != S->pending.end();) {
+                if (plain && !S->inflight.empty()) break;
+                Req *q = *it;
+                q->need = io_bytes(S, q->r);
+                if (S->static_bytes + S->used + q->need > budget) {
+                    if (q->need + S->static_bytes > budget) {  // can never fit: reject
+                        it = S->pending.erase(it);
+                        complete(S, q, MFFT_ERR_NOMEM);
+                        continue;
+                    }
+                    ++it;
+                    continue;
+                }
+                q->t_start = now_us();
+                q->admitted = true;
+                S->used += q->need;
+                S->peak = std::max(S->peak.load(), S->static_bytes + S->used);
+                const bool is_small = !plain && q->r.kind == MFFT_REQ_FFT1D && q->r.n <= 4096 &&
+                                      (int)small.size() < S->d.coalesce_max && q->r.direction == MFFT_FORWARD;
+                if (is_small) {
+                    small.push_back(q);
+                    items.push_back(mfft_batch_item{q->r.in, q->r.out, q->r.n, q->r.batch});
+                    q->out_scale = 1.0 / q->r.n;
                     it = S->pending.erase(it);
-                    complete(S, q, MFFT_ERR_NOMEM);
                     continue;
                 }
-                ++it;
-                continue;
-            }
-            q->t_start = now_us();
-            q->admitted = true;
-            S->used += q->need;
-            S->peak = std::max(S->peak.load(), S->static_bytes + S->used);
-            const bool is_small = !plain && q->r.kind == MFFT_REQ_FFT1D && q->r.n <= 4096 &&
-                                  (int)small.size() < S->d.coalesce_max && q->r.direction == MFFT_FORWARD;
-            if (is_small) {
-                small.push_back(q);
-                items.push_back(mfft_batch_item{q->r.in, q->r.out, q->r.n, q->r.batch});
-                q->out_scale = 1.0 / q->r.n;
-                it = S->pending.erase(it);
-                continue;
-            }
-            if (!plain && q->r.kind == MFFT_REQ_CONV2D) {
-                // held back to pair with another request on the same operator
-                int idx = 0;
-                ConvSlot *c = get_conv(S, q->r.nx, q->r.ny, q->r.filter_id, &idx);
-                it = S->pending.erase(it);
-                if (!c) {
-                    complete(S, q, sfail(MFFT_ERR_UNSUPPORTED, "conv operator for filter %d", q->r.filter_id));
+                if (!plain && q->r.kind == MFFT_REQ_CONV2D) {
+                    // held back to pair with another request on the same operator
+                    int idx = 0;
+                    ConvSlot *c = get_conv(S, q->r.nx, q->r.ny, q->r.filter_id, &idx);
+                    it = S->pending.erase(it);
+                    if (!c) {
+                        complete(S, q, sfail(MFFT_ERR_UNSUPPORTED, "conv operator for filter %d", q->r.filter_id));
+                        continue;
+                    }
+                    convq[c].push_back({q, idx});
                     continue;
                 }
-                convq[c].push_back({q, idx});
-                continue;
+                int st = plain ? 0 : pick_stream(S, req_points(q->r) >= kBulkPoints);
+                int rc = launch_one(S, q, st);
+                it = S->pending.erase(it);
+                if (rc) {
+                    complete(S, q, rc);
+                    continue;
+                }
+                S->inflight.push_back(q);
+                if (plain) break;
             }
-            int st = plain ? 0 : pick_stream(S, req_points(q->r) >= kBulkPoints);
-            int rc = launch_one(S, q, st);
-            it = S->pending.erase(it);
-            if (rc) {
-                complete(S, q, rc);
-                continue;
-            }
-            S->inflight.push_back(q);
-            if (plain) break;
         }
         for (auto &kv : convq) {
             auto &v = kv.second;
