@@ -147,25 +147,28 @@ __global__ void pack_filters_kernel(const T *src, float2 *dst, int fh, int fw, i
 // Blocks of the pointwise kernels: 256 points of a plane times a tile of output maps, the tiles
 // of the same points next to each other, so that what they share comes from the caches.
 constexpr int kMapTile = 4;
+// Filters of at most this many taps a side go through the short-filter kernels.
+constexpr int kShortTaps = 32;
 
 struct MapAt {
     long long p;
     int a0, b0;  // first map of the tile along each of the two map axes
 };
 
+template <int TA, int TB, int PTS = 256>
 __device__ __forceinline__ MapAt map_at(int na, int nb)
 {
-    const unsigned ta = (na + kMapTile - 1) / kMapTile, tb = (nb + kMapTile - 1) / kMapTile;
+    const unsigned ta = (na + TA - 1) / TA, tb = (nb + TB - 1) / TB;
     unsigned r = blockIdx.x;
     const unsigned pb = r / (ta * tb);
     r -= pb * (ta * tb);
     const unsigned ia = r / tb;
-    return {(long long)pb * 256 + threadIdx.x, (int)ia * kMapTile, (int)(r - ia * tb) * kMapTile};
+    return {(long long)pb * PTS + threadIdx.x % PTS, (int)ia * TA, (int)(r - ia * tb) * TB};
 }
 
-static long long map_blocks(long long P, long long na, long long nb)
+static long long map_blocks(long long P, long long na, long long nb, int ta = kMapTile, int tb = kMapTile, int pts = 256)
 {
-    return (P + 255) / 256 * ((na + kMapTile - 1) / kMapTile) * ((nb + kMapTile - 1) / kMapTile);
+    return (P + pts - 1) / pts * ((na + ta - 1) / ta) * ((nb + tb - 1) / tb);
 }
 
 // Y[k][f][p] = sum_c X[k][c][p] * H[f][c][p]   (X, Y: FMT; H: fp32). A thread sums a tile of 4
@@ -175,7 +178,7 @@ template <int XFMT, int YFMT>
 __global__ void __launch_bounds__(256) pointwise_mac_kernel(const void *X, const float2 *H, void *Y, int pairs, int C, int F,
                                                             long long P)
 {
-    const MapAt m = map_at(pairs, F);
+    const MapAt m = map_at<kMapTile, kMapTile>(pairs, F);
     if (m.p >= P) return;
     const int nk = min(kMapTile, pairs - m.a0), nf = min(kMapTile, F - m.b0);
     float2 acc[kMapTile][kMapTile];
@@ -356,21 +359,23 @@ __global__ void crop_two_kernel(const void *Y, T *out0, T *out1, int oh, int ow,
 // where X_k = spectrum of the image pair (a + i b) and D_k of the delta pair (da + i db),
 // separated per frequency with X(-p): A = (X + X*)/2, B = (X - X*)/2i (X* = conj X(-p)).
 // Its inverse is sum_b in[b][c] (correlated with) delta[b][f], which is real: G(-p) = conj G(p),
-// so a thread computes a tile of 4 filters x 4 channels at one point of the upper half plane
+// so a thread computes a tile of TF filters x 4 channels at one point of the upper half plane
 // and stores both. Per-map threads over the whole plane re-read X and D for every map (4
-// pairs, 3 channels, 16 filters of 256 x 256: 28.9 -> 18.3 us).
+// pairs, 3 channels, 16 filters of 256 x 256: 28.9 -> 18.3 us; with TF = 2 and twice the blocks,
+// where 4 would give fewer than four a compute unit, 17.2).
+template <int TF>
 __global__ void __launch_bounds__(256) pointwise_gw_kernel(const float2 *X, const float2 *D, float2 *G, int pairs, int C, int F,
                                                            int Ph, int Pw)
 {
-    const MapAt m = map_at(F, C);
+    const MapAt m = map_at<TF, kMapTile>(F, C);
     if (m.p >= (long long)(Ph / 2 + 1) * Pw) return;
     const long long P = (long long)Ph * Pw;
     const unsigned u = (unsigned)m.p / (unsigned)Pw, v = (unsigned)m.p - u * (unsigned)Pw;
     const long long q = (long long)(u ? Ph - u : 0) * Pw + (v ? Pw - v : 0);
-    const int nf = min(kMapTile, F - m.a0), nc = min(kMapTile, C - m.b0);
-    float2 g[kMapTile][kMapTile];
+    const int nf = min(TF, F - m.a0), nc = min(kMapTile, C - m.b0);
+    float2 g[TF][kMapTile];
 #pragma unroll
-    for (int f = 0; f < kMapTile; ++f)
+    for (int f = 0; f < TF; ++f)
 #pragma unroll
         for (int c = 0; c < kMapTile; ++c) g[f][c] = make_float2(0.f, 0.f);
     for (int k = 0; k < pairs; ++k) {
@@ -385,7 +390,7 @@ __global__ void __launch_bounds__(256) pointwise_gw_kernel(const float2 *X, cons
                 B[c] = make_float2(0.5f * (xp.y + xq.y), -0.5f * (xp.x - xq.x));
             }
 #pragma unroll
-        for (int f = 0; f < kMapTile; ++f)
+        for (int f = 0; f < TF; ++f)
             if (f < nf) {
                 const float2 *d = D + ((long long)k * F + m.a0 + f) * P;
                 const float2 dp = d[m.p], dq = d[q];
@@ -403,7 +408,7 @@ __global__ void __launch_bounds__(256) pointwise_gw_kernel(const float2 *X, cons
     // the rows that mirror into themselves (0 and, when Ph is even, Ph / 2) store their own points
     const bool both = u != 0 && 2 * u != (unsigned)Ph;
 #pragma unroll
-    for (int f = 0; f < kMapTile; ++f)
+    for (int f = 0; f < TF; ++f)
 #pragma unroll
         for (int c = 0; c < kMapTile; ++c)
             if (f < nf && c < nc) {
@@ -415,20 +420,26 @@ __global__ void __launch_bounds__(256) pointwise_gw_kernel(const float2 *X, cons
 
 // Input gradient spectrum: R[k][c][p] = sum_f D_k[f][p] conj(H[f][c][p]) with H the spectrum
 // of the 180-degree rotated filter; conj(H) is the spectrum of a real signal, so the image
-// pair stays separable in the inverse. Tiles of 4 pairs x 4 channels, as pointwise_mac_kernel
-// (4 pairs, 3 channels, 16 filters of 256 x 256: 20.0 -> 17.2 us).
+// pair stays separable in the inverse. Tiles of 4 pairs x 4 channels, as pointwise_mac_kernel.
+// NS: the waves of a block share 256 / NS points and each sums every NS-th filter: a layer has
+// few input maps, so one thread per point leaves most of the device idle (4 pairs, 3 channels, 16
+// filters of 256 x 256, 256 blocks of one point per thread: 18.5 us, split four ways 13.2).
+template <int NS>
 __global__ void __launch_bounds__(256) pointwise_gi_kernel(const float2 *D, const float2 *H, float2 *R, int pairs, int C, int F,
                                                            long long P)
 {
-    const MapAt m = map_at(pairs, C);
-    if (m.p >= P) return;
+    constexpr int PTS = 256 / NS;
+    __shared__ float2 red[NS > 1 ? NS : 1][kMapTile * kMapTile][NS > 1 ? PTS : 1];
+    const MapAt m = map_at<kMapTile, kMapTile, PTS>(pairs, C);
+    const int part = NS > 1 ? (int)threadIdx.x / PTS : 0, lane = threadIdx.x % PTS;
+    const bool in = m.p < P;
     const int nk = min(kMapTile, pairs - m.a0), nc = min(kMapTile, C - m.b0);
     float2 acc[kMapTile][kMapTile];
 #pragma unroll
     for (int k = 0; k < kMapTile; ++k)
 #pragma unroll
         for (int c = 0; c < kMapTile; ++c) acc[k][c] = make_float2(0.f, 0.f);
-    for (int f = 0; f < F; ++f) {
+    for (int f = part; f < F && in; f += NS) {
         float2 d[kMapTile], h[kMapTile];
 #pragma unroll
         for (int k = 0; k < kMapTile; ++k)
@@ -445,11 +456,119 @@ __global__ void __launch_bounds__(256) pointwise_gi_kernel(const float2 *D, cons
                     acc[k][c].y += d[k].y * h[c].x - d[k].x * h[c].y;
                 }
     }
+    if constexpr (NS > 1) {
+        // wave w finishes the tile's pair w (NS = kMapTile)
+        static_assert(NS == kMapTile, "one pair per part");
 #pragma unroll
-    for (int k = 0; k < kMapTile; ++k)
+        for (int k = 0; k < kMapTile; ++k)
+#pragma unroll
+            for (int c = 0; c < kMapTile; ++c) red[part][k * kMapTile + c][lane] = acc[k][c];
+        __syncthreads();
+        if (!in || part >= nk) return;
 #pragma unroll
         for (int c = 0; c < kMapTile; ++c)
-            if (k < nk && c < nc) R[((long long)(m.a0 + k) * C + m.b0 + c) * P + m.p] = acc[k][c];
+            if (c < nc) {
+                float2 s = make_float2(0.f, 0.f);
+#pragma unroll
+                for (int w = 0; w < NS; ++w) {
+                    const float2 t = red[w][part * kMapTile + c][lane];
+                    s.x += t.x;
+                    s.y += t.y;
+                }
+                R[((long long)(m.a0 + part) * C + m.b0 + c) * P + m.p] = s;
+            }
+    } else {
+        if (!in) return;
+#pragma unroll
+        for (int k = 0; k < kMapTile; ++k)
+#pragma unroll
+            for (int c = 0; c < kMapTile; ++c)
+                if (k < nk && c < nc) R[((long long)(m.a0 + k) * C + m.b0 + c) * P + m.p] = acc[k][c];
+    }
+}
+
+// ---------------------------------------------------------------- short filters
+// A filter of fh x fw taps, fh far below Ph: its Ph x Pw spectrum is a product of two small DFT
+// matrices, H = Ey w Ex, which one kernel computes straight from the taps instead of a padded
+// plane going through a whole 2D transform. 48 filters of 13 x 13 on 256 x 256: 12.3 us, 2 TB/s of
+// spectra written (packing, rows and columns took 30.6 us). Up to 32 taps the 2 x 32 products a
+// point stay below the transform's passes over memory. The matrices are tables: ty[ky][y] = W_Ph^(ky y) (rows
+// of NR entries, ky <= Ph / 2) and tx[x][kx] = W_Pw^(x kx), evaluated in FP64 and rounded once.
+
+// One block: 64 columns kx and a strip of rows ky of one filter's spectrum. The waves transform
+// the taps' rows along x into LDS; then a lane keeps its column's NR sums in registers, and a wave
+// takes one row ky at a time, the row's factors in scalar registers. The filter is real: row Ph -
+// ky is stored from row ky's sums.
+template <typename T, int NR>
+__global__ void __launch_bounds__(256) filter_spectrum_kernel(const T *__restrict__ src, float2 *__restrict__ H,
+                                                              const float2 *__restrict__ ty, const float2 *__restrict__ tx,
+                                                              int fh, int fw, int Ph, int Pw, int rotate, int nkx, int nstrip)
+{
+    __shared__ float2 r[NR][64];
+    __shared__ float taps[kShortTaps][NR];  // the rotation undone
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const unsigned fk = blockIdx.x / (unsigned)nstrip;
+    const int strip = (int)(blockIdx.x - fk * (unsigned)nstrip);
+    const unsigned fc = fk / (unsigned)nkx;
+    const int kx = (int)(fk - fc * (unsigned)nkx) * 64 + lane, kxc = min(kx, Pw - 1);
+    const T *w = src + (long long)fc * fh * fw;
+    for (int i = threadIdx.x; i < fw * NR; i += 256) {
+        const int x = i / NR, y = i - x * NR;
+        const int sy = rotate ? fh - 1 - y : y, sx = rotate ? fw - 1 - x : x;
+        taps[x][y] = y < fh ? (float)w[sy * fw + sx] : 0.f;
+    }
+    __syncthreads();
+    {
+        float2 a[NR / 4];
+#pragma unroll
+        for (int j = 0; j < NR / 4; ++j) a[j] = make_float2(0.f, 0.f);
+#pragma unroll 4
+        for (int x = 0; x < fw; ++x) {
+            const float2 t = tx[(long long)x * Pw + kxc];
+#pragma unroll
+            for (int j = 0; j < NR / 4; ++j) {
+                const float v = taps[x][wave + 4 * j];
+                a[j].x += v * t.x;
+                a[j].y += v * t.y;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NR / 4; ++j) r[wave + 4 * j][lane] = a[j];
+    }
+    __syncthreads();
+    float2 v[NR];
+#pragma unroll
+    for (int y = 0; y < NR; ++y) v[y] = r[y][lane];
+    const int rows = Ph / 2 + 1, per = (rows + nstrip - 1) / nstrip;
+    const int end = min(rows, (strip + 1) * per);
+    float2 *h = H + (long long)fc * Ph * Pw;
+    const int mx = kx ? Pw - kx : 0;
+    typedef __attribute__((address_space(4))) const float cf;
+    for (int ky = strip * per + wave; ky < end; ky += 4) {
+        const cf *t = (const cf *)(ty + (long long)ky * NR);
+        float2 a = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int y = 0; y < NR; ++y) {
+            a.x += v[y].x * t[2 * y] - v[y].y * t[2 * y + 1];
+            a.y += v[y].x * t[2 * y + 1] + v[y].y * t[2 * y];
+        }
+        if (kx < Pw) {
+            h[(long long)ky * Pw + kx] = a;
+            if (ky != 0 && 2 * ky != Ph) h[(long long)(Ph - ky) * Pw + mx] = make_float2(a.x, -a.y);
+        }
+    }
+}
+
+// ty and tx of the short-filter kernels (tx: entry i = x * Pw + kx).
+__global__ void gen_dft_rows_kernel(float2 *out, int n, int pitch, long long count)
+{
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= count) return;
+    const long long a = i / pitch, b = i - a * pitch;
+    const long long e = a * b % n;
+    double sn, cs;
+    sincospi(2.0 * (double)e / (double)n, &sn, &cs);
+    out[i] = make_float2((float)cs, (float)-sn);
 }
 
 // out[b][c][y][x] = scale * (Re or Im) Y[b/2][c][(y + oy) mod Ph][(x + ox) mod Pw], oy < Ph and
@@ -587,21 +706,95 @@ hipError_t conv_crop(const void *Y, int fmt, void *out, int f64, int B, int F, i
     return launch_crop<FMT_C32>(Y, out, f64, B, F, oh, ow, Ph, Pw, oy, ox, scale, s, map_scale);
 }
 
+// Blocks below which a launch of 256-thread blocks leaves compute units idle.
+constexpr long long kFillBlocks = 1024;
+
 hipError_t conv_pointwise_gw(const float2 *X, const float2 *D, float2 *G, int pairs, int C, int F, int Ph, int Pw,
                              hipStream_t s)
 {
-    const long long blocks = map_blocks((long long)(Ph / 2 + 1) * Pw, F, C);
+    const long long P = (long long)(Ph / 2 + 1) * Pw;
+    const bool small = map_blocks(P, F, C) < kFillBlocks;
+    const long long blocks = map_blocks(P, F, C, small ? 2 : kMapTile);
     if (blocks > 0x7fffffffLL || (long long)Ph * Pw > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pointwise_gw_kernel, dim3((unsigned)blocks), dim3(256), 0, s, X, D, G, pairs, C, F, Ph, Pw);
+    const dim3 grid((unsigned)blocks), block(256);
+    if (small)
+        hipLaunchKernelGGL(pointwise_gw_kernel<2>, grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
+    else
+        hipLaunchKernelGGL(pointwise_gw_kernel<kMapTile>, grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
     return hipGetLastError();
 }
 
 hipError_t conv_pointwise_gi(const float2 *D, const float2 *H, float2 *R, long long pairs, int C, int F, long long P,
                              hipStream_t s)
 {
-    const long long blocks = map_blocks(P, pairs, C);
+    const bool split = F >= kMapTile && map_blocks(P, pairs, C) < kFillBlocks;
+    const long long blocks = map_blocks(P, pairs, C, kMapTile, kMapTile, split ? 256 / kMapTile : 256);
     if (blocks > 0x7fffffffLL || pairs > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pointwise_gi_kernel, dim3((unsigned)blocks), dim3(256), 0, s, D, H, R, (int)pairs, C, F, P);
+    const dim3 grid((unsigned)blocks), block(256);
+    if (split)
+        hipLaunchKernelGGL(pointwise_gi_kernel<kMapTile>, grid, block, 0, s, D, H, R, (int)pairs, C, F, P);
+    else
+        hipLaunchKernelGGL(pointwise_gi_kernel<1>, grid, block, 0, s, D, H, R, (int)pairs, C, F, P);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------- short filters, host side
+int conv_short_rows(int fh, int fw)
+{
+    if (fw > kShortTaps || fh > kShortTaps) return 0;
+    for (int nr : {4, 8, 12, 16, 24})
+        if (fh <= nr) return nr;
+    return kShortTaps;
+}
+
+hipError_t conv_short_tables(float2 *ty, float2 *tx, int nr, int fw, int Ph, int Pw, hipStream_t s)
+{
+    const long long ny = (long long)(Ph / 2 + 1) * nr, nx = (long long)fw * Pw;
+    hipLaunchKernelGGL(gen_dft_rows_kernel, dim3((unsigned)((ny + 255) / 256)), dim3(256), 0, s, ty, Ph, nr, ny);
+    hipLaunchKernelGGL(gen_dft_rows_kernel, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, s, tx, Pw, Pw, nx);
+    return hipGetLastError();
+}
+
+// Strips of rows per (filter, 64 columns): enough blocks to fill the device, at least 8 rows each.
+static int short_strips(long long planes, int Ph, int nkx)
+{
+    const long long want = (kFillBlocks + planes * nkx - 1) / (planes * nkx), most = (Ph / 2 + 1 + 7) / 8;
+    return (int)(want < most ? want : most);
+}
+
+template <typename T, int NR>
+static void launch_filter_spectrum(const T *src, float2 *H, const float2 *ty, const float2 *tx, unsigned grid, int fh, int fw,
+                                   int Ph, int Pw, int rotate, int nkx, int nstrip, hipStream_t s)
+{
+    hipLaunchKernelGGL((filter_spectrum_kernel<T, NR>), dim3(grid), dim3(256), 0, s, src, H, ty, tx, fh, fw, Ph, Pw, rotate, nkx,
+                       nstrip);
+}
+
+hipError_t conv_filter_spectrum(const void *src, int f64, float2 *H, const float2 *ty, const float2 *tx, int nr, int FC, int fh,
+                                int fw, int Ph, int Pw, int rotate, hipStream_t s)
+{
+    const int nkx = (Pw + 63) / 64, ns = short_strips(FC, Ph, nkx);
+    const long long blocks = (long long)FC * nkx * ns;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+#define MFFT_SHORT_CASE(n)                                                                                                      \
+    case n:                                                                                                                     \
+        if (f64)                                                                                                                \
+            launch_filter_spectrum<double, n>((const double *)src, H, ty, tx, (unsigned)blocks, fh, fw, Ph, Pw, rotate, nkx,    \
+                                              ns, s);                                                                           \
+        else                                                                                                                    \
+            launch_filter_spectrum<float, n>((const float *)src, H, ty, tx, (unsigned)blocks, fh, fw, Ph, Pw, rotate, nkx, ns,  \
+                                             s);                                                                                \
+        break
+    switch (nr) {
+    MFFT_SHORT_CASE(4);
+    MFFT_SHORT_CASE(8);
+    MFFT_SHORT_CASE(12);
+    MFFT_SHORT_CASE(16);
+    MFFT_SHORT_CASE(24);
+    MFFT_SHORT_CASE(kShortTaps);
+    default: return hipErrorInvalidValue;
+    }
+#undef MFFT_SHORT_CASE
     return hipGetLastError();
 }
 

@@ -35,6 +35,11 @@ hipError_t conv_pointwise_gw(const float2 *X, const float2 *D, float2 *G, int pa
                              hipStream_t s);
 hipError_t conv_pointwise_gi(const float2 *D, const float2 *H, float2 *R, long long pairs, int C, int F, long long P,
                              hipStream_t s);
+// short filters: table rows of a filter height (0: not short), tables, spectra
+int conv_short_rows(int fh, int fw);
+hipError_t conv_short_tables(float2 *ty, float2 *tx, int nr, int fw, int Ph, int Pw, hipStream_t s);
+hipError_t conv_filter_spectrum(const void *src, int f64, float2 *H, const float2 *ty, const float2 *tx, int nr, int FC, int fh,
+                                int fw, int Ph, int Pw, int rotate, hipStream_t s);
 hipError_t conv_crop_cyclic(const float2 *Y, void *out, int f64, int B, int C, int oh, int ow, int Ph, int Pw, int oy,
                             int ox, float scale, hipStream_t s);
 hipError_t conv_crop_real(const float2 *Y, void *out, int f64, long long planes, int oh, int ow, int Ph, int Pw,
@@ -69,6 +74,10 @@ struct mfft_conv2d_s {
     // and (pair, channel) batches, and the filter-gradient spectra
     mfft_plan fwd_delta = nullptr, inv_fc = nullptr, inv_pc = nullptr;
     float2 *G = nullptr;
+    // short filters: entries a row of ty has (0: the filters go through padded transforms) and
+    // the tables
+    int short_rows = 0;
+    float2 *ty = nullptr, *tx = nullptr;
     bool have_filters = false;
     long long bytes = 0, spec_bytes = 0;
     std::mutex mu;
@@ -154,6 +163,8 @@ int mfft_conv2d_destroy(mfft_conv2d op)
     for (mfft_plan p : {op->fwd_delta, op->inv_fc, op->inv_pc})
         if (p) mfft_plan_destroy(p);
     (void)hipFree(op->G);
+    (void)hipFree(op->ty);
+    (void)hipFree(op->tx);
     (void)hipFree(op->H);
     (void)hipFree(op->X);
     (void)hipFree(op->Y);
@@ -237,7 +248,11 @@ int mfft_conv2d_create(mfft_conv2d *out, const mfft_conv2d_desc *d)
         fd.out_fmt = op->spec_fmt;
     }
     op->res_fmt = op->mid16 ? MFFT_FMT_C16 : op->spec_fmt;
-    if (!rc) {
+    // (with 16-bit words anywhere in the images' path a filter spectrum that differs in its last
+    // bits is rounded apart by whole fp16 steps later: those operators keep the transforms)
+    op->short_rows = op->spec_fmt == MFFT_FMT_C32 && !op->mid16 && d->precision == MFFT_PREC_SPLIT_FP16
+                         ? mfft::conv_short_rows(d->fh, d->fw) : 0;
+    if (!rc && !op->short_rows) {
         // the resident filter spectra stay fp32 whatever the image spectra
         fd.direction = MFFT_FORWARD;
         fd.in_fmt = fd.out_fmt = MFFT_FMT_C32;
@@ -260,6 +275,20 @@ int mfft_conv2d_create(mfft_conv2d *out, const mfft_conv2d_desc *d)
         return cfail(MFFT_ERR_NOMEM, "conv buffers (%lld + %lld + %lld bytes)", op->spec_bytes, xb, yb);
     }
     op->bytes = op->spec_bytes + xb + yb;
+    if (op->short_rows) {
+        const long long ty = (long long)(op->Ph / 2 + 1) * op->short_rows * 8, tx = (long long)d->fw * op->Pw * 8;
+        if (hipMalloc(&op->ty, ty) != hipSuccess || hipMalloc(&op->tx, tx) != hipSuccess) {
+            mfft_conv2d_destroy(op);
+            return cfail(MFFT_ERR_NOMEM, "filter tables (%lld bytes)", ty + tx);
+        }
+        // made before the call returns: any stream may use the operator next
+        if (mfft::conv_short_tables(op->ty, op->tx, op->short_rows, d->fw, op->Ph, op->Pw, 0) != hipSuccess ||
+            hipStreamSynchronize(0) != hipSuccess) {
+            mfft_conv2d_destroy(op);
+            return cfail(MFFT_ERR_HIP, "filter tables");
+        }
+        op->bytes += ty + tx;
+    }
     if (op->refq) {
         // quantised product spectra, one scale per map, chunk maxima (one chunk per 16K values)
         op->qchunks = (int)std::max(1LL, std::min(256LL, P / 16384));
@@ -273,7 +302,7 @@ int mfft_conv2d_create(mfft_conv2d *out, const mfft_conv2d_desc *d)
     }
     mfft_info inf;
     for (mfft_plan p : {op->fwd_img, op->fwd_filt, op->inv})
-        if (!mfft_plan_info(p, &inf)) op->bytes += inf.workspace_bytes;
+        if (p && !mfft_plan_info(p, &inf)) op->bytes += inf.workspace_bytes;
     *out = op;
     return MFFT_OK;
 }
@@ -285,6 +314,16 @@ int mfft_conv2d_set_filters(mfft_conv2d op, const void *filters, int real_fmt, v
     OpCall call(op, s);
     if (call.err != hipSuccess) return cfail(MFFT_ERR_HIP, "stream order: %s", hipGetErrorString(call.err));
     const mfft_conv2d_desc &d = op->d;
+    if (op->short_rows) {
+        mfft::trace_launch(s, "conv_filter_spectrum", (long long)d.filters * d.channels * d.fh * d.fw * (real_fmt == MFFT_REAL_F64 ? 8 : 4),
+                           op->spec_bytes);
+        if (mfft::conv_filter_spectrum(filters, real_fmt == MFFT_REAL_F64, op->H, op->ty, op->tx, op->short_rows,
+                                       d.filters * d.channels, d.fh, d.fw, op->Ph, op->Pw, d.mode == MFFT_CONV_VALID_CORR, s) !=
+            hipSuccess)
+            return cfail(MFFT_ERR_HIP, "filter spectra");
+        op->have_filters = true;
+        return MFFT_OK;
+    }
     mfft::trace_launch(s, "conv_pack_filters", (long long)d.filters * d.channels * d.fh * d.fw * (real_fmt == MFFT_REAL_F64 ? 8 : 4),
                        op->spec_bytes);
     if (mfft::conv_pack_filters(filters, real_fmt == MFFT_REAL_F64, op->H, d.filters * d.channels, d.fh, d.fw, op->Ph,
@@ -471,6 +510,31 @@ static int backward_setup(mfft_conv2d op)
     return MFFT_OK;
 }
 
+// Spectra of a batch of real planes [batch][maps][h][w], in pairs, zero-padded: from the planes
+// themselves where the transform's first pass reads them, else through a packing pass.
+static int image_spectra(mfft_conv2d op, mfft_plan plan, const void *src, int f64, int maps, int h, int w, float2 *dst,
+                         hipStream_t s)
+{
+    int rc;
+    if (mfft::plan_first_pass_fusable(plan)) {
+        mfft::ExecFuse f;
+        f.real_src = src;
+        f.real_f64 = f64;
+        f.real_b = op->d.batch;
+        f.real_c = maps;
+        f.real_h = h;
+        f.real_w = w;
+        rc = mfft::exec_fused(plan, dst, dst, op->pairs * maps, s, f);
+    } else {
+        mfft::trace_launch(s, "conv_pack", (long long)op->d.batch * maps * h * w * (f64 ? 8 : 4),
+                           op->pairs * maps * (long long)op->Ph * op->Pw * 8);
+        if (mfft::conv_pack_pairs(src, f64, dst, MFFT_FMT_C32, op->d.batch, maps, h, w, op->Ph, op->Pw, s) != hipSuccess)
+            return cfail(MFFT_ERR_HIP, "pack");
+        rc = mfft_exec(plan, dst, dst, s);
+    }
+    return rc ? cfail(rc, "%s", mfft_last_error()) : MFFT_OK;
+}
+
 int mfft_conv2d_backward(mfft_conv2d op, const void *in, const void *delta, int real_fmt, void *grad_in, void *grad_w,
                          void *stream)
 {
@@ -488,27 +552,20 @@ int mfft_conv2d_backward(mfft_conv2d op, const void *in, const void *delta, int 
     const int f64 = real_fmt == MFFT_REAL_F64;
     const long long P = (long long)op->Ph * op->Pw;
     // delta spectra (scaled 1/P) in Y
-    mfft::trace_launch(s, "conv_pack", (long long)d.batch * d.filters * op->oh * op->ow * (f64 ? 8 : 4),
-                       op->pairs * d.filters * P * 8);
-    if (mfft::conv_pack_pairs(delta, f64, op->Y, MFFT_FMT_C32, d.batch, d.filters, op->oh, op->ow, op->Ph, op->Pw, s) !=
-        hipSuccess)
-        return cfail(MFFT_ERR_HIP, "pack delta");
-    rc = mfft_exec(op->fwd_delta, op->Y, op->Y, s);
-    if (rc) return cfail(rc, "%s", mfft_last_error());
+    rc = image_spectra(op, op->fwd_delta, delta, f64, d.filters, op->oh, op->ow, op->Y, s);
+    if (rc) return rc;
     if (grad_w) {
-        mfft::trace_launch(s, "conv_pack", (long long)d.batch * d.channels * d.h * d.w * (f64 ? 8 : 4),
-                           op->pairs * d.channels * P * 8);
-        if (mfft::conv_pack_pairs(in, f64, op->X, MFFT_FMT_C32, d.batch, d.channels, d.h, d.w, op->Ph, op->Pw, s) !=
-            hipSuccess)
-            return cfail(MFFT_ERR_HIP, "pack input");
-        rc = mfft_exec(op->fwd_img, op->X, op->X, s);
-        if (rc) return cfail(rc, "%s", mfft_last_error());
+        rc = image_spectra(op, op->fwd_img, in, f64, d.channels, d.h, d.w, op->X, s);
+        if (rc) return rc;
         mfft::trace_launch(s, "conv_pointwise_gw", op->pairs * (d.channels + d.filters) * P * 8,
                            (long long)d.filters * d.channels * P * 8);
         if (mfft::conv_pointwise_gw(op->X, op->Y, op->G, (int)op->pairs, d.channels, d.filters, op->Ph, op->Pw, s) !=
             hipSuccess)
             return cfail(MFFT_ERR_HIP, "pointwise (filter gradient)");
-        rc = mfft_exec(op->inv_fc, op->G, op->G, s);
+        // the window is fw columns wide: the column passes transform those only
+        mfft::ExecFuse fw;
+        fw.cols = d.fw;
+        rc = mfft::exec_fused(op->inv_fc, op->G, op->G, (int64_t)d.filters * d.channels, s, fw);
         if (rc) return cfail(rc, "%s", mfft_last_error());
         // both spectra carry 1/P and the unnormalised inverse one factor P back
         mfft::trace_launch(s, "conv_crop_real", (long long)d.filters * d.channels * d.fh * d.fw * 8,

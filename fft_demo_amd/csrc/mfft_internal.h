@@ -17,6 +17,10 @@ struct ExecFuse {
     const void *real_src = nullptr;
     const void *real_src2 = nullptr;  // imaginary part from a second single image
     int real_f64 = 0, real_b = 0, real_c = 0, real_h = 0, real_w = 0;
+    // 2D plans, any first pass: the column passes transform the first `cols` columns only (the
+    // rest of the output is left undefined); 0 = all
+    int cols = 0;
+    bool input() const { return in_mul || real_src; }  // needs a first pass that takes it
 };
 
 // mfft_plan_create_2d for the conv operator: odd axes keep the streaming pass that takes an
@@ -28,8 +32,8 @@ int plan_create_2d_conv(mfft_plan *plan, int nx, int ny, int64_t batch, const mf
 
 // Whether the plan's first pass can take an ExecFuse.
 bool plan_first_pass_fusable(mfft_plan p);
-// mfft_exec_ex with the fused first pass (no caller workspace); MFFT_ERR_UNSUPPORTED when
-// the first pass is not fusable.
+// mfft_exec_ex with an ExecFuse (no caller workspace); MFFT_ERR_UNSUPPORTED when it fuses the
+// input and the first pass does not take that.
 int exec_fused(mfft_plan p, const void *in, void *out, int64_t batch, void *stream, const ExecFuse &f);
 
 // Set the calling thread's message returned by mfft_last_error().

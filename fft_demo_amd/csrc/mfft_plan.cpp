@@ -218,6 +218,7 @@ struct PassSpec {
     bool onchip_cols = false;  // 2048-point lines, 32 per workgroup (fft_onchip_cols)
     bool onchip_rows = false;  // ... contiguous lines stored transposed (its rows kind)
     bool mixed = false;     // lines on the mixed-radix kernels (fft_mixed, fft_mixed_cols)
+    bool col_axis = false;  // a pass of a 2D plan's column axis
     int mixed_cap = 0;      // strided lines: points per tile at most; 0 = dense contiguous lines
     MixSched mix{};
 };
@@ -1012,6 +1013,9 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
         a.TL = ps.TL;
         auto cnt = [&](int li) -> long long {
             if (li < 0) return 1;
+            // a pass of the column axis: the level of the columns
+            if (fz && fz->cols && ps.col_axis && ps.lines[li].in_stride == 1 && !ps.lines[li].batch)
+                return std::min<long long>(ps.lines[li].count, fz->cols);
             return ps.lines[li].batch ? nb : ps.lines[li].count;
         };
         a.c0 = (int)cnt(ps.l0);
@@ -1343,6 +1347,7 @@ static int create_2d(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_
     const int odd_hint = d->split_hint == 1 ? 1 : 0;  // 1 keeps odd * 2^a axes in one pass
     rc = plan_axis(p->passes, ny, 1, 1, rows, BUF_IN, BUF_WORK, rev ? 1 : -1, odd_hint, narrow_mid(d), false,
                    !conv && find_mixed_kernel(d->precision, d->in_fmt, col_in_fmt) ? d->precision : -1);
+    const size_t nrow_passes = p->passes.size();
     // columns (x axis, stride ny): lines = (y, b)
     if (!rc) {
         // split_hint > 1: the first-pass length of the column axis when it is split
@@ -1369,6 +1374,7 @@ static int create_2d(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_
                            !conv && find_mixed_kernel(d->precision, col_in_fmt, d->out_fmt) ? d->precision : -1);
         }
     }
+    for (size_t i = nrow_passes; i < p->passes.size(); ++i) p->passes[i].col_axis = true;
     p->out_mid = out_mid;
     if (!rc) rc = finalize_plan(p);
     if (rc) {
@@ -1466,7 +1472,7 @@ static int exec_all(mfft_plan p, const void *in, void *out, void *stream, hipEve
                     hipEvent_t kstart = nullptr, hipEvent_t kstop = nullptr)
 {
     if (p->small && batch >= 0 && batch < p->small_below && only < 0 && !ev &&
-        (!fz || (p->small->passes.front().small && p->small->passes.front().src == BUF_IN)))
+        (!fz || !fz->input() || (p->small->passes.front().small && p->small->passes.front().src == BUF_IN)))
         return exec_all(p->small, in, out, stream, nullptr, batch, work, fz, -1, nullptr, nullptr);
     if (p->out_mid && in == out)
         for (const PassSpec &ps : p->passes) {
@@ -2036,7 +2042,7 @@ bool plan_first_pass_fusable(mfft_plan p)
 
 int exec_fused(mfft_plan p, const void *in, void *out, int64_t batch, void *stream, const ExecFuse &f)
 {
-    if (!plan_first_pass_fusable(p)) return fail(MFFT_ERR_UNSUPPORTED, "first pass takes no fused input");
+    if (f.input() && !plan_first_pass_fusable(p)) return fail(MFFT_ERR_UNSUPPORTED, "first pass takes no fused input");
     if (batch < 1 || batch > p->batch) return fail(MFFT_ERR_INVALID, "batch %lld outside 1..%lld", (long long)batch, p->batch);
     return exec_all(p, in, out, stream, nullptr, batch, nullptr, &f);
 }
