@@ -108,6 +108,16 @@ struct TileArgs {
     const void *real_src2;     // set: the imaginary part comes from this second image instead
     int real_f64, real_b, real_c, real_h, real_w, real_pw;
     long long real_p, batch_base;
+    // last pass of a 2D plan, fused crop (fast strided kernel with crop_out set): point (y, x) of
+    // transform m = crop_c k + c is stored as real planes: its real part, times crop_mul, at row
+    // (y - crop_y) mod R and column (x - crop_x) mod c0 of plane [2k][c] of [crop_b][crop_c][crop_h]
+    // [crop_w], its imaginary part in plane [2k + 1][c] (absent past the batch), what lies outside
+    // the plane nowhere. crop_b = 0: plane m from the real part alone.
+    float *crop_out;
+    int crop_b, crop_c, crop_h, crop_w, crop_y, crop_x;
+    unsigned crop_span;        // bytes of crop_out, below 2^31
+    unsigned real_span;        // fast kernels: bytes of real_src (fp32), below 2^31
+    float crop_mul;
     // fast kernels, digit-reversed input (the order of tcfftExec, gen_rev of a radix list
     // whose first radix is 16): natural point col + (R/16) j of a line is stored at point
     // position j + 16 * digit_rev(col, in_rev), so each lane's four first-stage operands

@@ -335,6 +335,49 @@ int mfft_conv2d_set_filters(mfft_conv2d op, const void *filters, int real_fmt, v
     return MFFT_OK;
 }
 
+// Spectra of a batch of real planes [batch][maps][h][w], in pairs, zero-padded: from the planes
+// themselves where the transform's first pass reads them, else through a packing pass.
+static int image_spectra(mfft_conv2d op, mfft_plan plan, const void *src, int f64, int maps, int h, int w, void *dst,
+                         hipStream_t s)
+{
+    int rc;
+    if (mfft::plan_takes_real(plan, f64, (long long)op->d.batch * maps, h, w)) {
+        mfft::ExecFuse f;
+        f.real_src = src;
+        f.real_f64 = f64;
+        f.real_b = op->d.batch;
+        f.real_c = maps;
+        f.real_h = h;
+        f.real_w = w;
+        rc = mfft::exec_fused(plan, dst, dst, op->pairs * maps, s, f);
+    } else {
+        // with 16-bit boundaries out of place: Y holds at least as many spectra as X (one channel)
+        void *packed = op->mid16 ? (void *)op->Y : dst;
+        mfft::trace_launch(s, "conv_pack", (long long)op->d.batch * maps * h * w * (f64 ? 8 : 4),
+                           op->pairs * maps * (long long)op->Ph * op->Pw * spec_eb(op));
+        if (mfft::conv_pack_pairs(src, f64, packed, op->spec_fmt, op->d.batch, maps, h, w, op->Ph, op->Pw, s) != hipSuccess)
+            return cfail(MFFT_ERR_HIP, "pack");
+        rc = mfft_exec(plan, packed, dst, s);
+    }
+    return rc ? cfail(rc, "%s", mfft_last_error()) : MFFT_OK;
+}
+
+// Whether an inverse's last pass stores its real planes [batch][maps][oh][ow], read at the cyclic
+// offset (oy, ox), itself; f then says so.
+static bool fuse_crop(mfft_conv2d op, mfft_plan plan, void *out, int f64, int maps, int oh, int ow, int oy, int ox,
+                      mfft::ExecFuse &f)
+{
+    if (!mfft::plan_takes_crop(plan, f64, (long long)op->d.batch * maps, oh, ow)) return false;
+    f.crop_out = (float *)out;
+    f.crop_b = op->d.batch;
+    f.crop_c = maps;
+    f.crop_h = oh;
+    f.crop_w = ow;
+    f.crop_y = oy % op->Ph;
+    f.crop_x = ox % op->Pw;
+    return true;
+}
+
 static int conv_run(mfft_conv2d op, const void *in, int in_fmt, void *out, int out_fmt, int fsel, void *stream)
 {
     if (!op || !in || !out) return cfail(MFFT_ERR_INVALID, "null argument");
@@ -346,28 +389,8 @@ static int conv_run(mfft_conv2d op, const void *in, int in_fmt, void *out, int o
     OpCall call(op, s);
     if (call.err != hipSuccess) return cfail(MFFT_ERR_HIP, "stream order: %s", hipGetErrorString(call.err));
     const mfft_conv2d_desc &d = op->d;
-    int rc;
-    if (mfft::plan_first_pass_fusable(op->fwd_img)) {
-        // the forward transform's first pass reads the real images, zero-padded
-        mfft::ExecFuse f;
-        f.real_src = in;
-        f.real_f64 = in_fmt == MFFT_REAL_F64;
-        f.real_b = d.batch;
-        f.real_c = d.channels;
-        f.real_h = d.h;
-        f.real_w = d.w;
-        rc = mfft::exec_fused(op->fwd_img, op->X, op->X, op->pairs * d.channels, s, f);
-    } else {
-        // Y holds at least as many spectra as X (one channel whenever mid16)
-        void *packed = op->mid16 ? (void *)op->Y : (void *)op->X;
-        mfft::trace_launch(s, "conv_pack", (long long)d.batch * d.channels * d.h * d.w * (in_fmt == MFFT_REAL_F64 ? 8 : 4),
-                           op->pairs * d.channels * (long long)op->Ph * op->Pw * spec_eb(op));
-        if (mfft::conv_pack_pairs(in, in_fmt == MFFT_REAL_F64, packed, op->spec_fmt, d.batch, d.channels, d.h, d.w,
-                                  op->Ph, op->Pw, s) != hipSuccess)
-            return cfail(MFFT_ERR_HIP, "pack");
-        rc = mfft_exec(op->fwd_img, packed, op->X, s);
-    }
-    if (rc) return cfail(rc, "%s", mfft_last_error());
+    int rc = image_spectra(op, op->fwd_img, in, in_fmt == MFFT_REAL_F64, d.channels, d.h, d.w, op->X, s);
+    if (rc) return rc;
     const long long P = (long long)op->Ph * op->Pw;
     const int nf = fsel >= 0 ? 1 : d.filters;
     const float2 *H = fsel >= 0 ? op->H + (long long)fsel * d.channels * P : op->H;
@@ -392,9 +415,10 @@ static int conv_run(mfft_conv2d op, const void *in, int in_fmt, void *out, int o
             return cfail(MFFT_ERR_HIP, "crop");
         return MFFT_OK;
     }
+    mfft::ExecFuse f;
+    const bool cropped = fuse_crop(op, op->inv, out, out_fmt == MFFT_REAL_F64, nf, op->oh, op->ow, op->oy, op->ox, f);
     if (d.channels == 1 && nf == 1 && mfft::plan_first_pass_fusable(op->inv)) {
         // one filter, one channel: the inverse's first pass multiplies by the spectrum
-        mfft::ExecFuse f;
         f.in_mul = H;
         f.in_mul_period = P;
         rc = mfft::exec_fused(op->inv, op->X, op->Y, op->pairs, s, f);
@@ -404,9 +428,10 @@ static int conv_run(mfft_conv2d op, const void *in, int in_fmt, void *out, int o
         if (mfft::conv_pointwise(op->X, H, op->Y, op->spec_fmt, op->pairs, d.channels, nf, P, s) != hipSuccess)
             return cfail(MFFT_ERR_HIP, "pointwise");
         if (op->mid16) res = op->X;  // out of place; X holds pairs x 1 spectra and nf == 1 here
-        rc = mfft_exec_ex(op->inv, op->Y, res, op->pairs * nf, nullptr, s);
+        rc = mfft::exec_fused(op->inv, op->Y, res, op->pairs * nf, s, f);
     }
     if (rc) return cfail(rc, "%s", mfft_last_error());
+    if (cropped) return MFFT_OK;
     mfft::trace_launch(s, "conv_crop", op->pairs * nf * (long long)op->oh * op->ow * (op->res_fmt == MFFT_FMT_C16 ? 4 : 8),
                        (long long)d.batch * nf * op->oh * op->ow * (out_fmt == MFFT_REAL_F64 ? 8 : 4));
     if (mfft::conv_crop(res, op->res_fmt, out, out_fmt == MFFT_REAL_F64, d.batch, nf, op->oh, op->ow, op->Ph,
@@ -510,31 +535,6 @@ static int backward_setup(mfft_conv2d op)
     return MFFT_OK;
 }
 
-// Spectra of a batch of real planes [batch][maps][h][w], in pairs, zero-padded: from the planes
-// themselves where the transform's first pass reads them, else through a packing pass.
-static int image_spectra(mfft_conv2d op, mfft_plan plan, const void *src, int f64, int maps, int h, int w, float2 *dst,
-                         hipStream_t s)
-{
-    int rc;
-    if (mfft::plan_first_pass_fusable(plan)) {
-        mfft::ExecFuse f;
-        f.real_src = src;
-        f.real_f64 = f64;
-        f.real_b = op->d.batch;
-        f.real_c = maps;
-        f.real_h = h;
-        f.real_w = w;
-        rc = mfft::exec_fused(plan, dst, dst, op->pairs * maps, s, f);
-    } else {
-        mfft::trace_launch(s, "conv_pack", (long long)op->d.batch * maps * h * w * (f64 ? 8 : 4),
-                           op->pairs * maps * (long long)op->Ph * op->Pw * 8);
-        if (mfft::conv_pack_pairs(src, f64, dst, MFFT_FMT_C32, op->d.batch, maps, h, w, op->Ph, op->Pw, s) != hipSuccess)
-            return cfail(MFFT_ERR_HIP, "pack");
-        rc = mfft_exec(plan, dst, dst, s);
-    }
-    return rc ? cfail(rc, "%s", mfft_last_error()) : MFFT_OK;
-}
-
 int mfft_conv2d_backward(mfft_conv2d op, const void *in, const void *delta, int real_fmt, void *grad_in, void *grad_w,
                          void *stream)
 {
@@ -563,28 +563,41 @@ int mfft_conv2d_backward(mfft_conv2d op, const void *in, const void *delta, int 
             hipSuccess)
             return cfail(MFFT_ERR_HIP, "pointwise (filter gradient)");
         // the window is fw columns wide: the column passes transform those only
-        mfft::ExecFuse fw;
-        fw.cols = d.fw;
-        rc = mfft::exec_fused(op->inv_fc, op->G, op->G, (int64_t)d.filters * d.channels, s, fw);
+        mfft::ExecFuse f;
+        f.cols = d.fw;
+        const long long fc = (long long)d.filters * d.channels;
+        const bool cropped = mfft::plan_takes_crop(op->inv_fc, f64, fc, d.fh, d.fw);
+        if (cropped) {
+            f.crop_out = (float *)grad_w;
+            f.crop_c = 1;
+            f.crop_h = d.fh;
+            f.crop_w = d.fw;
+            // both spectra carry 1/P and the unnormalised inverse one factor P back
+            f.crop_mul = (float)P;
+        }
+        rc = mfft::exec_fused(op->inv_fc, op->G, op->G, fc, s, f);
         if (rc) return cfail(rc, "%s", mfft_last_error());
-        // both spectra carry 1/P and the unnormalised inverse one factor P back
-        mfft::trace_launch(s, "conv_crop_real", (long long)d.filters * d.channels * d.fh * d.fw * 8,
-                           (long long)d.filters * d.channels * d.fh * d.fw * (f64 ? 8 : 4));
-        if (mfft::conv_crop_real(op->G, grad_w, f64, (long long)d.filters * d.channels, d.fh, d.fw, op->Ph, op->Pw,
-                                 (float)P, s) != hipSuccess)
-            return cfail(MFFT_ERR_HIP, "crop (filter gradient)");
+        if (!cropped) {
+            mfft::trace_launch(s, "conv_crop_real", fc * d.fh * d.fw * 8, fc * d.fh * d.fw * (f64 ? 8 : 4));
+            if (mfft::conv_crop_real(op->G, grad_w, f64, fc, d.fh, d.fw, op->Ph, op->Pw, (float)P, s) != hipSuccess)
+                return cfail(MFFT_ERR_HIP, "crop (filter gradient)");
+        }
     }
     if (grad_in) {
         mfft::trace_launch(s, "conv_pointwise_gi", op->pairs * d.filters * P * 8 + (long long)d.filters * d.channels * P * 8,
                            op->pairs * d.channels * P * 8);
         if (mfft::conv_pointwise_gi(op->Y, op->H, op->X, op->pairs, d.channels, d.filters, P, s) != hipSuccess)
             return cfail(MFFT_ERR_HIP, "pointwise (input gradient)");
-        rc = mfft_exec(op->inv_pc, op->X, op->X, s);
+        mfft::ExecFuse f;
+        const int oy = op->Ph - (d.fh - 1), ox = op->Pw - (d.fw - 1);
+        const bool cropped = fuse_crop(op, op->inv_pc, grad_in, f64, d.channels, d.h, d.w, oy, ox, f);
+        rc = mfft::exec_fused(op->inv_pc, op->X, op->X, op->pairs * d.channels, s, f);
         if (rc) return cfail(rc, "%s", mfft_last_error());
+        if (cropped) return MFFT_OK;
         mfft::trace_launch(s, "conv_crop_cyclic", op->pairs * d.channels * (long long)d.h * d.w * 8,
                            (long long)d.batch * d.channels * d.h * d.w * (f64 ? 8 : 4));
-        if (mfft::conv_crop_cyclic(op->X, grad_in, f64, d.batch, d.channels, d.h, d.w, op->Ph, op->Pw,
-                                   op->Ph - (d.fh - 1), op->Pw - (d.fw - 1), 1.0f, s) != hipSuccess)
+        if (mfft::conv_crop_cyclic(op->X, grad_in, f64, d.batch, d.channels, d.h, d.w, op->Ph, op->Pw, oy, ox, 1.0f, s) !=
+            hipSuccess)
             return cfail(MFFT_ERR_HIP, "crop (input gradient)");
     }
     return MFFT_OK;

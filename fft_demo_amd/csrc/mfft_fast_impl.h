@@ -264,6 +264,47 @@ __device__ __forceinline__ void dft16(const float2 *x, const h8 &raw16, const b8
     }
 }
 
+// ------------------------------------------------------------------ fused ends
+// Both ends go through a buffer resource that spans the whole tensor: an element outside a plane
+// (padding on the way in, what the crop drops on the way out) takes an offset past the resource's
+// end, which reads as zero and drops the store, so neither end needs execution masks. 64 maps of 256
+// x 256: rows from real planes 15.0 us (packing 13.9 + rows 11.8), columns into real planes 16.7
+// (columns 15.1 + crop 9.9).
+constexpr unsigned kOutside = 0x80000000u;
+
+struct PlanePair {
+    __amdgpu_buffer_rsrc_t rsrc;
+    unsigned first, second;  // byte offsets of the two planes
+};
+
+// Planes of transform m of [b][c][h][w] fp32; b = 0: plane m alone.
+__device__ __forceinline__ PlanePair plane_pair(const void *base, unsigned span, unsigned m, int b, int c, int h, int w)
+{
+    const unsigned k = m / (unsigned)c, hw = 4u * (unsigned)h * (unsigned)w;
+    PlanePair p;
+    p.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)span, 0x00020000);
+    p.first = b ? (k * (unsigned)c + m) * hw : m * hw;  // (2k c + m - k c) planes before it
+    p.second = 2 * (int)k + 1 < b ? p.first + (unsigned)c * hw : kOutside;
+    return p;
+}
+
+__device__ __forceinline__ void crop_store(const TileArgs &a, const PlanePair &pp, int R, int xx, int pt, float2 v)
+{
+    int yy = pt - a.crop_y;
+    yy += yy < 0 ? R : 0;
+    const bool ok = yy < a.crop_h && xx < a.crop_w;
+    const unsigned o = 4u * ((unsigned)yy * (unsigned)a.crop_w + (unsigned)xx);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v.x * a.crop_mul), pp.rsrc, (int)(ok ? pp.first + o : kOutside), 0, 0);
+    if (pp.second != kOutside)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v.y * a.crop_mul), pp.rsrc, (int)(ok ? pp.second + o : kOutside), 0, 0);
+}
+
+__device__ __forceinline__ int crop_col(const TileArgs &a, int x)
+{
+    x -= a.crop_x;
+    return x + (x < 0 ? a.c0 : 0);
+}
+
 // Wait for every outstanding vector-memory operation of this wave. Called in the last stage
 // before the tile's stores: what is then outstanding is the next tile's prefetch (issued a
 // whole tile earlier) and the previous tile's stores. Loads and stores share the counter,
@@ -289,12 +330,38 @@ struct Prefetch {
     // digit-reversed order (TileArgs::rev_input): the lane's four operands of a group,
     // natural points col + R16 (4g + i), sit at the consecutive positions
     // 16 digit_rev(col) + 4g + i.
-    template <bool FULL, bool REV = false>
+    template <bool FULL, bool REV = false, int ENDS = ENDS_PLAIN>
     __device__ __forceinline__ void load(const TileArgs &a, const Origin &o)
     {
         constexpr int MAP = KIND == KIND_COLS ? MAP_LINES : MAP_POINTS;
         constexpr int R16 = G::R16;
         const raw *src = reinterpret_cast<const raw *>(a.in);
+        if constexpr (ENDS == ENDS_REAL) {
+            const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+            const int g = lane >> 4, c = lane & 15;
+            const PlanePair pp = plane_pair(a.real_src, a.real_span, (unsigned)((int)a.batch_base + o.l1), a.real_b, a.real_c,
+                                            a.real_h, a.real_w);
+#pragma unroll
+            for (int u = 0; u < G::MAXP; ++u) {
+                const int P = wave + u * G::NW;
+                int t, col;
+                slot_tc<R, G::T, MAP>(P * 16 + c, t, col);
+                const int y = o.l0b + t;
+                const bool ok = (G::PAIRS % G::NW == 0 || P < G::PAIRS) && t < o.nv && y < a.real_h;
+                const unsigned row = (unsigned)y * (unsigned)a.real_w;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int x = col + (4 * g + i) * R16;
+                    const unsigned off = 4u * (row + (unsigned)x);
+                    const bool in = ok && x < a.real_w;
+                    w[4 * u + i] = make_float2(
+                        __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(pp.rsrc, (int)(in ? pp.first + off : kOutside), 0, 0)),
+                        __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                            pp.rsrc, (int)(in && pp.second != kOutside ? pp.second + off : kOutside), 0, 0)));
+                }
+            }
+            return;
+        }
         if constexpr (REV) {
             static_assert(PREC != PREC_FP32, "digit-reversed loads are for the matrix-core kernels");
             const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -450,7 +517,7 @@ __device__ __forceinline__ unsigned tw_line(const TileArgs &a, const Origin &o, 
 // each keeps its address space (LDS reads wait on the LDS counter only, never on the
 // next tile's prefetch loads).
 template <int PREC, int R, int KIND, int MAP, bool FIRST, bool LAST, int INF, int OUTF, bool TW = false,
-          bool REV = false>
+          bool REV = false, int ENDS = ENDS_PLAIN>
 __device__ __forceinline__ void mstage(float2 *lds, const TileArgs &a, const Origin &o, int s, const Ops<PREC> &op,
                                        const Prefetch<PREC, R, KIND, INF> &pf, const float2 *stw,
                                        const float2 *twl)
@@ -494,6 +561,9 @@ __device__ __forceinline__ void mstage(float2 *lds, const TileArgs &a, const Ori
     // lane's line is the same for every group, s is looked up once per tile.
     constexpr bool SAME_T = MAP == MAP_LINES && (16 * G::NW) % T == 0;
     float2 tw_step = make_float2(0.f, 0.f);
+    PlanePair pp;
+    if constexpr (LAST && ENDS == ENDS_CROP)
+        pp = plane_pair(a.crop_out, a.crop_span, (unsigned)((int)a.batch_base + o.l1), a.crop_b, a.crop_c, a.crop_h, a.crop_w);
     if constexpr (LAST && TW && SAME_T) {
         int t, col;
         slot_tc<R, T, MAP>(wave * 16 + c, t, col);
@@ -548,7 +618,10 @@ __device__ __forceinline__ void mstage(float2 *lds, const TileArgs &a, const Ori
                         y.x *= a.last_mul;
                         y.y *= a.last_mul;
                     }
-                    dst[(long long)pt * a.out_ps] = Elem<OUTF>::pack(y);
+                    if constexpr (ENDS == ENDS_CROP)
+                        crop_store(a, pp, R, crop_col(a, o.l0b + t), pt, y);
+                    else
+                        dst[(long long)pt * a.out_ps] = Elem<OUTF>::pack(y);
                 }
             }
         }
@@ -731,7 +804,7 @@ __device__ __forceinline__ void tstage(float2 *lds, const TileArgs &a, int s, fl
 // unscaled tables: this stage is VALU, no x16 operand factor), the tail's stage scale and
 // the output conversion. Lanes walk the points of a line (ROWS) or the lines (the
 // transposed and strided kinds), whichever is contiguous in the output.
-template <int R, int KIND, int RADIX, int NW, int OUTF, bool TW, bool REV = false>
+template <int R, int KIND, int RADIX, int NW, int OUTF, bool TW, bool REV = false, int ENDS = ENDS_PLAIN>
 __device__ __forceinline__ void tstage_last(float2 *lds, const TileArgs &a, const Origin &o, const float2 *twl)
 {
     typedef Geo<R, KIND, NW> G;
@@ -741,6 +814,9 @@ __device__ __forceinline__ void tstage_last(float2 *lds, const TileArgs &a, cons
     constexpr int NT = G::NT;
     constexpr int PER = (ITEMS + NT - 1) / NT;
     typedef typename Elem<OUTF>::raw raw;
+    PlanePair pp;
+    if constexpr (ENDS == ENDS_CROP)
+        pp = plane_pair(a.crop_out, a.crop_span, (unsigned)((int)a.batch_base + o.l1), a.crop_b, a.crop_c, a.crop_h, a.crop_w);
     wait_prefetch();
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
@@ -772,7 +848,10 @@ __device__ __forceinline__ void tstage_last(float2 *lds, const TileArgs &a, cons
                         y = cmulf(y, tw1<G::TWC>(a, twl, mult * (unsigned)pt));
                     }
                 }
-                dst[(long long)pt * a.out_ps] = Elem<OUTF>::pack(y);
+                if constexpr (ENDS == ENDS_CROP)
+                    crop_store(a, pp, R, crop_col(a, o.l0b + t), pt, y);
+                else
+                    dst[(long long)pt * a.out_ps] = Elem<OUTF>::pack(y);
             }
         }
     }
@@ -802,7 +881,7 @@ __device__ __forceinline__ void stage_tables(const TileArgs &a, float2 *s_stw, f
     if constexpr (PREC != PREC_FP32) op.load(reinterpret_cast<const DftOps *>(a.dft_ops), threadIdx.x & 63);
 }
 
-template <int PREC, int R, int KIND, int INF, int OUTF, bool TW, bool FULL, bool REV = false>
+template <int PREC, int R, int KIND, int INF, int OUTF, bool TW, bool FULL, bool REV = false, int ENDS = ENDS_PLAIN>
 __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float2 *stw, float2 *s_tw)
 {
     typedef Geo<R, KIND, fast_waves<PREC, KIND, R>()> G;
@@ -830,7 +909,7 @@ __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float
     TileWalk walk;
     walk.init(a, G::T, tile < end ? tile : 0, step);
     Origin o = walk.origin(a, G::T);
-    if (tile < end) cur.template load<FULL, REV>(a, o);
+    if (tile < end) cur.template load<FULL, REV, ENDS>(a, o);
     // the tables are loaded after the first tile's operands, so the two global-memory
     // round trips overlap (a workgroup with one tile waits for one, not two)
     Ops<PREC> op;
@@ -846,7 +925,7 @@ __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float
         if (next < end) {
             walk.advance(a);
             on = walk.origin(a, G::T);
-            nxt.template load<FULL, REV>(a, on);
+            nxt.template load<FULL, REV, ENDS>(a, on);
         }
         int s = 1;
         if constexpr (PREC == PREC_FP32)
@@ -856,7 +935,7 @@ __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float
         s = 16;
         if constexpr (NS == 1) {
             // R = 16 * TAIL: the tail is the last stage and stores to global memory
-            tstage_last<R, KIND, TAIL, G::NW, OUTF, TW, REV>(lds, a, o, s_tw);
+            tstage_last<R, KIND, TAIL, G::NW, OUTF, TW, REV, ENDS>(lds, a, o, s_tw);
         } else {
             if constexpr (TAIL > 1) {
                 tstage<R, KIND, TAIL, G::NW>(lds, a, s, a.tail_mul, stw);
@@ -873,7 +952,7 @@ __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float
             if constexpr (PREC == PREC_FP32)
                 vstage16<R, KIND, MAP_OUT, false, true, INF, OUTF, TW>(lds, a, o, s, cur, stw, s_tw);
             else
-                mstage<PREC, R, KIND, MAP_OUT, false, true, INF, OUTF, TW, REV>(lds, a, o, s, op, cur, stw, s_tw);
+                mstage<PREC, R, KIND, MAP_OUT, false, true, INF, OUTF, TW, REV, ENDS>(lds, a, o, s, op, cur, stw, s_tw);
         }
         tile_sync<PREC, R, KIND>();  // the next tile's first stage overwrites LDS
         tile = next;
@@ -924,6 +1003,36 @@ __global__ void __launch_bounds__((fast_waves<PREC, KIND, R>() * 64)) fft_fast(T
             fast_tiles<PREC, R, KIND, INF, OUTF, false, true>(a, lds, s_stw, s_tw);
         else
             fast_tiles<PREC, R, KIND, INF, OUTF, false, false>(a, lds, s_stw, s_tw);
+    }
+}
+
+// One pass of a whole axis with a fused end (ENDS_REAL, ENDS_CROP): split fp16, fp32 words.
+template <int R, int KIND, int ENDS>
+__global__ void __launch_bounds__((fast_waves<PREC_SPLIT, KIND, R>() * 64)) fft_fast_ends(TileArgs a)
+{
+    typedef Geo<R, KIND, fast_waves<PREC_SPLIT, KIND, R>()> G;
+    __shared__ float2 lds[G::SIZE];
+    __shared__ float2 s_stw[G::STW];
+    if (a.c0 % G::T == 0)
+        fast_tiles<PREC_SPLIT, R, KIND, FMT_C32, FMT_C32, false, true, false, ENDS>(a, lds, s_stw, nullptr);
+    else
+        fast_tiles<PREC_SPLIT, R, KIND, FMT_C32, FMT_C32, false, false, false, ENDS>(a, lds, s_stw, nullptr);
+}
+
+template <int KIND, int ENDS>
+fast_fn pick_ends(int R)
+{
+    switch (R) {
+    case 64: return fft_fast_ends<64, KIND, ENDS>;
+    case 128:
+        // not the strided kind: the compiler contracts the radix-8 tail's products differently there
+        // than in fft_fast, whose values a fused end is to give bit for bit
+        if constexpr (KIND == KIND_ROWS) return fft_fast_ends<128, KIND, ENDS>;
+        return nullptr;
+    case 256: return fft_fast_ends<256, KIND, ENDS>;
+    case 512: return fft_fast_ends<512, KIND, ENDS>;
+    case 1024: return fft_fast_ends<1024, KIND, ENDS>;
+    default: return nullptr;
     }
 }
 

@@ -16,6 +16,10 @@ static fast_fn pick_part(int R, int kind) { return fast::pick_kind<PREC_SPLIT, F
 static fast_fn pick_part(int R, int kind) { return fast::pick_kind<PREC_SPLIT, FMT_C16, FMT_C16>(R, kind); }
 #else
 static fast_fn pick_part(int R, int kind) { return fast::pick_kind<PREC_SPLIT, FMT_C32, FMT_C32>(R, kind); }
+fast_fn find_fast_ends(int R, int ends)
+{
+    return ends == ENDS_REAL ? fast::pick_ends<KIND_ROWS, ENDS_REAL>(R) : fast::pick_ends<KIND_COLS, ENDS_CROP>(R);
+}
 #endif
 
 #define MFFT_PART_FN_(k) find_fast_split_part##k

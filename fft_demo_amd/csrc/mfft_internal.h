@@ -20,6 +20,11 @@ struct ExecFuse {
     // 2D plans, any first pass: the column passes transform the first `cols` columns only (the
     // rest of the output is left undefined); 0 = all
     int cols = 0;
+    // the output as real planes (TileArgs::crop_out) instead of `out`; the plan must take it
+    // (plan_takes_crop)
+    float *crop_out = nullptr;
+    int crop_b = 0, crop_c = 0, crop_h = 0, crop_w = 0, crop_y = 0, crop_x = 0;
+    float crop_mul = 1.f;
     bool input() const { return in_mul || real_src; }  // needs a first pass that takes it
 };
 
@@ -30,8 +35,13 @@ struct ExecFuse {
 // fused real source instead of the input.
 int plan_create_2d_conv(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_desc *d, bool out_mid = false);
 
-// Whether the plan's first pass can take an ExecFuse.
+// Whether the plan's first pass can take a fused multiplier or real source.
 bool plan_first_pass_fusable(mfft_plan p);
+// Whether its first pass can read `planes` real planes of h x w (one buffer: no real_src2): the
+// streaming kernel, or with fp32 planes the matrix-core row kernel.
+bool plan_takes_real(mfft_plan p, int f64, long long planes, int h, int w);
+// Whether its last pass can store `planes` fp32 planes of h x w (ExecFuse::crop_out).
+bool plan_takes_crop(mfft_plan p, int f64, long long planes, int h, int w);
 // mfft_exec_ex with an ExecFuse (no caller workspace); MFFT_ERR_UNSUPPORTED when it fuses the
 // input and the first pass does not take that.
 int exec_fused(mfft_plan p, const void *in, void *out, int64_t batch, void *stream, const ExecFuse &f);

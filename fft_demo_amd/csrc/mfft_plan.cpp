@@ -971,7 +971,10 @@ static void trace_pass(const mfft_plan_s *p, const PassSpec &ps, const TileArgs 
     char name[64];
     snprintf(name, sizeof name, "%s R%d %s%s>%s", fam, ps.R, src, a.in_mul ? "*H" : "", fmt_name(a.out_fmt));
     (void)p;
-    trace_launch(s, name, rd, pts * fmt_bytes(a.out_fmt));
+    long long wr = pts * fmt_bytes(a.out_fmt);
+    if (a.crop_out)  // the planes of the chunk's transforms (2 per transform, or 1)
+        wr = (a.crop_b ? std::min(2 * nb, (long long)a.crop_b * a.crop_c) : nb) * a.crop_h * a.crop_w * 4;
+    trace_launch(s, name, rd, wr);
 }
 
 // only >= 0: run that pass alone; kstart/kstop: events the runtime records around that
@@ -997,7 +1000,24 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
             a.real_w = fz->real_w;
             a.real_pw = p->kind == 2 ? p->ny : p->n;
             a.real_p = p->total;
+            a.real_span = fz->real_f64 ? 0u : (unsigned)std::min<long long>(4LL * a.real_b * a.real_c * a.real_h * a.real_w, 0x7fffffff);
             a.batch_base = b0;
+        }
+        const void *fn = ps.fn;
+        if (a.real_src && ps.fast_kind == KIND_ROWS) fn = (const void *)find_fast_ends(ps.R, ENDS_REAL);
+        if (fz && fz->crop_out && &ps == &p->passes.back()) {
+            a.crop_out = fz->crop_out;
+            a.crop_b = fz->crop_b;
+            a.crop_c = fz->crop_c;
+            a.crop_h = fz->crop_h;
+            a.crop_w = fz->crop_w;
+            a.crop_y = fz->crop_y;
+            a.crop_x = fz->crop_x;
+            a.crop_mul = fz->crop_mul;
+            const long long planes = a.crop_b ? (long long)a.crop_b * a.crop_c : p->batch;
+            a.crop_span = (unsigned)(4 * planes * a.crop_h * a.crop_w);
+            a.batch_base = b0;
+            fn = (const void *)find_fast_ends(ps.R, ENDS_CROP);
         }
         a.in = buf_ptr(ps.src, in, out, work);
         a.out = buf_ptr(ps.dst, in, out, work);
@@ -1056,8 +1076,8 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
         if (ev) HIP_TRY(hipEventRecord(ev[evi++], s));
         auto launch = [&](dim3 grid, dim3 block) -> hipError_t {
             void *args[] = {&a};
-            if (kstart || kstop) return hipExtLaunchKernel(ps.fn, grid, block, args, 0, s, kstart, kstop, 0);
-            return hipLaunchKernel(ps.fn, grid, block, args, 0, s);
+            if (kstart || kstop) return hipExtLaunchKernel(fn, grid, block, args, 0, s, kstart, kstop, 0);
+            return hipLaunchKernel(fn, grid, block, args, 0, s);
         };
         if (ps.fast_kind == KIND_ONCHIP_COLS) {
             // one workgroup per 32 adjacent columns of one image
@@ -2040,9 +2060,36 @@ bool plan_first_pass_fusable(mfft_plan p)
     return p && !p->passes.empty() && p->passes.front().small && p->passes.front().src == BUF_IN;
 }
 
+// A pass of a whole axis on a matrix-core kernel that has a form with this end fused: transforms
+// along l1 alone, fp32 words on both sides.
+static bool fast_ends_pass(mfft_plan p, const PassSpec &ps, int kind, int ends)
+{
+    return !p->small && p->d.precision == PREC_SPLIT && ps.fast_kind == kind && !ps.tw_N && !ps.rev_fast && ps.l1 >= 0 &&
+           ps.lines[ps.l1].batch && ps.l2 < 0 && src_fmt(p, ps) == FMT_C32 && dst_fmt(p, ps) == FMT_C32 &&
+           find_fast_ends(ps.R, ends) != nullptr;
+}
+
+bool plan_takes_real(mfft_plan p, int f64, long long planes, int h, int w)
+{
+    if (plan_first_pass_fusable(p)) return true;
+    return p && p->kind == 2 && !p->passes.empty() && !f64 && planes * h * w < (1LL << 29) &&
+           p->passes.front().src == BUF_IN && p->passes.front().R == p->ny &&
+           fast_ends_pass(p, p->passes.front(), KIND_ROWS, ENDS_REAL);
+}
+
+bool plan_takes_crop(mfft_plan p, int f64, long long planes, int h, int w)
+{
+    return p && p->kind == 2 && !p->passes.empty() && !f64 && planes * h * w < (1LL << 29) && p->passes.back().col_axis &&
+           p->passes.back().R == p->nx && fast_ends_pass(p, p->passes.back(), KIND_COLS, ENDS_CROP);
+}
+
 int exec_fused(mfft_plan p, const void *in, void *out, int64_t batch, void *stream, const ExecFuse &f)
 {
-    if (f.input() && !plan_first_pass_fusable(p)) return fail(MFFT_ERR_UNSUPPORTED, "first pass takes no fused input");
+    const bool rows = !f.in_mul && !f.real_src2 && plan_takes_real(p, f.real_f64, (long long)f.real_b * f.real_c, f.real_h, f.real_w);
+    if (f.input() && !rows && !plan_first_pass_fusable(p))
+        return fail(MFFT_ERR_UNSUPPORTED, "first pass takes no fused input");
+    if (f.crop_out && !plan_takes_crop(p, 0, f.crop_b ? (long long)f.crop_b * f.crop_c : p->batch, f.crop_h, f.crop_w))
+        return fail(MFFT_ERR_UNSUPPORTED, "last pass takes no fused crop");
     if (batch < 1 || batch > p->batch) return fail(MFFT_ERR_INVALID, "batch %lld outside 1..%lld", (long long)batch, p->batch);
     return exec_all(p, in, out, stream, nullptr, batch, nullptr, &f);
 }
