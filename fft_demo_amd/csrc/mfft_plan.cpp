@@ -246,6 +246,11 @@ struct mfft_plan_s {
     // small_below transforms, which would leave most of the device idle on the on-chip pass.
     mfft_plan_s *small = nullptr;
     long long small_below = 0;
+    // A transform of the conv operator: no mixed-radix kernels. Their stages round in another order
+    // than the passes its filters and images have always gone through; with 16-bit words on the way
+    // the difference grows to whole fp16 steps (1e-4 of the fp32 result), and the filter gradient's
+    // inverse, whose values are near fp16's smallest, changes in its third digit.
+    bool conv = false;
     // Intermediates that a pass stores in the output buffer are kept in mid_fmt (the last
     // pass writes out_fmt there): with 16-bit intermediates and 32-bit output, every pass
     // boundary then moves 16-bit words. Execs must not alias a pass's source and destination
@@ -753,7 +758,7 @@ static int finish_passes(mfft_plan_s *p)
         }
         if (ps.fast_kind < 0) ps.rev_fast = false;
         const bool mixed_cols = !is_pow2(ps.R) && ps.ps_in != 1 && mixed_one_pass(p->d.precision, ps.R, ps.ps_in, ps.ps_out, ps.lines);
-        if (!ps.small && ps.fast_kind < 0 && !rev && !ps.tw_N && (mixed_cols || (ps.generic && dense_rows(ps)))) {
+        if (!p->conv && !ps.small && ps.fast_kind < 0 && !rev && !ps.tw_N && (mixed_cols || (ps.generic && dense_rows(ps)))) {
             const int T = mixed_cols ? mixed_col_lines(ps.R) : 0;
             ps.mixed_cap = !mixed_cols ? 0 : ps.R * T <= kMixColSmall ? kMixColSmall : kMixColLarge;
             const void *fn = find_mixed_kernel(p->d.precision, in_fmt, out_fmt, ps.mixed_cap);
@@ -1396,6 +1401,7 @@ static int create_2d(mfft_plan *plan, int nx, int ny, int64_t batch, const mfft_
     }
     for (size_t i = nrow_passes; i < p->passes.size(); ++i) p->passes[i].col_axis = true;
     p->out_mid = out_mid;
+    p->conv = conv;
     if (!rc) rc = finalize_plan(p);
     if (rc) {
         std::string msg = g_err;
