@@ -26,6 +26,7 @@ constexpr int kMaxStages = 8;
 constexpr int kWaves = 4;                 // waves per workgroup of the tile kernel
 constexpr int kThreads = kWaves * 64;
 constexpr int kMaxTile = 4096;            // complex points per workgroup tile
+constexpr int kSmallTile = 1024;          // the same for launches of few tiles of short lines
 constexpr int kMaxPairsPerWave = kMaxTile / 256 / kWaves;  // MFMA column groups per wave/stage
 constexpr int kMaxValuPerThread = 32;
 // Cache policy of the 2048-point on-chip line kernels' output stores: nt (non-temporal, bit
@@ -108,6 +109,13 @@ struct TileArgs {
     const void *real_src2;     // set: the imaginary part comes from this second image instead
     int real_f64, real_b, real_c, real_h, real_w, real_pw;
     long long real_p, batch_base;
+    // contiguous lines stored transposed (fast and tile kernels), groups of lines merged into one
+    // level (merge lines a group, 0 = not merged): line l0 is stored at group l0 / merge (merge_out
+    // elements apart), line l0 % merge of it; x / merge = (x * merge_mul) >> 16 for x < merge + T.
+    // out_s0 is 0 then.
+    int merge;
+    unsigned merge_mul;
+    long long merge_out;
     // last pass of a 2D plan, fused crop (fast strided kernel with crop_out set): point (y, x) of
     // transform m = crop_c k + c is stored as real planes: its real part, times crop_mul, at row
     // (y - crop_y) mod R and column (x - crop_x) mod c0 of plane [2k][c] of [crop_b][crop_c][crop_h]

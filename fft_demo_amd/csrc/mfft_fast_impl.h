@@ -101,6 +101,31 @@ struct Origin {
     long long in_base, out_base;
 };
 
+// Where the lines of a tile are stored. The transposed-store kind (lines adjacent in the output,
+// out_s0 = 1) may have the lines of many groups merged into one level (TileArgs::merge): the second
+// pass of a length such as 17 x 128 has groups of 17 lines, which would fill 17 of a tile's 32.
+template <int KIND, bool TW>
+struct OutLines {
+    int q0 = 0, r0 = 0;
+    __device__ __forceinline__ OutLines(const TileArgs &a, const Origin &o)
+    {
+        if constexpr (KIND == KIND_ROWS_TR && !TW)
+            if (a.merge) {
+                q0 = (int)((unsigned)o.l0b / (unsigned)a.merge);
+                r0 = o.l0b - q0 * a.merge;
+            }
+    }
+    __device__ __forceinline__ long long at(const TileArgs &a, const Origin &o, int t) const
+    {
+        if constexpr (KIND == KIND_ROWS_TR && !TW) {
+            const unsigned x = (unsigned)(r0 + t), q = (x * a.merge_mul) >> 16;
+            return o.out_base + (q0 + (int)q) * a.merge_out + (int)(x - q * (unsigned)a.merge);
+        } else {
+            return o.out_base + (long long)t * a.out_s0;
+        }
+    }
+};
+
 // Row tiles of 256-point lines: on the matrix cores MFMA group P of a stage is line P in
 // both radix-16 stages (16 slots of a line per group) and P = wave + u NW; in the fp32 path
 // thread i holds a column of line i / 16 in both stages. Either way every line's LDS
@@ -555,6 +580,7 @@ __device__ __forceinline__ void mstage(float2 *lds, const TileArgs &a, const Ori
     }
     if constexpr (!FIRST && !LAST) __syncthreads();  // all reads of the tile precede the writes
     if constexpr (LAST) wait_prefetch();
+    const OutLines<LAST ? KIND : -1, TW> lines(a, o);
     // Last stage with the four-step twiddle: the lane's outputs of group u are the points
     // col + R16 (4g + i), i = 0..3, so their twiddles are w_i = W^(mult (col + 4g R16)) *
     // s^i with s = W^(mult R16): one table lookup for w_0, products for the rest. When the
@@ -592,7 +618,7 @@ __device__ __forceinline__ void mstage(float2 *lds, const TileArgs &a, const Ori
         } else {
             if (t < o.nv) {
                 typedef typename Elem<OUTF>::raw raw;
-                raw *dst = reinterpret_cast<raw *>(a.out) + o.out_base + (long long)t * a.out_s0;
+                raw *dst = reinterpret_cast<raw *>(a.out) + lines.at(a, o, t);
                 float2 w[4];
                 if constexpr (TW) {
                     const unsigned mult = tw_line<REV>(a, o, t);
@@ -702,7 +728,8 @@ __device__ __forceinline__ void vstage16(float2 *lds, const TileArgs &a, const O
         wait_prefetch();
         if (t >= o.nv) return;
         typedef typename Elem<OUTF>::raw raw;
-        raw *dst = reinterpret_cast<raw *>(a.out) + o.out_base + (long long)t * a.out_s0;
+        const OutLines<KIND, TW> lines(a, o);
+        raw *dst = reinterpret_cast<raw *>(a.out) + lines.at(a, o, t);
         const unsigned mult = (unsigned)(a.tw_level ? o.l1 : o.l0b + t);
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) {
@@ -817,6 +844,7 @@ __device__ __forceinline__ void tstage_last(float2 *lds, const TileArgs &a, cons
     PlanePair pp;
     if constexpr (ENDS == ENDS_CROP)
         pp = plane_pair(a.crop_out, a.crop_span, (unsigned)((int)a.batch_base + o.l1), a.crop_b, a.crop_c, a.crop_h, a.crop_w);
+    const OutLines<KIND, TW> lines(a, o);
     wait_prefetch();
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
@@ -829,7 +857,7 @@ __device__ __forceinline__ void tstage_last(float2 *lds, const TileArgs &a, cons
         for (int j = 0; j < RADIX; ++j) v[j] = lds[G::phys(t, col + j * COLS)];
         if (t >= o.nv) continue;
         dft_tail<RADIX>(v, a.sign, a.w16);
-        raw *dst = reinterpret_cast<raw *>(a.out) + o.out_base + (long long)t * a.out_s0;
+        raw *dst = reinterpret_cast<raw *>(a.out) + lines.at(a, o, t);
         const unsigned mult = tw_line<REV>(a, o, t);
 #pragma unroll
         for (int q4 = 0; q4 < RADIX; q4 += 4) {

@@ -494,6 +494,20 @@ __device__ void copy_out(const float2 *lds, const Geo &G, const TileArgs &a, con
     const int R = G.R;
     const int nv = o.nvalid;
     constexpr int UNR = 4;
+    if (a.merge) {
+        // merged line groups (TileArgs::merge): a group's merge * R values are adjacent in the
+        // output, so the threads walk the groups the tile has lines of
+        const int m = a.merge, q0 = o.l0b / m, r0 = o.l0b - q0 * m;
+        const int n = ((r0 + nv - 1) / m + 1) * m * R;  // below 2^17 (checked on the host)
+        const float inv = 1.0f / (float)m;
+        for (int e = threadIdx.x; e < n; e += kThreads) {
+            const int w = (int)(((float)e + 0.5f) * inv), r = e - w * m, q = w / R, p = w - q * R, t = q * m + r - r0;
+            if ((unsigned)t < (unsigned)nv)
+                cstore1(a.out, o.out_base + (q0 + q) * a.merge_out + (long long)p * a.out_ps + r, a.out_fmt,
+                        out_value(lds, G, a, o.l0b, o.l1, t, p));
+        }
+        return;
+    }
     if (a.out_vec && a.out_ps == 1 && (R & 3) == 0 && (a.out_s0 & 3) == 0 && (o.out_base & 3) == 0) {
         const int per_line = R >> 2;
         const int nch = nv * per_line;
@@ -765,6 +779,24 @@ tile_fn find_tile_kernel(int prec, int R, int TL, bool generic)
     case PREC_BF16: return fft_tile_generic<PREC_BF16>;
     case PREC_SPLIT: return fft_tile_generic<PREC_SPLIT>;
     case PREC_FP32: return fft_tile_generic<PREC_FP32>;
+    default: return nullptr;
+    }
+}
+
+// The same with tiles of kSmallTile points (16- and 32-point contiguous lines).
+template <int PREC>
+static tile_fn pick_small_tile(int R)
+{
+    return R == 16 ? (tile_fn)fft_tile_pow2<PREC, 16, 1, kSmallTile / 16> : R == 32 ? (tile_fn)fft_tile_pow2<PREC, 32, 1, kSmallTile / 32> : nullptr;
+}
+
+tile_fn find_small_tile_kernel(int prec, int R)
+{
+    switch (prec) {
+    case PREC_FP16: return pick_small_tile<PREC_FP16>(R);
+    case PREC_BF16: return pick_small_tile<PREC_BF16>(R);
+    case PREC_SPLIT: return pick_small_tile<PREC_SPLIT>(R);
+    case PREC_FP32: return pick_small_tile<PREC_FP32>(R);
     default: return nullptr;
     }
 }
