@@ -96,6 +96,25 @@ __device__ __forceinline__ void slot_tc(int slot, int &t, int &col)
     }
 }
 
+// Strided lines of 512 and 1024 points on the matrix cores: the radix-2 or radix-4 stage between the
+// two radix-16 stages is done in registers (mstage_tail). Column col of the first stage meets
+// columns col + R / 2^k of it there, so those are the ones a wave holds: its two groups are half a
+// line apart and, at 1024 points, so are by a quarter the lanes c and c ^ 8.
+template <int PREC, int R, int KIND>
+constexpr bool tail_in_regs() { return PREC != PREC_FP32 && KIND == KIND_COLS && (R == 512 || R == 1024); }
+
+// (line, column) of a lane in group u of the first stage.
+template <int PREC, int R, int KIND, int T, int NW, int MAP>
+__device__ __forceinline__ void first_tc(int wave, int u, int c, int &t, int &col)
+{
+    if constexpr (tail_in_regs<PREC, R, KIND>() && R == 1024) {
+        t = c & 7;
+        col = wave + 16 * (c >> 3) + 32 * u;
+    } else {
+        slot_tc<R, T, MAP>((wave + u * NW) * 16 + c, t, col);
+    }
+}
+
 struct Origin {
     int l0b, l1, nv;
     long long in_base, out_base;
@@ -118,8 +137,11 @@ struct OutLines {
     __device__ __forceinline__ long long at(const TileArgs &a, const Origin &o, int t) const
     {
         if constexpr (KIND == KIND_ROWS_TR && !TW) {
-            const unsigned x = (unsigned)(r0 + t), q = (x * a.merge_mul) >> 16;
-            return o.out_base + (q0 + (int)q) * a.merge_out + (int)(x - q * (unsigned)a.merge);
+            if (a.merge) {
+                const unsigned x = (unsigned)(r0 + t), q = (x * a.merge_mul) >> 16;
+                return o.out_base + (q0 + (int)q) * a.merge_out + (int)(x - q * (unsigned)a.merge);
+            }
+            return o.out_base + t;
         } else {
             return o.out_base + (long long)t * a.out_s0;
         }
@@ -395,7 +417,7 @@ struct Prefetch {
             for (int u = 0; u < G::MAXP; ++u) {
                 const int P = wave + u * G::NW;
                 int t, col;
-                slot_tc<R, G::T, MAP>(P * 16 + c, t, col);
+                first_tc<PREC, R, KIND, G::T, G::NW, MAP>(wave, u, c, t, col);
                 const bool ok = (G::PAIRS % G::NW == 0 || P < G::PAIRS) && (FULL || t < o.nv);
                 const long long pos = 16LL * digit_rev(col, a.in_rev) + 4 * g;
                 if constexpr (KIND == KIND_COLS) {
@@ -461,7 +483,7 @@ struct Prefetch {
             for (int u = 0; u < G::MAXP; ++u) {
                 const int P = wave + u * G::NW;
                 int t, col;
-                slot_tc<R, G::T, MAP>(P * 16 + c, t, col);
+                first_tc<PREC, R, KIND, G::T, G::NW, MAP>(wave, u, c, t, col);
                 const bool ok = (G::PAIRS % G::NW == 0 || P < G::PAIRS) && (FULL || t < o.nv);
                 const raw *base = src + o.in_base + (long long)t * a.in_s0 + (long long)(col + 4 * g * R16) * a.in_ps;
                 const long long step = (long long)R16 * a.in_ps;
@@ -653,6 +675,76 @@ __device__ __forceinline__ void mstage(float2 *lds, const TileArgs &a, const Ori
         }
     }
     if constexpr (!LAST) tile_sync<PREC, R, KIND>();
+}
+
+// The first radix-16 stage and the radix-2 or radix-4 stage after it (tail_in_regs), from the
+// prefetched inputs to LDS: one exchange through LDS a tile instead of two, and two barriers fewer.
+// 1024^2 x 64 2D 291 -> 278 us an exec, 2^20 x 16 (512-point first pass) 76.3 -> 72.6 (16-bit words).
+__device__ __forceinline__ float swap8(float v)  // the value of lane c ^ 8 of the 16
+{
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+}
+
+template <int PREC, int R, int KIND, int INF>
+__device__ __forceinline__ void mstage_tail(float2 *lds, const TileArgs &a, const Ops<PREC> &op,
+                                            const Prefetch<PREC, R, KIND, INF> &pf, const float2 *stw)
+{
+    typedef Geo<R, KIND, fast_waves<PREC, KIND, R>()> G;
+    static_assert(G::MAXP == 2 && G::NW == 16 && G::PAIRS == 32, "two groups a wave");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    constexpr bool EXACT = (INF == FMT_C16 && PREC != PREC_BF16) || (INF == FMT_CBF16 && PREC == PREC_BF16);
+    float2 z[2][4];
+    int t, col;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        first_tc<PREC, R, KIND, G::T, G::NW, MAP_LINES>(wave, u, c, t, col);
+        float2 x[4];
+        h8 r16;
+        b8 rb;
+        if constexpr (EXACT) {
+            const u4 v = {pf.w[4 * u], pf.w[4 * u + 1], pf.w[4 * u + 2], pf.w[4 * u + 3]};
+            r16 = __builtin_bit_cast(h8, v);
+            rb = __builtin_bit_cast(b8, v);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = Elem<INF>::f(pf.w[4 * u + i]);
+        }
+        f4 ar, ai;
+        dft16<PREC, EXACT>(x, r16, rb, op, ar, ai);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[u][i] = cmulf(make_float2(ar[i], ai[i]), stw[col * (4 * g + i)]);
+    }
+    // output tq of the tail's column (4 g + i, wave) goes to point 4 g + i + 16 (RADIX wave + tq),
+    // times W_R^(16 wave tq); the table carries a matrix-core stage's scale, undone by comp
+    constexpr int RADIX = R / 256;
+    const int half = RADIX == 4 ? c >> 3 : 0, tq = 2 * half;
+    const float mul = a.tail_mul, comp = mul / a.last_mul, sg = half ? -1.f : 1.f;
+    const float2 w0 = stw[16 * wave * tq], w1 = stw[16 * wave * (tq + 1)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float2 y0 = make_float2(z[0][i].x + z[1][i].x, z[0][i].y + z[1][i].y);
+        float2 y1 = make_float2(z[0][i].x - z[1][i].x, z[0][i].y - z[1][i].y);
+        if constexpr (RADIX == 4) {
+            // lanes c < 8 have the sum and difference of columns 0 and 2 and keep outputs 0 and 1,
+            // lanes c >= 8 those of columns 1 and 3 and keep outputs 2 and 3
+            const float2 r = make_float2(-a.sign * y1.y, a.sign * y1.x);
+            y1 = half ? r : y1;
+            y0 = make_float2(swap8(y0.x) + sg * y0.x, swap8(y0.y) + sg * y0.y);
+            y1 = make_float2(swap8(y1.x) + sg * y1.x, swap8(y1.y) + sg * y1.y);
+        }
+        if (wave) {
+            y0 = cmulf(make_float2(y0.x * comp, y0.y * comp), w0);
+            y1 = cmulf(make_float2(y1.x * comp, y1.y * comp), w1);
+        } else {
+            y0 = make_float2(y0.x * mul, y0.y * mul);
+            y1 = make_float2(y1.x * mul, y1.y * mul);
+        }
+        float2 *d = lds + G::phys(t, 4 * g + i + 16 * (RADIX * wave + tq));
+        d[0] = y0;
+        d[16 * G::T] = y1;
+    }
+    __syncthreads();
 }
 
 // ------------------------------------------------------------------ radix-16 stage (fp32 VALU)
@@ -958,6 +1050,8 @@ __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float
         int s = 1;
         if constexpr (PREC == PREC_FP32)
             vstage16<R, KIND, MAP_IN, true, false, INF, OUTF>(lds, a, o, s, cur, stw, s_tw);
+        else if constexpr (tail_in_regs<PREC, R, KIND>())
+            mstage_tail<PREC, R, KIND, INF>(lds, a, op, cur, stw);
         else
             mstage<PREC, R, KIND, MAP_IN, true, false, INF, OUTF>(lds, a, o, s, op, cur, stw, s_tw);
         s = 16;
@@ -965,7 +1059,9 @@ __device__ __forceinline__ void fast_tiles(const TileArgs &a, float2 *lds, float
             // R = 16 * TAIL: the tail is the last stage and stores to global memory
             tstage_last<R, KIND, TAIL, G::NW, OUTF, TW, REV, ENDS>(lds, a, o, s_tw);
         } else {
-            if constexpr (TAIL > 1) {
+            if constexpr (tail_in_regs<PREC, R, KIND>()) {
+                s *= TAIL;
+            } else if constexpr (TAIL > 1) {
                 tstage<R, KIND, TAIL, G::NW>(lds, a, s, a.tail_mul, stw);
                 s *= TAIL;
             }
