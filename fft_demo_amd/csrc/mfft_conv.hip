@@ -199,8 +199,11 @@ __global__ void __launch_bounds__(256) pointwise_mac_kernel(const void *X, const
 #pragma unroll
             for (int f = 0; f < kMapTile; ++f)
                 if (k < nk && f < nf) {
-                    acc[k][f].x += a[k].x * b[f].x - a[k].y * b[f].y;
-                    acc[k][f].y += a[k].x * b[f].y + a[k].y * b[f].x;
+                    // which product is fused is fixed here, as the kernel of one output a thread had
+                    // it per format: 16-bit words further on show a change of it
+                    acc[k][f].x += __builtin_fmaf(a[k].x, b[f].x, -(a[k].y * b[f].y));
+                    acc[k][f].y += XFMT == FMT_C16 ? __builtin_fmaf(a[k].x, b[f].y, a[k].y * b[f].x)
+                                                   : __builtin_fmaf(a[k].y, b[f].x, a[k].x * b[f].y);
                 }
     }
 #pragma unroll
