@@ -336,12 +336,16 @@ int mfft_conv2d_set_filters(mfft_conv2d op, const void *filters, int real_fmt, v
 }
 
 // Spectra of a batch of real planes [batch][maps][h][w], in pairs, zero-padded: from the planes
-// themselves where the transform's first pass reads them, else through a packing pass.
+// themselves where the transform's first pass reads them, else through a packing pass. streaming:
+// also where that is the streaming kernel, whose fused form rounds the stage scale apart from the
+// twiddles: not for the filter gradient, whose products are near fp16's smallest values (a change
+// in the spectra's last bits moved it by 1e-4 at 192 x 192).
 static int image_spectra(mfft_conv2d op, mfft_plan plan, const void *src, int f64, int maps, int h, int w, void *dst,
-                         hipStream_t s)
+                         bool streaming, hipStream_t s)
 {
     int rc;
-    if (mfft::plan_takes_real(plan, f64, (long long)op->d.batch * maps, h, w)) {
+    if ((streaming || !mfft::plan_first_pass_fusable(plan)) &&
+        mfft::plan_takes_real(plan, f64, (long long)op->d.batch * maps, h, w)) {
         mfft::ExecFuse f;
         f.real_src = src;
         f.real_f64 = f64;
@@ -389,7 +393,7 @@ static int conv_run(mfft_conv2d op, const void *in, int in_fmt, void *out, int o
     OpCall call(op, s);
     if (call.err != hipSuccess) return cfail(MFFT_ERR_HIP, "stream order: %s", hipGetErrorString(call.err));
     const mfft_conv2d_desc &d = op->d;
-    int rc = image_spectra(op, op->fwd_img, in, in_fmt == MFFT_REAL_F64, d.channels, d.h, d.w, op->X, s);
+    int rc = image_spectra(op, op->fwd_img, in, in_fmt == MFFT_REAL_F64, d.channels, d.h, d.w, op->X, true, s);
     if (rc) return rc;
     const long long P = (long long)op->Ph * op->Pw;
     const int nf = fsel >= 0 ? 1 : d.filters;
@@ -552,10 +556,10 @@ int mfft_conv2d_backward(mfft_conv2d op, const void *in, const void *delta, int 
     const int f64 = real_fmt == MFFT_REAL_F64;
     const long long P = (long long)op->Ph * op->Pw;
     // delta spectra (scaled 1/P) in Y
-    rc = image_spectra(op, op->fwd_delta, delta, f64, d.filters, op->oh, op->ow, op->Y, s);
+    rc = image_spectra(op, op->fwd_delta, delta, f64, d.filters, op->oh, op->ow, op->Y, false, s);
     if (rc) return rc;
     if (grad_w) {
-        rc = image_spectra(op, op->fwd_img, in, f64, d.channels, d.h, d.w, op->X, s);
+        rc = image_spectra(op, op->fwd_img, in, f64, d.channels, d.h, d.w, op->X, false, s);
         if (rc) return rc;
         mfft::trace_launch(s, "conv_pointwise_gw", op->pairs * (d.channels + d.filters) * P * 8,
                            (long long)d.filters * d.channels * P * 8);
