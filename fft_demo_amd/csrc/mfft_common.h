@@ -118,11 +118,12 @@ struct TileArgs {
     long long merge_out;
     // last pass of a 2D plan, fused crop (fast strided kernel with crop_out set): point (y, x) of
     // transform m = crop_c k + c is stored as real planes: its real part, times crop_mul, at row
-    // (y - crop_y) mod R and column (x - crop_x) mod c0 of plane [2k][c] of [crop_b][crop_c][crop_h]
-    // [crop_w], its imaginary part in plane [2k + 1][c] (absent past the batch), what lies outside
-    // the plane nowhere. crop_b = 0: plane m from the real part alone.
+    // (y - crop_y) mod crop_rows and column (x - crop_x) mod c0 of plane [2k][c] of [crop_b][crop_c]
+    // [crop_h][crop_w], its imaginary part in plane [2k + 1][c] (absent past the batch), what lies
+    // outside the plane nowhere. crop_b = 0: plane m from the real part alone. Transforms are l1, and
+    // y = crop_s2 l2 + crop_sp point.
     float *crop_out;
-    int crop_b, crop_c, crop_h, crop_w, crop_y, crop_x;
+    int crop_b, crop_c, crop_h, crop_w, crop_y, crop_x, crop_rows, crop_s2, crop_sp;
     unsigned crop_span;        // bytes of crop_out, below 2^31
     unsigned real_span;        // fast kernels: bytes of real_src (fp32), below 2^31
     float crop_mul;

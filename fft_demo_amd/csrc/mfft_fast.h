@@ -54,11 +54,12 @@ constexpr int fast_waves_of(int prec, int R, int kind)
 constexpr bool fast_rev_ok(int prec, int in_fmt) { return prec != PREC_FP32 && in_fmt != FMT_CBF16; }
 
 typedef void (*fast_fn)(TileArgs);
-// Kernels of the convolution layers with an end of the transform fused (split fp16, fp32 words):
-// ENDS_REAL, row kind: the first stage reads pairs of real planes (TileArgs::real_src); ENDS_CROP,
-// strided kind: the last stage stores real planes (TileArgs::crop_out).
+// Kernels of the conv operator with an end of the transform fused (split fp16): ENDS_REAL, row kind,
+// fp32 words: the first stage reads pairs of real planes (TileArgs::real_src); ENDS_CROP, strided
+// kind, the same words on both sides: the last stage stores real planes (TileArgs::crop_out), of
+// values rounded to the words first.
 enum { ENDS_PLAIN = 0, ENDS_REAL = 1, ENDS_CROP = 2 };
-fast_fn find_fast_ends(int R, int ends);
+fast_fn find_fast_ends(int R, int ends, int fmt);
 fast_fn find_fast_kernel(int prec, int R, int kind, int in_fmt, int out_fmt);
 int fast_tile_lines(int R, int kind);
 int fast_threads(int prec, int R, int kind);

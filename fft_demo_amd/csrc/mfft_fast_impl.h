@@ -116,7 +116,7 @@ __device__ __forceinline__ void first_tc(int wave, int u, int c, int &t, int &co
 }
 
 struct Origin {
-    int l0b, l1, nv;
+    int l0b, l1, l2, nv;
     long long in_base, out_base;
 };
 
@@ -209,6 +209,7 @@ struct TileWalk {
         Origin o;
         o.l0b = t0 * T;
         o.l1 = l1;
+        o.l2 = (int)l2;
         o.nv = min(T, a.c0 - o.l0b);
         o.in_base = in_base;
         o.out_base = out_base;
@@ -335,21 +336,19 @@ __device__ __forceinline__ PlanePair plane_pair(const void *base, unsigned span,
     return p;
 }
 
-__device__ __forceinline__ void crop_store(const TileArgs &a, const PlanePair &pp, int R, int xx, int pt, float2 v)
+template <int FMT>
+__device__ __forceinline__ void crop_store(const TileArgs &a, const PlanePair &pp, const Origin &o, int t, int pt, float2 v)
 {
-    int yy = pt - a.crop_y;
-    yy += yy < 0 ? R : 0;
+    int yy = a.crop_s2 * o.l2 + a.crop_sp * pt - a.crop_y, xx = o.l0b + t - a.crop_x;
+    yy += yy < 0 ? a.crop_rows : 0;
+    xx += xx < 0 ? a.c0 : 0;
     const bool ok = yy < a.crop_h && xx < a.crop_w;
-    const unsigned o = 4u * ((unsigned)yy * (unsigned)a.crop_w + (unsigned)xx);
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v.x * a.crop_mul), pp.rsrc, (int)(ok ? pp.first + o : kOutside), 0, 0);
-    if (pp.second != kOutside)
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v.y * a.crop_mul), pp.rsrc, (int)(ok ? pp.second + o : kOutside), 0, 0);
-}
-
-__device__ __forceinline__ int crop_col(const TileArgs &a, int x)
-{
-    x -= a.crop_x;
-    return x + (x < 0 ? a.c0 : 0);
+    const unsigned off = 4u * ((unsigned)yy * (unsigned)a.crop_w + (unsigned)xx);
+    v = Elem<FMT>::f(Elem<FMT>::pack(v));
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v.x * a.crop_mul), pp.rsrc, (int)(ok ? pp.first + off : kOutside), 0, 0);
+    // no branch on it: the tail's arithmetic stays one block, contracted as in fft_fast
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v.y * a.crop_mul), pp.rsrc,
+                                          (int)(ok && pp.second != kOutside ? pp.second + off : kOutside), 0, 0);
 }
 
 // Wait for every outstanding vector-memory operation of this wave. Called in the last stage
@@ -667,7 +666,7 @@ __device__ __forceinline__ void mstage(float2 *lds, const TileArgs &a, const Ori
                         y.y *= a.last_mul;
                     }
                     if constexpr (ENDS == ENDS_CROP)
-                        crop_store(a, pp, R, crop_col(a, o.l0b + t), pt, y);
+                        crop_store<OUTF>(a, pp, o, t, pt, y);
                     else
                         dst[(long long)pt * a.out_ps] = Elem<OUTF>::pack(y);
                 }
@@ -683,6 +682,13 @@ __device__ __forceinline__ void mstage(float2 *lds, const TileArgs &a, const Ori
 __device__ __forceinline__ float swap8(float v)  // the value of lane c ^ 8 of the 16
 {
     return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+}
+
+// cmulf with its contraction written out, as the compiler has it where the stages meet in LDS: the
+// same values bit for bit, whichever way a line goes.
+__device__ __forceinline__ float2 cmul_fixed(float2 a, float2 b)
+{
+    return make_float2(__builtin_fmaf(a.x, b.x, -(a.y * b.y)), __builtin_fmaf(a.y, b.x, a.x * b.y));
 }
 
 template <int PREC, int R, int KIND, int INF>
@@ -713,7 +719,12 @@ __device__ __forceinline__ void mstage_tail(float2 *lds, const TileArgs &a, cons
         f4 ar, ai;
         dft16<PREC, EXACT>(x, r16, rb, op, ar, ai);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) z[u][i] = cmulf(make_float2(ar[i], ai[i]), stw[col * (4 * g + i)]);
+        for (int i = 0; i < 4; ++i) {
+            z[u][i] = cmul_fixed(make_float2(ar[i], ai[i]), stw[col * (4 * g + i)]);
+            // rounded here, as where LDS lies between the stages: no product is contracted into the
+            // sums below
+            __asm__("" : "+v"(z[u][i].x), "+v"(z[u][i].y));
+        }
     }
     // output tq of the tail's column (4 g + i, wave) goes to point 4 g + i + 16 (RADIX wave + tq),
     // times W_R^(16 wave tq); the table carries a matrix-core stage's scale, undone by comp
@@ -734,8 +745,8 @@ __device__ __forceinline__ void mstage_tail(float2 *lds, const TileArgs &a, cons
             y1 = make_float2(swap8(y1.x) + sg * y1.x, swap8(y1.y) + sg * y1.y);
         }
         if (wave) {
-            y0 = cmulf(make_float2(y0.x * comp, y0.y * comp), w0);
-            y1 = cmulf(make_float2(y1.x * comp, y1.y * comp), w1);
+            y0 = cmul_fixed(make_float2(y0.x * comp, y0.y * comp), w0);
+            y1 = cmul_fixed(make_float2(y1.x * comp, y1.y * comp), w1);
         } else {
             y0 = make_float2(y0.x * mul, y0.y * mul);
             y1 = make_float2(y1.x * mul, y1.y * mul);
@@ -969,7 +980,7 @@ __device__ __forceinline__ void tstage_last(float2 *lds, const TileArgs &a, cons
                     }
                 }
                 if constexpr (ENDS == ENDS_CROP)
-                    crop_store(a, pp, R, crop_col(a, o.l0b + t), pt, y);
+                    crop_store<OUTF>(a, pp, o, t, pt, y);
                 else
                     dst[(long long)pt * a.out_ps] = Elem<OUTF>::pack(y);
             }
@@ -1130,32 +1141,28 @@ __global__ void __launch_bounds__((fast_waves<PREC, KIND, R>() * 64)) fft_fast(T
     }
 }
 
-// One pass of a whole axis with a fused end (ENDS_REAL, ENDS_CROP): split fp16, fp32 words.
-template <int R, int KIND, int ENDS>
+// A pass with a fused end (ENDS_REAL, ENDS_CROP): split fp16, words of one format.
+template <int R, int KIND, int FMT, int ENDS>
 __global__ void __launch_bounds__((fast_waves<PREC_SPLIT, KIND, R>() * 64)) fft_fast_ends(TileArgs a)
 {
     typedef Geo<R, KIND, fast_waves<PREC_SPLIT, KIND, R>()> G;
     __shared__ float2 lds[G::SIZE];
     __shared__ float2 s_stw[G::STW];
     if (a.c0 % G::T == 0)
-        fast_tiles<PREC_SPLIT, R, KIND, FMT_C32, FMT_C32, false, true, false, ENDS>(a, lds, s_stw, nullptr);
+        fast_tiles<PREC_SPLIT, R, KIND, FMT, FMT, false, true, false, ENDS>(a, lds, s_stw, nullptr);
     else
-        fast_tiles<PREC_SPLIT, R, KIND, FMT_C32, FMT_C32, false, false, false, ENDS>(a, lds, s_stw, nullptr);
+        fast_tiles<PREC_SPLIT, R, KIND, FMT, FMT, false, false, false, ENDS>(a, lds, s_stw, nullptr);
 }
 
-template <int KIND, int ENDS>
+template <int KIND, int FMT, int ENDS>
 fast_fn pick_ends(int R)
 {
     switch (R) {
-    case 64: return fft_fast_ends<64, KIND, ENDS>;
-    case 128:
-        // not the strided kind: the compiler contracts the radix-8 tail's products differently there
-        // than in fft_fast, whose values a fused end is to give bit for bit
-        if constexpr (KIND == KIND_ROWS) return fft_fast_ends<128, KIND, ENDS>;
-        return nullptr;
-    case 256: return fft_fast_ends<256, KIND, ENDS>;
-    case 512: return fft_fast_ends<512, KIND, ENDS>;
-    case 1024: return fft_fast_ends<1024, KIND, ENDS>;
+    case 64: return fft_fast_ends<64, KIND, FMT, ENDS>;
+    case 128: return fft_fast_ends<128, KIND, FMT, ENDS>;
+    case 256: return fft_fast_ends<256, KIND, FMT, ENDS>;
+    case 512: return fft_fast_ends<512, KIND, FMT, ENDS>;
+    case 1024: return fft_fast_ends<1024, KIND, FMT, ENDS>;
     default: return nullptr;
     }
 }

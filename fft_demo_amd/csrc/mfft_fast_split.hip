@@ -14,11 +14,14 @@ static fast_fn pick_part(int R, int kind) { return fast::pick_kind<PREC_SPLIT, F
 static fast_fn pick_part(int R, int kind) { return fast::pick_kind<PREC_SPLIT, FMT_C32, FMT_C16>(R, kind); }
 #elif MFFT_PART == 2
 static fast_fn pick_part(int R, int kind) { return fast::pick_kind<PREC_SPLIT, FMT_C16, FMT_C16>(R, kind); }
+fast_fn find_fast_crop16(int R) { return fast::pick_ends<KIND_COLS, FMT_C16, ENDS_CROP>(R); }
 #else
 static fast_fn pick_part(int R, int kind) { return fast::pick_kind<PREC_SPLIT, FMT_C32, FMT_C32>(R, kind); }
-fast_fn find_fast_ends(int R, int ends)
+fast_fn find_fast_crop16(int R);
+fast_fn find_fast_ends(int R, int ends, int fmt)
 {
-    return ends == ENDS_REAL ? fast::pick_ends<KIND_ROWS, ENDS_REAL>(R) : fast::pick_ends<KIND_COLS, ENDS_CROP>(R);
+    if (ends == ENDS_REAL) return fmt == FMT_C32 ? fast::pick_ends<KIND_ROWS, FMT_C32, ENDS_REAL>(R) : nullptr;
+    return fmt == FMT_C32 ? fast::pick_ends<KIND_COLS, FMT_C32, ENDS_CROP>(R) : fmt == FMT_C16 ? find_fast_crop16(R) : nullptr;
 }
 #endif
 

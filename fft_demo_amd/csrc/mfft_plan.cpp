@@ -987,7 +987,9 @@ static void trace_pass(const mfft_plan_s *p, const PassSpec &ps, const TileArgs 
 // and on the input the lines of all groups follow each other. Where a group does not fill whole
 // tiles, tiles take lines across groups (TileArgs::merge): 17 x 128 points otherwise fill 17 of a
 // fast tile's 32 lines, 15 x 32 15 of a tile kernel's 128 (2176 points x 8704 lines, 16-bit words:
-// 39.2 -> 32.1 us; 480 x 15360, fp32: 113 -> 37.6).
+// 39.2 -> 32.1 us; 480 x 15360, fp32: 113 -> 37.6). Not where the groups' own tiles all run at once:
+// fewer, fuller tiles then leave compute units idle (conv 183 x 657 x 2, 240 groups of 3 lines: 36
+// us, merged into 45 tiles 42).
 static void merge_line_groups(const PassSpec &ps, TileArgs &a)
 {
     const bool fast = ps.fast_kind == KIND_ROWS_TR;
@@ -996,6 +998,7 @@ static void merge_line_groups(const PassSpec &ps, TileArgs &a)
         a.c1 * (long long)a.c2 == 1)
         return;
     const long long m = a.c0, groups = (long long)a.c1 * a.c2;
+    if ((m + a.T - 1) / a.T * groups <= (fast ? ps.max_grid : 2 * device_cus())) return;
     const bool flat = a.c2 == 1 || (a.in_s2 == a.c1 * a.in_s1 && a.out_s2 == a.c1 * a.out_s1);
     if (a.in_s1 != m * a.in_s0 || (a.c2 > 1 && !flat) || m * groups >= (1LL << 31)) return;
     const unsigned mul = (65536u + (unsigned)m - 1) / (unsigned)m;
@@ -1035,7 +1038,7 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
             a.batch_base = b0;
         }
         const void *fn = ps.fn;
-        if (a.real_src && ps.fast_kind == KIND_ROWS) fn = (const void *)find_fast_ends(ps.R, ENDS_REAL);
+        if (a.real_src && ps.fast_kind == KIND_ROWS) fn = (const void *)find_fast_ends(ps.R, ENDS_REAL, FMT_C32);
         if (fz && fz->crop_out && &ps == &p->passes.back()) {
             a.crop_out = fz->crop_out;
             a.crop_b = fz->crop_b;
@@ -1048,7 +1051,10 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
             const long long planes = a.crop_b ? (long long)a.crop_b * a.crop_c : p->batch;
             a.crop_span = (unsigned)(4 * planes * a.crop_h * a.crop_w);
             a.batch_base = b0;
-            fn = (const void *)find_fast_ends(ps.R, ENDS_CROP);
+            a.crop_rows = p->nx;
+            a.crop_sp = (int)(ps.ps_out / p->ny);
+            a.crop_s2 = ps.l2 >= 0 ? (int)(ps.lines[ps.l2].out_stride / p->ny) : 0;
+            fn = (const void *)find_fast_ends(ps.R, ENDS_CROP, dst_fmt(p, ps));
         }
         a.in = buf_ptr(ps.src, in, out, work);
         a.out = buf_ptr(ps.dst, in, out, work);
@@ -2101,27 +2107,31 @@ bool plan_first_pass_fusable(mfft_plan p)
     return p && !p->passes.empty() && p->passes.front().small && p->passes.front().src == BUF_IN;
 }
 
-// A pass of a whole axis on a matrix-core kernel that has a form with this end fused: transforms
-// along l1 alone, fp32 words on both sides.
+// A pass on a matrix-core kernel that has a form with this end fused: transforms along l1, the same
+// words on both sides.
 static bool fast_ends_pass(mfft_plan p, const PassSpec &ps, int kind, int ends)
 {
     return !p->small && p->d.precision == PREC_SPLIT && ps.fast_kind == kind && !ps.tw_N && !ps.rev_fast && ps.l1 >= 0 &&
-           ps.lines[ps.l1].batch && ps.l2 < 0 && src_fmt(p, ps) == FMT_C32 && dst_fmt(p, ps) == FMT_C32 &&
-           find_fast_ends(ps.R, ends) != nullptr;
+           ps.lines[ps.l1].batch && src_fmt(p, ps) == dst_fmt(p, ps) && find_fast_ends(ps.R, ends, dst_fmt(p, ps)) != nullptr;
 }
 
 bool plan_takes_real(mfft_plan p, int f64, long long planes, int h, int w)
 {
     if (plan_first_pass_fusable(p)) return true;
     return p && p->kind == 2 && !p->passes.empty() && !f64 && planes * h * w < (1LL << 29) &&
-           p->passes.front().src == BUF_IN && p->passes.front().R == p->ny &&
+           p->passes.front().src == BUF_IN && p->passes.front().R == p->ny && p->passes.front().l2 < 0 &&
            fast_ends_pass(p, p->passes.front(), KIND_ROWS, ENDS_REAL);
 }
 
+// The last pass of the column axis, whole (R = nx) or the second of two (its l2 level is then the
+// first pass's frequency).
 bool plan_takes_crop(mfft_plan p, int f64, long long planes, int h, int w)
 {
-    return p && p->kind == 2 && !p->passes.empty() && !f64 && planes * h * w < (1LL << 29) && p->passes.back().col_axis &&
-           p->passes.back().R == p->nx && fast_ends_pass(p, p->passes.back(), KIND_COLS, ENDS_CROP);
+    if (!p || p->kind != 2 || p->passes.empty() || f64 || planes * h * w >= (1LL << 29)) return false;
+    const PassSpec &ps = p->passes.back();
+    if (!ps.col_axis || !fast_ends_pass(p, ps, KIND_COLS, ENDS_CROP)) return false;
+    if (ps.R == p->nx) return ps.l2 < 0;
+    return ps.l2 >= 0 && !ps.lines[ps.l2].batch && ps.lines[ps.l2].out_stride % p->ny == 0 && ps.ps_out % p->ny == 0;
 }
 
 int exec_fused(mfft_plan p, const void *in, void *out, int64_t batch, void *stream, const ExecFuse &f)

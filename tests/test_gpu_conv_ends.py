@@ -32,3 +32,22 @@ def test_fused_ends_match_separate_passes(dev, B, C, F, pad, h, w, fh, fw):
         op = Conv2d(B, C, F, h, w, fh, fw, mode="same", pad=pad)
         op.set_filters(f)
         assert torch.equal(op.forward(x), op.forward(x.double()).float())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("option", [{}, {"mid_fp16": True}, {"spec_fp16": True}])
+@pytest.mark.parametrize("pad,h,w,k", [((192, 64), 180, 50, 5), ((1088, 80), 1080, 70, 9), ((384, 128), 380, 100, 3),
+                                       ((768, 96), 700, 90, 7), ((2560, 68), 2500, 60, 5), ((3072, 64), 3066, 64, 1),
+                                       ((512, 48), 500, 40, 8)])
+def test_crop_in_the_last_pass_of_split_columns(dev, option, pad, h, w, k):
+    import torch
+
+    from fft_demo_amd.conv import Conv2d
+
+    g = torch.Generator(device=dev)
+    g.manual_seed(11)
+    x = torch.rand((3, 1, h, w), generator=g, device=dev)
+    f = torch.rand((1, 1, k, k), generator=g, device=dev)
+    op = Conv2d(3, 1, 1, h, w, k, k, mode="same", pad=pad, **option)
+    op.set_filters(f)
+    assert torch.equal(op.forward(x), op.forward(x.double()).float())
