@@ -382,8 +382,11 @@ static int plan_axis(std::vector<PassSpec> &out, long long L, long long ps_in, l
     const bool odd_split = perm_axis < 0 && split_hint != 1 && odd > 1 && small_odd(odd) && L / odd >= 16 &&
                            L / odd <= kMaxTile;
     const bool fast_cols = (perm_axis < 0 || rev_cols) && split_hint <= 1;  // no split asked for
+    // 1088 = 17 * 64 columns of 16-bit words at a wide pitch keep their two passes (1088 x 2048 x 14
+    // with 16-bit intermediates: 146 us, in one 150)
+    const bool wide = narrow && odd_split && L > 1024 && ps_in >= 2048;
     const bool one_mixed =
-        mixed >= 0 && perm_axis < 0 && split_hint <= 1 && mixed_one_pass(mixed, L, ps_in, ps_out, lines);
+        mixed >= 0 && perm_axis < 0 && split_hint <= 1 && !wide && mixed_one_pass(mixed, L, ps_in, ps_out, lines);
     if (one_mixed || (!odd_split && single_pass_ok((int)std::min<long long>(L, 1 << 30), ps_in, lines, fast_cols))) {
         PassSpec p;
         p.R = (int)L;
