@@ -343,7 +343,7 @@ static int mixed_col_lines(long long R)
 // pass and a power-of-two pass. Where the two passes stay (us, two passes / one): contiguous
 // lines above 2048 points with a factor 17 on the matrix cores, one line a tile, whose radix-17
 // stage then keeps a quarter of the threads busy (2176 x 4000 split fp16: 39 / 43, with 16-bit
-// intermediates 33 / 43; plain fp32 45 / 36, 3072 x 4000 split fp16 60 / 42); strided lines
+// intermediates 31 / 43; plain fp32 45 / 36, 3072 x 4000 split fp16 60 / 42); strided lines
 // above 1088 points with 16-bit words, 8 lines a tile, segments of 32 bytes (2176 x 2176 x 4
 // split fp16 110 / 151, plain fp32 209 / 185; 1088 x 1088 x 16 split fp16 129 / 119).
 static bool mixed_one_pass(int prec, long long L, long long ps_in, long long ps_out, const std::vector<Level> &lines)
