@@ -501,7 +501,8 @@ __global__ void __launch_bounds__(256) pointwise_gi_kernel(const float2 *D, cons
 // One block: 64 columns kx and a strip of rows ky of one filter's spectrum. The waves transform
 // the taps' rows along x into LDS; then a lane keeps its column's NR sums in registers, and a wave
 // takes one row ky at a time, the row's factors in scalar registers. The filter is real: row Ph -
-// ky is stored from row ky's sums.
+// ky is stored from row ky's sums. Both sums go in parts (four taps of a row, a quarter of the rows),
+// added up last: in one chain of 31 taps their rounding came to twice that of a transform's stages.
 template <typename T, int NR>
 __global__ void __launch_bounds__(256) filter_spectrum_kernel(const T *__restrict__ src, float2 *__restrict__ H,
                                                               const float2 *__restrict__ ty, const float2 *__restrict__ tx,
@@ -525,14 +526,13 @@ __global__ void __launch_bounds__(256) filter_spectrum_kernel(const T *__restric
         float2 a[NR / 4];
 #pragma unroll
         for (int j = 0; j < NR / 4; ++j) a[j] = make_float2(0.f, 0.f);
-#pragma unroll 4
-        for (int x = 0; x < fw; ++x) {
+        auto tap = [&](int x, float2 *p) {
             const float2 t = tx[(long long)x * Pw + kxc];
 #pragma unroll
             for (int j = 0; j < NR / 4; ++j) {
                 const float v = taps[x][wave + 4 * j];
-                a[j].x += v * t.x;
-                a[j].y += v * t.y;
+                p[j].x += v * t.x;
+                p[j].y += v * t.y;
             }
         }
 #pragma unroll
@@ -549,11 +549,26 @@ __global__ void __launch_bounds__(256) filter_spectrum_kernel(const T *__restric
     typedef __attribute__((address_space(4))) const float cf;
     for (int ky = strip * per + wave; ky < end; ky += 4) {
         const cf *t = (const cf *)(ty + (long long)ky * NR);
-        float2 a = make_float2(0.f, 0.f);
+        float2 p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j] = make_float2(0.f, 0.f);
 #pragma unroll
         for (int y = 0; y < NR; ++y) {
-            a.x += v[y].x * t[2 * y] - v[y].y * t[2 * y + 1];
-            a.y += v[y].x * t[2 * y + 1] + v[y].y * t[2 * y];
+        };
+        for (int x0 = 0; x0 < fw; x0 += 4) {
+            float2 p[NR / 4];
+#pragma unroll
+            for (int j = 0; j < NR / 4; ++j) p[j] = make_float2(0.f, 0.f);
+            if (x0 + 4 <= fw) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) tap(x0 + x, p);
+            } else {
+                for (int x = x0; x < fw; ++x) tap(x, p);
+            }
+#pragma unroll
+            for (int j = 0; j < NR / 4; ++j) a[j] = make_float2(a[j].x + p[j].x, a[j].y + p[j].y);
+            p[y / (NR / 4)].x += v[y].x * t[2 * y] - v[y].y * t[2 * y + 1];
+            p[y / (NR / 4)].y += v[y].x * t[2 * y + 1] + v[y].y * t[2 * y];
         }
         if (kx < Pw) {
             h[(long long)ky * Pw + kx] = a;
@@ -573,6 +588,7 @@ __global__ void gen_dft_rows_kernel(float2 *out, int n, int pitch, long long cou
     sincospi(2.0 * (double)e / (double)n, &sn, &cs);
     out[i] = make_float2((float)cs, (float)-sn);
 }
+        const float2 a = make_float2((p[0].x + p[1].x) + (p[2].x + p[3].x), (p[0].y + p[1].y) + (p[2].y + p[3].y));
 
 // out[b][c][y][x] = scale * (Re or Im) Y[b/2][c][(y + oy) mod Ph][(x + ox) mod Pw], oy < Ph and
 // ox < Pw; both images of a pair from one read (rows: pairs x C x oh).
