@@ -70,10 +70,19 @@ struct MixQueueArgs {
     MixItem item_in[kMixInline];
 };
 
+// Where a single radix-16 stage, the one on the matrix cores, stands among the others (two or more
+// always come last): its operands are 16-bit words, so what has been summed before it takes of fp16's
+// range, and what a scaled stage has divided by is lost to fp16's smallest value.
+enum MixOrder {
+    MIX_16_LAST,       // the fastest
+    MIX_16_AFTER_ODD,  // after the odd factors, before the even rest
+    MIX_16_EARLY,      // that, or first of all where that takes fewer stages
+    MIX_NO16,          // no such stage: all in fp32
+};
 // The radices of a length, stage order, as the kernels want them; false: not such a length.
-bool mix_radices(int n, std::vector<int> &out);
+bool mix_radices(int n, std::vector<int> &out, MixOrder order = MIX_16_LAST);
 // Schedule of a length for a precision (scale: every stage multiplies by 1/radix).
-bool mix_schedule(int n, int prec, bool scale, MixSched &sc);
+bool mix_schedule(int n, int prec, bool scale, MixOrder order, MixSched &sc);
 inline size_t mix_lds_bytes(int tile_points, int R) { return sizeof(float2) * ((size_t)tile_points + R); }
 
 // cap: 0 = contiguous lines, kMixColSmall or kMixColLarge = strided lines

@@ -60,8 +60,18 @@ const void *find_mixed_queue_kernel(int prec, int inf, int outf) { return find_m
 // Radices of n with the least sum of stage costs: a stage costs an LDS round trip of every
 // point (about 20 issue slots a point) plus its butterfly. 16 is the matrix-core stage; 6, 10,
 // 12 and 15 are coprime products, which save a round trip for a few additions.
-bool mix_radices(int n, std::vector<int> &out)
+bool mix_radices(int n, std::vector<int> &out, MixOrder order)
 {
+    if (order == MIX_16_EARLY) {
+        std::vector<int> last;
+        if (!mix_radices(n, last, MIX_16_LAST) || !mix_radices(n, out, MIX_16_AFTER_ODD)) return false;
+        if (last.size() < out.size()) {
+            const auto m16 = std::find(last.begin(), last.end(), 16);
+            std::rotate(last.begin(), m16, m16 + 1);
+            out = last;
+        }
+        return true;
+    }
     static const struct { int r; float cost; } kRadix[] = {{17, 51}, {16, 28}, {15, 31}, {12, 28}, {10, 29}, {9, 35},
                                                            {8, 27},  {6, 26},  {5, 27},  {4, 24},  {3, 24},  {2, 23}};
     out.clear();
@@ -76,9 +86,10 @@ bool mix_radices(int n, std::vector<int> &out)
             return;
         }
         for (size_t i = from; i < sizeof kRadix / sizeof *kRadix; ++i) {
-            if (m % kRadix[i].r) continue;
-            cur.push_back(kRadix[i].r);
-            go(m / kRadix[i].r, i, cost + kRadix[i].cost);
+            const int r = kRadix[i].r;
+            if (m % r || (order == MIX_NO16 && r == 16) || (order == MIX_16_AFTER_ODD && (r == 6 || r == 10 || r == 12))) continue;
+            cur.push_back(r);
+            go(m / r, i, cost + kRadix[i].cost);
             cur.pop_back();
         }
     };
@@ -91,7 +102,7 @@ bool mix_radices(int n, std::vector<int> &out)
     // one radix takes a copying first stage (radix 1).
     auto rank = [](int r) { return r == 16 ? 2 : (r & (r - 1)) == 0 ? 1 : 0; };
     std::stable_sort(best.begin(), best.end(), [&](int a, int b) { return rank(a) != rank(b) ? rank(a) < rank(b) : a > b; });
-    if ((n & (n - 1)) == 0 && best.size() > 1) {
+    if ((n & (n - 1)) == 0 && best.size() > 1 && order != MIX_NO16) {
         // [16, tail, 16, ...]; the lengths below 16 are one radix
         std::vector<int> o{16};
         for (int r : best)
@@ -100,29 +111,34 @@ bool mix_radices(int n, std::vector<int> &out)
         best = o;
     }
     if (best.size() == 1) best.insert(best.begin(), 1);
+    const auto m16 = std::find(best.begin(), best.end(), 16);
+    if (order == MIX_16_AFTER_ODD && std::count(best.begin(), best.end(), 16) == 1)
+        std::rotate(std::find_if(best.begin(), best.end(), [](int r) { return r % 2 == 0; }), m16, m16 + 1);
     out = best;
     return out.size() <= (size_t)kMixStages;
 }
 
-bool mix_schedule(int n, int prec, bool scale, MixSched &sc)
+bool mix_schedule(int n, int prec, bool scale, MixOrder order, MixSched &sc)
 {
     std::vector<int> r;
-    if (!mix_radices(n, r)) return false;
+    if (!mix_radices(n, r, prec == PREC_FP32 ? MIX_16_LAST : order)) return false;
     sc = MixSched();
     sc.R = n;
     sc.nst = (int)r.size();
     // The vector-ALU stages' scales are one factor on the first stage's outputs: before the
     // matrix-core stages (fp16 operands), whose own scale stays with them, as every stage's
-    // scale keeps values from growing past the input's magnitude.
+    // scale keeps values from growing past the input's magnitude. A last stage behind them has its own.
     float valu = 1.f;
     int s = 1;
+    bool behind = false;
     for (int i = 0; i < sc.nst; ++i) {
         const bool mfma = r[i] == 16 && prec != PREC_FP32;
         sc.radix[i] = r[i];
         sc.cols[i] = n / r[i];
         sc.s[i] = s;
         sc.mul[i] = mfma ? (scale ? 1.f / 256 : 1.f / 16) : 1.f;  // the operands carry a factor 16
-        if (scale && !mfma) valu /= r[i];
+        if (scale && !mfma) (behind && i == sc.nst - 1 ? sc.mul[i] : valu) /= r[i];
+        behind |= mfma;
         s *= r[i];
     }
     sc.mul[0] *= valu;

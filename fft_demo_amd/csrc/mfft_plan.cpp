@@ -638,6 +638,23 @@ static int mixed_tile_lines(int R, long long nlines, long long tiles)
     return (int)std::max(1LL, std::min(most, want));
 }
 
+// Order of a pass's stages on the mixed-radix kernels: none in which a 16-bit operand has less range
+// or precision than in the passes of the same axis in two, a streaming pass of the odd factor in fp32,
+// then the power of two, from 64 points on 16 before the even rest. (Strided lines of odd * 16 points
+// are two streaming passes: 272 x 64 bf16 3.0e-3 off, with a matrix-core stage 3.2e-3. 320 points, split
+// fp16 with 32-bit ends: unscaled inputs above 65504 / 5 overflow, with 16 last above 65504 / 20;
+// scaled ones of 2^-8 are 1.7e-5 off, with 16 last 3.5e-5.) Results of split fp16 in 16-bit words are
+// coarser than either; there 16 comes last, which rows of 64 and 128 times an odd factor run up to 5%
+// faster.
+static MixOrder mixed_order(const mfft_desc &d, int in_fmt, int R, bool cols)
+{
+    const int odd = (int)odd_part(R);
+    if (!small_odd(odd) || (d.precision == PREC_SPLIT && d.out_fmt != FMT_C32)) return MIX_16_LAST;
+    if (cols && R / odd == 16) return MIX_NO16;
+    if (R / odd < 64) return MIX_16_LAST;
+    return d.scale == MFFT_SCALE_STAGE || in_fmt != FMT_C32 ? MIX_16_EARLY : MIX_16_AFTER_ODD;
+}
+
 // Choose tile geometry and kernel for every pass.
 static int finish_passes(mfft_plan_s *p)
 {
@@ -766,7 +783,7 @@ static int finish_passes(mfft_plan_s *p)
             const int T = mixed_cols ? mixed_col_lines(ps.R) : 0;
             ps.mixed_cap = !mixed_cols ? 0 : ps.R * T <= kMixColSmall ? kMixColSmall : kMixColLarge;
             const void *fn = find_mixed_kernel(p->d.precision, in_fmt, out_fmt, ps.mixed_cap);
-            if (fn && mix_schedule(ps.R, p->d.precision, p->d.scale == MFFT_SCALE_STAGE, ps.mix)) {
+            if (fn && mix_schedule(ps.R, p->d.precision, p->d.scale == MFFT_SCALE_STAGE, mixed_order(p->d, in_fmt, ps.R, mixed_cols), ps.mix)) {
                 ps.mixed = true;
                 ps.fn = fn;
                 ps.radix.assign(ps.mix.radix, ps.mix.radix + ps.mix.nst);
@@ -1711,7 +1728,7 @@ static int batch_tables(mfft_batcher b, const mfft_batch_item *items, int nitems
     for (size_t i = 0; i < fresh.size() && e == hipSuccess; ++i) {
         len[i].tw = t;
         if (b->fn && (have + i >= kMixLengths ||
-                      !mix_schedule(fresh[i], b->d.precision, b->d.scale == MFFT_SCALE_STAGE, len[i].sc)))
+                      !mix_schedule(fresh[i], b->d.precision, b->d.scale == MFFT_SCALE_STAGE, MIX_16_LAST, len[i].sc)))
             e = hipErrorInvalidValue;
         else
             e = gen_twiddle(t, fresh[i], fresh[i], 1, b->d.direction, 0);
