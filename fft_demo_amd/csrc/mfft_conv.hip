@@ -11,6 +11,8 @@
 // (read_out_scale_double2double_kernel :1390-1397).
 #include "mfft_common.h"
 
+#include <type_traits>
+
 namespace mfft {
 
 // Image and product spectra are complex fp32 (FMT_C32) or fp16 (FMT_C16) per operator.
@@ -155,9 +157,15 @@ struct MapAt {
     int a0, b0;  // first map of the tile along each of the two map axes
 };
 
+// Tiles of one map (TA = TB = 1): the threads walk all planes without gaps, so that small planes
+// leave no lanes idle (p = P past the last one); na nb P < 2^31.
 template <int TA, int TB, int PTS = 256>
-__device__ __forceinline__ MapAt map_at(int na, int nb)
+__device__ __forceinline__ MapAt map_at(int na, int nb, long long P)
 {
+    if constexpr (TA * TB == 1) {
+        const unsigned i = blockIdx.x * 256 + threadIdx.x, n = (unsigned)P, t = i / n, a = t / (unsigned)nb;
+        return {a < (unsigned)na ? (long long)(i - t * n) : P, (int)a, (int)(t - a * (unsigned)nb)};
+    }
     const unsigned ta = (na + TA - 1) / TA, tb = (nb + TB - 1) / TB;
     unsigned r = blockIdx.x;
     const unsigned pb = r / (ta * tb);
@@ -168,48 +176,50 @@ __device__ __forceinline__ MapAt map_at(int na, int nb)
 
 static long long map_blocks(long long P, long long na, long long nb, int ta = kMapTile, int tb = kMapTile, int pts = 256)
 {
+    if (ta * tb == 1) return (P * na * nb + 255) / 256;
     return (P + pts - 1) / pts * ((na + ta - 1) / ta) * ((nb + tb - 1) / tb);
 }
 
-// Y[k][f][p] = sum_c X[k][c][p] * H[f][c][p]   (X, Y: FMT; H: fp32). A thread sums a tile of 4
-// pairs x 4 filters at its point: an X or H value is read once per tile instead of once per
-// output map (4 pairs, 3 channels, 16 filters of 256 x 256: 21.1 -> 16.5 us; memory-bound, 3.7 TB/s).
-template <int XFMT, int YFMT>
+// Y[k][f][p] = sum_c X[k][c][p] * H[f][c][p]   (X, Y: FMT; H: fp32). A thread sums a tile of T
+// pairs x T filters at its point: an X or H value is read once per tile instead of once per
+// output map (4 pairs, 3 channels, 16 filters of 256 x 256: 19.7 us with one map a thread, 15.9
+// with 4 x 4; memory-bound, 3.9 TB/s).
+template <int XFMT, int YFMT, int T>
 __global__ void __launch_bounds__(256) pointwise_mac_kernel(const void *X, const float2 *H, void *Y, int pairs, int C, int F,
                                                             long long P)
 {
-    const MapAt m = map_at<kMapTile, kMapTile>(pairs, F);
+    const MapAt m = map_at<T, T>(pairs, F, P);
     if (m.p >= P) return;
-    const int nk = min(kMapTile, pairs - m.a0), nf = min(kMapTile, F - m.b0);
-    float2 acc[kMapTile][kMapTile];
+    const int nk = min(T, pairs - m.a0), nf = min(T, F - m.b0);
+    float2 acc[T][T];
 #pragma unroll
-    for (int k = 0; k < kMapTile; ++k)
+    for (int k = 0; k < T; ++k)
 #pragma unroll
-        for (int f = 0; f < kMapTile; ++f) acc[k][f] = make_float2(0.f, 0.f);
+        for (int f = 0; f < T; ++f) acc[k][f] = make_float2(0.f, 0.f);
+    constexpr int U = T > 1 ? 2 : 1;
+#pragma unroll U
     for (int c = 0; c < C; ++c) {
-        float2 a[kMapTile], b[kMapTile];
+        // maps past the last one repeat it: the loads of a step stay in one block and in flight together
+        float2 a[T], b[T];
 #pragma unroll
-        for (int k = 0; k < kMapTile; ++k)
-            if (k < nk) a[k] = spec_ld<XFMT>(X, ((long long)(m.a0 + k) * C + c) * P + m.p);
+        for (int k = 0; k < T; ++k) a[k] = spec_ld<XFMT>(X, ((long long)(T > 1 ? min(m.a0 + k, pairs - 1) : m.a0) * C + c) * P + m.p);
 #pragma unroll
-        for (int f = 0; f < kMapTile; ++f)
-            if (f < nf) b[f] = H[((long long)(m.b0 + f) * C + c) * P + m.p];
+        for (int f = 0; f < T; ++f) b[f] = H[((long long)(T > 1 ? min(m.b0 + f, F - 1) : m.b0) * C + c) * P + m.p];
 #pragma unroll
-        for (int k = 0; k < kMapTile; ++k)
+        for (int k = 0; k < T; ++k)
 #pragma unroll
-            for (int f = 0; f < kMapTile; ++f)
-                if (k < nk && f < nf) {
-                    // which product is fused is fixed here, as the kernel of one output a thread had
-                    // it per format: 16-bit words further on show a change of it
-                    acc[k][f].x += __builtin_fmaf(a[k].x, b[f].x, -(a[k].y * b[f].y));
-                    acc[k][f].y += XFMT == FMT_C16 ? __builtin_fmaf(a[k].x, b[f].y, a[k].y * b[f].x)
-                                                   : __builtin_fmaf(a[k].y, b[f].x, a[k].x * b[f].y);
-                }
+            for (int f = 0; f < T; ++f) {
+                // which product is fused is fixed here, as the kernel of one output a thread had
+                // it per format: 16-bit words further on show a change of it
+                acc[k][f].x += __builtin_fmaf(a[k].x, b[f].x, -(a[k].y * b[f].y));
+                acc[k][f].y += XFMT == FMT_C16 ? __builtin_fmaf(a[k].x, b[f].y, a[k].y * b[f].x)
+                                               : __builtin_fmaf(a[k].y, b[f].x, a[k].x * b[f].y);
+            }
     }
 #pragma unroll
-    for (int k = 0; k < kMapTile; ++k)
+    for (int k = 0; k < T; ++k)
 #pragma unroll
-        for (int f = 0; f < kMapTile; ++f)
+        for (int f = 0; f < T; ++f)
             if (k < nk && f < nf) spec_st<YFMT>(Y, ((long long)(m.a0 + k) * F + m.b0 + f) * P + m.p, acc[k][f]);
 }
 
@@ -362,58 +372,57 @@ __global__ void crop_two_kernel(const void *Y, T *out0, T *out1, int oh, int ow,
 // where X_k = spectrum of the image pair (a + i b) and D_k of the delta pair (da + i db),
 // separated per frequency with X(-p): A = (X + X*)/2, B = (X - X*)/2i (X* = conj X(-p)).
 // Its inverse is sum_b in[b][c] (correlated with) delta[b][f], which is real: G(-p) = conj G(p),
-// so a thread computes a tile of TF filters x 4 channels at one point of the upper half plane
+// so a thread computes a tile of TF filters x TC channels at one point of the upper half plane
 // and stores both. Per-map threads over the whole plane re-read X and D for every map (4
-// pairs, 3 channels, 16 filters of 256 x 256: 28.9 -> 18.3 us; with TF = 2 and twice the blocks,
-// where 4 would give fewer than four a compute unit, 17.2).
-template <int TF>
+// pairs, 3 channels, 16 filters of 256 x 256: 27.2 us, 2 x 2 tiles 18.6).
+template <int TF, int TC>
 __global__ void __launch_bounds__(256) pointwise_gw_kernel(const float2 *X, const float2 *D, float2 *G, int pairs, int C, int F,
                                                            int Ph, int Pw)
 {
-    const MapAt m = map_at<TF, kMapTile>(F, C);
+    const MapAt m = map_at<TF, TC>(F, C, (long long)(Ph / 2 + 1) * Pw);
     if (m.p >= (long long)(Ph / 2 + 1) * Pw) return;
     const long long P = (long long)Ph * Pw;
     const unsigned u = (unsigned)m.p / (unsigned)Pw, v = (unsigned)m.p - u * (unsigned)Pw;
     const long long q = (long long)(u ? Ph - u : 0) * Pw + (v ? Pw - v : 0);
-    const int nf = min(TF, F - m.a0), nc = min(kMapTile, C - m.b0);
-    float2 g[TF][kMapTile];
+    const int nf = min(TF, F - m.a0), nc = min(TC, C - m.b0);
+    float2 g[TF][TC];
 #pragma unroll
     for (int f = 0; f < TF; ++f)
 #pragma unroll
-        for (int c = 0; c < kMapTile; ++c) g[f][c] = make_float2(0.f, 0.f);
+        for (int c = 0; c < TC; ++c) g[f][c] = make_float2(0.f, 0.f);
+    constexpr int U = TF * TC > 4 ? 1 : 2;
+#pragma unroll U
     for (int k = 0; k < pairs; ++k) {
-        float2 A[kMapTile], B[kMapTile];
+        // maps past the last one repeat it, as in pointwise_mac_kernel
+        float2 A[TC], B[TC];
 #pragma unroll
-        for (int c = 0; c < kMapTile; ++c)
-            if (c < nc) {
-                const float2 *x = X + ((long long)k * C + m.b0 + c) * P;
-                const float2 xp = x[m.p], xq = x[q];
-                // A = (xp + conj xq)/2, B = (xp - conj xq)/(2i)
-                A[c] = make_float2(0.5f * (xp.x + xq.x), 0.5f * (xp.y - xq.y));
-                B[c] = make_float2(0.5f * (xp.y + xq.y), -0.5f * (xp.x - xq.x));
+        for (int c = 0; c < TC; ++c) {
+            const float2 *x = X + ((long long)k * C + (TC > 1 ? min(m.b0 + c, C - 1) : m.b0)) * P;
+            const float2 xp = x[m.p], xq = x[q];
+            // A = (xp + conj xq)/2, B = (xp - conj xq)/(2i)
+            A[c] = make_float2(0.5f * (xp.x + xq.x), 0.5f * (xp.y - xq.y));
+            B[c] = make_float2(0.5f * (xp.y + xq.y), -0.5f * (xp.x - xq.x));
+        }
+#pragma unroll
+        for (int f = 0; f < TF; ++f) {
+            const float2 *d = D + ((long long)k * F + (TF > 1 ? min(m.a0 + f, F - 1) : m.a0)) * P;
+            const float2 dp = d[m.p], dq = d[q];
+            const float2 DA = make_float2(0.5f * (dp.x + dq.x), 0.5f * (dp.y - dq.y));
+            const float2 DB = make_float2(0.5f * (dp.y + dq.y), -0.5f * (dp.x - dq.x));
+            // A conj(DA) + B conj(DB)
+#pragma unroll
+            for (int c = 0; c < TC; ++c) {
+                g[f][c].x += A[c].x * DA.x + A[c].y * DA.y + B[c].x * DB.x + B[c].y * DB.y;
+                g[f][c].y += A[c].y * DA.x - A[c].x * DA.y + B[c].y * DB.x - B[c].x * DB.y;
             }
-#pragma unroll
-        for (int f = 0; f < TF; ++f)
-            if (f < nf) {
-                const float2 *d = D + ((long long)k * F + m.a0 + f) * P;
-                const float2 dp = d[m.p], dq = d[q];
-                const float2 DA = make_float2(0.5f * (dp.x + dq.x), 0.5f * (dp.y - dq.y));
-                const float2 DB = make_float2(0.5f * (dp.y + dq.y), -0.5f * (dp.x - dq.x));
-                // A conj(DA) + B conj(DB)
-#pragma unroll
-                for (int c = 0; c < kMapTile; ++c)
-                    if (c < nc) {
-                        g[f][c].x += A[c].x * DA.x + A[c].y * DA.y + B[c].x * DB.x + B[c].y * DB.y;
-                        g[f][c].y += A[c].y * DA.x - A[c].x * DA.y + B[c].y * DB.x - B[c].x * DB.y;
-                    }
-            }
+        }
     }
     // the rows that mirror into themselves (0 and, when Ph is even, Ph / 2) store their own points
     const bool both = u != 0 && 2 * u != (unsigned)Ph;
 #pragma unroll
     for (int f = 0; f < TF; ++f)
 #pragma unroll
-        for (int c = 0; c < kMapTile; ++c)
+        for (int c = 0; c < TC; ++c)
             if (f < nf && c < nc) {
                 float2 *o = G + ((long long)(m.a0 + f) * C + m.b0 + c) * P;
                 o[m.p] = g[f][c];
@@ -423,58 +432,67 @@ __global__ void __launch_bounds__(256) pointwise_gw_kernel(const float2 *X, cons
 
 // Input gradient spectrum: R[k][c][p] = sum_f D_k[f][p] conj(H[f][c][p]) with H the spectrum
 // of the 180-degree rotated filter; conj(H) is the spectrum of a real signal, so the image
-// pair stays separable in the inverse. Tiles of 4 pairs x 4 channels, as pointwise_mac_kernel.
+// pair stays separable in the inverse. Tiles of T pairs x T channels, as pointwise_mac_kernel.
 // NS: the waves of a block share 256 / NS points and each sums every NS-th filter: a layer has
 // few input maps, so one thread per point leaves most of the device idle (4 pairs, 3 channels, 16
-// filters of 256 x 256, 256 blocks of one point per thread: 18.5 us, split four ways 13.2).
-template <int NS>
+// filters of 256 x 256, 256 blocks of one point per thread: 17.4 us, split four ways 12.2).
+template <int NS, int T>
 __global__ void __launch_bounds__(256) pointwise_gi_kernel(const float2 *D, const float2 *H, float2 *R, int pairs, int C, int F,
                                                            long long P)
 {
     constexpr int PTS = 256 / NS;
-    __shared__ float2 red[NS > 1 ? NS : 1][kMapTile * kMapTile][NS > 1 ? PTS : 1];
-    const MapAt m = map_at<kMapTile, kMapTile, PTS>(pairs, C);
+    __shared__ float2 red[NS > 1 ? NS : 1][T * T][NS > 1 ? PTS : 1];
+    const MapAt m = map_at<T, T, PTS>(pairs, C, P);
     const int part = NS > 1 ? (int)threadIdx.x / PTS : 0, lane = threadIdx.x % PTS;
     const bool in = m.p < P;
-    const int nk = min(kMapTile, pairs - m.a0), nc = min(kMapTile, C - m.b0);
-    float2 acc[kMapTile][kMapTile];
+    const int nk = min(T, pairs - m.a0), nc = min(T, C - m.b0);
+    float2 acc[T][T];
 #pragma unroll
-    for (int k = 0; k < kMapTile; ++k)
+    for (int k = 0; k < T; ++k)
 #pragma unroll
-        for (int c = 0; c < kMapTile; ++c) acc[k][c] = make_float2(0.f, 0.f);
-    for (int f = part; f < F && in; f += NS) {
-        float2 d[kMapTile], h[kMapTile];
+        for (int c = 0; c < T; ++c) acc[k][c] = make_float2(0.f, 0.f);
+    auto step = [&](int f, auto whole) {
+        constexpr bool W = decltype(whole)::value;
+        float2 d[T], h[T];
 #pragma unroll
-        for (int k = 0; k < kMapTile; ++k)
-            if (k < nk) d[k] = D[((long long)(m.a0 + k) * F + f) * P + m.p];
+        for (int k = 0; k < T; ++k)
+            if (W || k < nk) d[k] = D[((long long)(m.a0 + k) * F + f) * P + m.p];
 #pragma unroll
-        for (int c = 0; c < kMapTile; ++c)
-            if (c < nc) h[c] = H[((long long)f * C + m.b0 + c) * P + m.p];
+        for (int c = 0; c < T; ++c)
+            if (W || c < nc) h[c] = H[((long long)f * C + m.b0 + c) * P + m.p];
 #pragma unroll
-        for (int k = 0; k < kMapTile; ++k)
+        for (int k = 0; k < T; ++k)
 #pragma unroll
-            for (int c = 0; c < kMapTile; ++c)
-                if (k < nk && c < nc) {
+            for (int c = 0; c < T; ++c)
+                if (W || (k < nk && c < nc)) {
                     acc[k][c].x += d[k].x * h[c].x + d[k].y * h[c].y;
                     acc[k][c].y += d[k].y * h[c].x - d[k].x * h[c].y;
                 }
+    };
+    // whole tiles without a branch between the loads of a step, which then are in flight together
+    if (T == 1 || (nk == T && nc == T)) {
+        constexpr int U = T > 1 ? 2 : 1;
+#pragma unroll U
+        for (int f = part; f < F && in; f += NS) step(f, std::true_type{});
+    } else {
+        for (int f = part; f < F && in; f += NS) step(f, std::false_type{});
     }
     if constexpr (NS > 1) {
-        // wave w finishes the tile's pair w (NS = kMapTile)
-        static_assert(NS == kMapTile, "one pair per part");
+        // wave w finishes the tile's pair w (NS = T)
+        static_assert(NS == T, "one pair per part");
 #pragma unroll
-        for (int k = 0; k < kMapTile; ++k)
+        for (int k = 0; k < T; ++k)
 #pragma unroll
-            for (int c = 0; c < kMapTile; ++c) red[part][k * kMapTile + c][lane] = acc[k][c];
+            for (int c = 0; c < T; ++c) red[part][k * T + c][lane] = acc[k][c];
         __syncthreads();
         if (!in || part >= nk) return;
 #pragma unroll
-        for (int c = 0; c < kMapTile; ++c)
+        for (int c = 0; c < T; ++c)
             if (c < nc) {
                 float2 s = make_float2(0.f, 0.f);
 #pragma unroll
                 for (int w = 0; w < NS; ++w) {
-                    const float2 t = red[w][part * kMapTile + c][lane];
+                    const float2 t = red[w][part * T + c][lane];
                     s.x += t.x;
                     s.y += t.y;
                 }
@@ -483,9 +501,9 @@ __global__ void __launch_bounds__(256) pointwise_gi_kernel(const float2 *D, cons
     } else {
         if (!in) return;
 #pragma unroll
-        for (int k = 0; k < kMapTile; ++k)
+        for (int k = 0; k < T; ++k)
 #pragma unroll
-            for (int c = 0; c < kMapTile; ++c)
+            for (int c = 0; c < T; ++c)
                 if (k < nk && c < nc) R[((long long)(m.a0 + k) * C + m.b0 + c) * P + m.p] = acc[k][c];
     }
 }
@@ -670,20 +688,38 @@ hipError_t conv_pack_filters(const void *src, int f64, float2 *dst, int FC, int 
                : launch_pack_filters((const float *)src, dst, FC, fh, fw, Ph, Pw, rotate, s);
 }
 
+// Blocks below which a launch of 256-thread blocks leaves compute units idle.
+constexpr long long kFillBlocks = 1024;
+
+// Whether tiles of one map may be used: their threads are numbered in 32 bits.
+static bool flat_fits(long long P, long long na, long long nb) { return map_blocks(P, na, nb, 1, 1) <= 0x7fffff; }
+
+template <int XFMT, int YFMT>
+static hipError_t launch_pointwise(const void *X, const float2 *H, void *Y, int pairs, int C, int F, long long P, hipStream_t s)
+{
+    // Tiles where both map axes have something to share and the launch fills the device; a tile's
+    // thread waits as long for each channel's loads, so with fewer blocks one map a thread is faster
+    // (us, tiles / one map: 1 pair, 128 channels, 16 filters of 64 x 64 59 / 37; 8 x 64 x 64 of 16 x 16,
+    // 32 blocks, 22 / 11; 2 x 8 x 8 of 192 x 192, 288 blocks, 7.9 / 7.0; 4 x 8 x 16 of 160 x 160, 400
+    // blocks, 12 / 17).
+    const int T = flat_fits(P, pairs, F) && (map_blocks(P, pairs, F) < 300 || pairs == 1 || F == 1) ? 1 : kMapTile;
+    const long long blocks = map_blocks(P, pairs, F, T, T);
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)blocks), block(256);
+    if (T == 1)
+        hipLaunchKernelGGL((pointwise_mac_kernel<XFMT, YFMT, 1>), grid, block, 0, s, X, H, Y, pairs, C, F, P);
+    else
+        hipLaunchKernelGGL((pointwise_mac_kernel<XFMT, YFMT, kMapTile>), grid, block, 0, s, X, H, Y, pairs, C, F, P);
+    return hipGetLastError();
+}
+
 hipError_t conv_pointwise(const void *X, const float2 *H, void *Y, int fmt, long long pairs, int C, int F, long long P,
                           hipStream_t s, int yfmt)
 {
-    const long long blocks = map_blocks(P, pairs, F);
-    if (blocks > 0x7fffffffLL || pairs > 0x7fffffffLL) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)blocks), block(256);
-    if (yfmt < 0) yfmt = fmt;
-    if (fmt == FMT_C16 && yfmt == FMT_C16)
-        hipLaunchKernelGGL((pointwise_mac_kernel<FMT_C16, FMT_C16>), grid, block, 0, s, X, H, Y, (int)pairs, C, F, P);
-    else if (fmt == FMT_C16)
-        hipLaunchKernelGGL((pointwise_mac_kernel<FMT_C16, FMT_C32>), grid, block, 0, s, X, H, Y, (int)pairs, C, F, P);
-    else
-        hipLaunchKernelGGL((pointwise_mac_kernel<FMT_C32, FMT_C32>), grid, block, 0, s, X, H, Y, (int)pairs, C, F, P);
-    return hipGetLastError();
+    if (pairs > 0x7fffffffLL) return hipErrorInvalidValue;
+    if (fmt != FMT_C16) return launch_pointwise<FMT_C32, FMT_C32>(X, H, Y, (int)pairs, C, F, P, s);
+    return yfmt < 0 || yfmt == FMT_C16 ? launch_pointwise<FMT_C16, FMT_C16>(X, H, Y, (int)pairs, C, F, P, s)
+                                       : launch_pointwise<FMT_C16, FMT_C32>(X, H, Y, (int)pairs, C, F, P, s);
 }
 
 hipError_t conv_quantise(const float2 *R, void *Q, float *partial, float *scale, long long maps, long long P,
@@ -726,35 +762,50 @@ hipError_t conv_crop(const void *Y, int fmt, void *out, int f64, int B, int F, i
     return launch_crop<FMT_C32>(Y, out, f64, B, F, oh, ow, Ph, Pw, oy, ox, scale, s, map_scale);
 }
 
-// Blocks below which a launch of 256-thread blocks leaves compute units idle.
-constexpr long long kFillBlocks = 1024;
-
 hipError_t conv_pointwise_gw(const float2 *X, const float2 *D, float2 *G, int pairs, int C, int F, int Ph, int Pw,
                              hipStream_t s)
 {
     const long long P = (long long)(Ph / 2 + 1) * Pw;
-    const bool small = map_blocks(P, F, C) < kFillBlocks;
-    const long long blocks = map_blocks(P, F, C, small ? 2 : kMapTile);
-    if (blocks > 0x7fffffffLL || (long long)Ph * Pw > 0x7fffffffLL) return hipErrorInvalidValue;
+    if ((long long)Ph * Pw > 0x7fffffffLL) return hipErrorInvalidValue;
+    // Tiles by the blocks that the largest would give; a tile's thread walks the pairs one after the
+    // other, so a launch of few blocks takes the time of one thread's walk (us, 4 x 4 / 2 x 2 / 1 x 1:
+    // 64 pairs, 3 channels, 8 filters of 16 x 16, 2 blocks, 80 / 17 / 11; 16 x 16 x 32 of 40 x 40, 128
+    // blocks, 39 / 12 / 20; 16 x 16 x 32 of 128 x 128, 1056 blocks, 62 / 84 / 211). 4 x 4 tiles of one
+    // filter or channel repeat loads (32 x 1 x 64 of 128 x 128: 121, 2 x 2 54).
+    const long long full = map_blocks(P, F, C);
+    const int T = full < 128 && flat_fits(P, F, C) ? 1 : full < kFillBlocks || F == 1 || C == 1 ? 2 : kMapTile;
+    const long long blocks = map_blocks(P, F, C, T, T);
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)blocks), block(256);
-    if (small)
-        hipLaunchKernelGGL(pointwise_gw_kernel<2>, grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
+    if (T == 1)
+        hipLaunchKernelGGL((pointwise_gw_kernel<1, 1>), grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
+    else if (T == 2)
+        hipLaunchKernelGGL((pointwise_gw_kernel<2, 2>), grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
     else
-        hipLaunchKernelGGL(pointwise_gw_kernel<kMapTile>, grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
+        hipLaunchKernelGGL((pointwise_gw_kernel<kMapTile, kMapTile>), grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
     return hipGetLastError();
 }
 
 hipError_t conv_pointwise_gi(const float2 *D, const float2 *H, float2 *R, long long pairs, int C, int F, long long P,
                              hipStream_t s)
 {
-    const bool split = F >= kMapTile && map_blocks(P, pairs, C) < kFillBlocks;
+    const long long full = map_blocks(P, pairs, C);
+    // One map a thread where tiles would leave the device idle or share nothing along an axis (us,
+    // one map / tiles: 64 pairs, 3 channels, 8 filters of 16 x 16, 16 blocks, 3.1 / 4.1; 1 x 32 x 32 of
+    // 128 x 128 21 / 26; 16 x 16 x 32 of 64 x 64, 256 blocks, 34 / 18); many filters gain from the split.
+    if (flat_fits(P, pairs, C) && F <= 32 && (full < 32 || ((pairs == 1 || C == 1) && full < kFillBlocks))) {
+        const dim3 flat((unsigned)map_blocks(P, pairs, C, 1, 1));
+        hipLaunchKernelGGL((pointwise_gi_kernel<1, 1>), flat, dim3(256), 0, s, D, H, R, (int)pairs, C, F, P);
+        return hipGetLastError();
+    }
+    const bool split = F >= kMapTile && full < kFillBlocks;
     const long long blocks = map_blocks(P, pairs, C, kMapTile, kMapTile, split ? 256 / kMapTile : 256);
     if (blocks > 0x7fffffffLL || pairs > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)blocks), block(256);
     if (split)
-        hipLaunchKernelGGL(pointwise_gi_kernel<kMapTile>, grid, block, 0, s, D, H, R, (int)pairs, C, F, P);
+        hipLaunchKernelGGL((pointwise_gi_kernel<kMapTile, kMapTile>), grid, block, 0, s, D, H, R, (int)pairs, C, F, P);
     else
-        hipLaunchKernelGGL(pointwise_gi_kernel<1>, grid, block, 0, s, D, H, R, (int)pairs, C, F, P);
+        hipLaunchKernelGGL((pointwise_gi_kernel<1, kMapTile>), grid, block, 0, s, D, H, R, (int)pairs, C, F, P);
     return hipGetLastError();
 }
 
