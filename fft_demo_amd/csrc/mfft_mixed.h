@@ -84,6 +84,12 @@ bool mix_radices(int n, std::vector<int> &out, MixOrder order = MIX_16_LAST);
 // Schedule of a length for a precision (scale: every stage multiplies by 1/radix).
 bool mix_schedule(int n, int prec, bool scale, MixOrder order, MixSched &sc);
 inline size_t mix_lds_bytes(int tile_points, int R) { return sizeof(float2) * ((size_t)tile_points + R); }
+// The most that a launch of a kernel takes (cap as find_mixed_kernel's): its largest tile beside the
+// longest line that comes in such tiles, 16 lines of 512 points or 8 of 2176.
+constexpr int mix_lds_max(int cap)
+{
+    return (int)sizeof(float2) * (!cap ? 2 * kMaxTile : cap + (cap == kMixColSmall ? kMixColSmall / 16 : kMixColLarge / 8));
+}
 
 // cap: 0 = contiguous lines, kMixColSmall or kMixColLarge = strided lines
 const void *find_mixed_kernel(int prec, int in_fmt, int out_fmt, int cap = 0);

@@ -792,16 +792,15 @@ static int finish_passes(mfft_plan_s *p)
                 ps.max_grid = 2 * device_cus();
                 ps.TL = 1;
                 ps.l0 = 0;
-                int lds = (int)mix_lds_bytes(kMaxTile, kMaxTile);
                 if (mixed_cols) {
                     for (int i = 0; i < (int)ps.lines.size(); ++i)
                         if (ps.lines[i].in_stride == 1 && ps.lines[i].out_stride == 1 && !ps.lines[i].batch) ps.l0 = i;
                     ps.T = (int)std::min<long long>(T, ps.lines[ps.l0].count);
-                    lds = (int)mix_lds_bytes(ps.mixed_cap, ps.R);
                 } else {
                     ps.T = mixed_tile_lines(ps.R, nl, ps.max_grid);
                 }
-                HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, std::max(lds, 65536)));
+                // every plan of the kernel sets its largest: plans share the function
+                HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, mix_lds_max(ps.mixed_cap)));
             }
         }
         if (rev && !ps.rev_fast && ps.perm_axis < 0)
@@ -1675,7 +1674,7 @@ int mfft_batcher_create(mfft_batcher *out, const mfft_desc *d, int max_items)
     if (b->fn) {
         if (e == hipSuccess) e = hipMalloc((void **)&b->lens, sizeof(MixLen) * kMixLengths);
         if (e == hipSuccess)
-            e = hipFuncSetAttribute(b->fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix_lds_bytes(kMaxTile, kMaxTile));
+            e = hipFuncSetAttribute(b->fn, hipFuncAttributeMaxDynamicSharedMemorySize, mix_lds_max(0));
     }
     for (auto &sl : b->slot) {
         if (b->fn) {
