@@ -1030,6 +1030,19 @@ static void merge_line_groups(const PassSpec &ps, TileArgs &a)
     a.out_s0 = 0;
 }
 
+// The runtime takes fewer than 2^32 threads a launch. A workgroup of the mixed-radix kernels has few
+// points where lines are few (columns of a narrow 2D transform), so a large batch goes in several
+// launches; kstart and kstop are then those of the first and the last.
+constexpr long long kMaxGridThreads = 0xffffffffLL;
+static hipError_t launch_mixed(const void *fn, void *arg, long long blocks, int threads, size_t lds, hipStream_t s,
+                               hipEvent_t kstart, hipEvent_t kstop)
+{
+    void *args[] = {arg};
+    const dim3 grid((unsigned)blocks), block(threads);
+    if (kstart || kstop) return hipExtLaunchKernel(fn, grid, block, args, lds, s, kstart, kstop, 0);
+    return hipLaunchKernel(fn, grid, block, args, lds, s);
+}
+
 // only >= 0: run that pass alone; kstart/kstop: events the runtime records around that
 // pass's kernel (its own execution window; one launch per exec).
 static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, hipStream_t s, hipEvent_t *ev,
@@ -1212,14 +1225,15 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
             m.out_dist = a.out_s1;
             memcpy(m.w16, g_w16, sizeof m.w16);
             m.sc = ps.mix;
-            const long long blocks = (long long)m.tiles0 * a.c1;
-            if (blocks >= (1LL << 31)) return fail(MFFT_ERR_UNSUPPORTED, "grid too large");
-            void *margs[] = {&m};
-            const size_t lds = mix_lds_bytes(m.T * ps.R, ps.R);
-            if (kstart || kstop)
-                HIP_TRY(hipExtLaunchKernel(ps.fn, dim3((unsigned)blocks), dim3(mix_col_threads(ps.mixed_cap)), margs, lds, s, kstart, kstop, 0));
-            else
-                HIP_TRY(hipLaunchKernel(ps.fn, dim3((unsigned)blocks), dim3(mix_col_threads(ps.mixed_cap)), margs, lds, s));
+            const int threads = mix_col_threads(ps.mixed_cap);
+            const long long step = std::max(1LL, kMaxGridThreads / threads / m.tiles0);
+            for (long long t0 = 0; t0 < a.c1; t0 += step) {
+                const long long nt = std::min<long long>(step, a.c1 - t0);
+                m.in = (const char *)a.in + t0 * m.in_dist * fmt_bytes(a.in_fmt);
+                m.out = (char *)a.out + t0 * m.out_dist * fmt_bytes(a.out_fmt);
+                HIP_TRY(launch_mixed(ps.fn, &m, nt * m.tiles0, threads, mix_lds_bytes(m.T * ps.R, ps.R), s, t0 ? nullptr : kstart,
+                                     t0 + nt < a.c1 ? nullptr : kstop));
+            }
             continue;
         }
         if (ps.mixed) {
@@ -1233,14 +1247,14 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
             m.sign = p->d.direction;
             memcpy(m.w16, g_w16, sizeof m.w16);
             m.sc = ps.mix;
-            const long long blocks = (m.nlines + m.T - 1) / m.T;
-            if (blocks >= (1LL << 31)) return fail(MFFT_ERR_UNSUPPORTED, "grid too large");
-            void *margs[] = {&m};
-            const size_t lds = mix_lds_bytes(m.T * ps.R, ps.R);
-            if (kstart || kstop)
-                HIP_TRY(hipExtLaunchKernel(ps.fn, dim3((unsigned)blocks), dim3(kMixThreads), margs, lds, s, kstart, kstop, 0));
-            else
-                HIP_TRY(hipLaunchKernel(ps.fn, dim3((unsigned)blocks), dim3(kMixThreads), margs, lds, s));
+            const long long lines = m.nlines, step = kMaxGridThreads / kMixThreads * m.T;
+            for (long long l0 = 0; l0 < lines; l0 += step) {
+                m.nlines = std::min(step, lines - l0);
+                m.in = (const char *)a.in + l0 * ps.R * fmt_bytes(a.in_fmt);
+                m.out = (char *)a.out + l0 * ps.R * fmt_bytes(a.out_fmt);
+                HIP_TRY(launch_mixed(ps.fn, &m, (m.nlines + m.T - 1) / m.T, kMixThreads, mix_lds_bytes(m.T * ps.R, ps.R), s,
+                                     l0 ? nullptr : kstart, l0 + m.nlines < lines ? nullptr : kstop));
+            }
             continue;
         }
         if (ps.small) {

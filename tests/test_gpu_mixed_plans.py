@@ -1,5 +1,6 @@
-"""GPU test of two plans on the mixed-radix kernels that share a kernel and take different amounts of
-LDS."""
+"""GPU tests of plans on the mixed-radix kernels beside other plans and at their limits: two plans that
+share a kernel and take different amounts of LDS, and batches of more workgroups than one launch may
+have."""
 import numpy as np
 import pytest
 
@@ -22,3 +23,25 @@ def test_plans_that_share_a_kernel(dev, prec, first, second):
         y = from_device(a.exec(to_device(x, dt, dev))) / a.out_scale
     l2, mx = rel_errors(y, oracle.fft2d(x))
     assert l2 <= (1e-5 if prec == "fp32" else 1e-3) and mx <= (4e-5 if prec == "fp32" else 4e-3), (l2, mx)
+
+
+@pytest.mark.gpu
+def test_more_workgroups_than_a_launch_takes(dev):
+    import torch
+
+    import fft_demo_amd as F
+
+    # one workgroup of 512 threads per transform's columns: 2^23 of them are 2^32 threads; the workspace
+    # holds all, so that the batch is not cut into chunks before
+    batch = (1 << 23) + 3
+    base = to_device(complex_input((1024, 48, 2), 5), torch.float16, dev)
+    x = base.repeat(batch // 1024 + 1, 1, 1, 1)[:batch].contiguous()
+    with F.Plan((48, 2), batch, precision="split_fp16", workspace_limit=8 << 30) as plan, \
+            F.Plan((48, 2), 1024, precision="split_fp16") as one:
+        assert plan.info["batch_chunk"] == batch
+        y = plan.exec(x)
+        want = one.exec(base)
+    del x
+    whole = batch // 1024 * 1024
+    assert torch.equal(y[:whole].view(-1, 1024, 48, 2, 2), want.expand(whole // 1024, 1024, 48, 2, 2))
+    assert torch.equal(y[whole:], want[:batch - whole])
