@@ -46,6 +46,9 @@ bool plan_takes_crop(mfft_plan p, int f64, long long planes, int h, int w);
 // input and the first pass does not take that.
 int exec_fused(mfft_plan p, const void *in, void *out, int64_t batch, void *stream, const ExecFuse &f);
 
+// Bytes of workspace that the plan's execs need, out of place or in place too.
+long long plan_scratch_bytes(mfft_plan p, bool in_place);
+
 // Set the calling thread's message returned by mfft_last_error().
 void set_last_error(const char *msg);
 

@@ -63,19 +63,17 @@ int noalloc_scratch(void **out)
 extern "C" int mfft_exec_noalloc(mfft_plan plan, const void *in, void *out, int64_t batch, void *stream)
 {
     if (!plan || !in || !out) return nfail(MFFT_ERR_INVALID, "mfft_exec_noalloc: null argument");
-    mfft_info inf;
-    int rc = mfft_plan_info(plan, &inf);
-    if (rc) return rc;
-    if (inf.workspace_bytes > MFFT_NOALLOC_SCRATCH_BYTES) {
+    const long long need = mfft::plan_scratch_bytes(plan, in == out);
+    if (need > MFFT_NOALLOC_SCRATCH_BYTES) {
         char buf[256];
         snprintf(buf, sizeof buf,
                  "mfft_exec_noalloc: the plan's intermediates take %lld bytes per batch chunk, more than the %lld "
                  "bytes of its scratch (create the plan with workspace_limit <= MFFT_NOALLOC_SCRATCH_BYTES)",
-                 (long long)inf.workspace_bytes, (long long)MFFT_NOALLOC_SCRATCH_BYTES);
+                 need, (long long)MFFT_NOALLOC_SCRATCH_BYTES);
         return nfail(MFFT_ERR_NOMEM, buf);
     }
     void *ws = nullptr;
-    rc = mfft::noalloc_scratch(&ws);
+    const int rc = mfft::noalloc_scratch(&ws);
     if (rc) return rc;
     return mfft_exec_ex(plan, in, out, batch, ws, stream);
 }

@@ -247,6 +247,10 @@ struct mfft_plan_s {
     // small_below transforms, which would leave most of the device idle on the on-chip pass.
     mfft_plan_s *small = nullptr;
     long long small_below = 0;
+    // A 1D plan of odd * 2^a points whose one pass writes elements of another size than it reads keeps
+    // the plan of an odd pass and a power-of-two pass, which meet in a workspace, for execs in place:
+    // in one pass, tiles would overwrite lines that others have not read.
+    mfft_plan_s *aliased = nullptr;
     // A transform of the conv operator: no mixed-radix kernels. Their stages round in another order
     // than the passes its filters and images have always gone through; with 16-bit words on the way
     // the difference grows to whole fp16 steps (1e-4 of the fp32 result), and the filter gradient's
@@ -1335,7 +1339,7 @@ static mfft_desc resolve_tuned(const mfft_desc *d, int nx, int ny, int64_t batch
     return r;
 }
 
-static int create_1d(mfft_plan *plan, int n, int64_t batch, const mfft_desc *d_in, bool allow_onchip)
+static int create_1d(mfft_plan *plan, int n, int64_t batch, const mfft_desc *d_in, bool allow_onchip, bool allow_mixed = true)
 {
     if (!plan || !d_in) return fail(MFFT_ERR_INVALID, "null argument");
     *plan = nullptr;
@@ -1365,9 +1369,16 @@ static int create_1d(mfft_plan *plan, int n, int64_t batch, const mfft_desc *d_i
     } else {
         std::vector<Level> lines{Level{batch, n, n, true}};
         rc = plan_axis(p->passes, n, 1, 1, lines, BUF_IN, BUF_OUT, rev ? 0 : -1, d->split_hint, narrow_mid(d), false,
-                       find_mixed_kernel(d->precision, d->in_fmt, d->out_fmt) ? d->precision : -1);
+                       allow_mixed && find_mixed_kernel(d->precision, d->in_fmt, d->out_fmt) ? d->precision : -1);
     }
     if (!rc) rc = finalize_plan(p);
+    if (!rc && allow_mixed && p->passes.size() == 1 && p->passes[0].mixed && fmt_bytes(d->in_fmt) != fmt_bytes(d->out_fmt)) {
+        rc = create_1d(&p->aliased, n, batch, &dt, false, false);
+        if (!rc && p->aliased->passes.size() == 1) {  // no better: a length without the two passes
+            mfft_plan_destroy(p->aliased);
+            p->aliased = nullptr;
+        }
+    }
     if (rc) {
         std::string msg = g_err;
         mfft_plan_destroy(p);
@@ -1518,11 +1529,23 @@ int mfft_plan_destroy(mfft_plan plan)
     if (!plan) return MFFT_OK;
     (void)hipDeviceSynchronize();
     if (plan->small) mfft_plan_destroy(plan->small);
+    if (plan->aliased) mfft_plan_destroy(plan->aliased);
     for (void *ptr : plan->allocs) (void)hipFree(ptr);
     plan->ws_order.destroy();
     delete plan;
     return MFFT_OK;
 }
+
+}  // extern "C"
+
+namespace mfft {
+long long plan_scratch_bytes(mfft_plan p, bool in_place)
+{
+    return std::max({p->work_bytes, p->small ? p->small->work_bytes : 0LL, in_place && p->aliased ? p->aliased->work_bytes : 0LL});
+}
+}  // namespace mfft
+
+extern "C" {
 
 int mfft_plan_info(mfft_plan p, mfft_info *info)
 {
@@ -1560,8 +1583,8 @@ int mfft_plan_info(mfft_plan p, mfft_info *info)
                     : ps.generic ? MFFT_KERNEL_GENERIC : MFFT_KERNEL_TILE;
     }
     info->out_scale = p->out_scale;
-    // a caller-supplied workspace also serves the companion plan of small execs
-    info->workspace_bytes = std::max(p->work_bytes, p->small ? p->small->work_bytes : 0LL);
+    // a caller-supplied workspace also serves the companion plans
+    info->workspace_bytes = std::max(mfft::plan_scratch_bytes(p, false), mfft::plan_scratch_bytes(p, true));
     info->batch_chunk = p->chunk;
     info->launches_per_exec = nchunks * (long long)p->passes.size();
     return MFFT_OK;
@@ -1574,6 +1597,10 @@ static int exec_all(mfft_plan p, const void *in, void *out, void *stream, hipEve
     if (p->small && batch >= 0 && batch < p->small_below && only < 0 && !ev &&
         (!fz || !fz->input() || (p->small->passes.front().small && p->small->passes.front().src == BUF_IN)))
         return exec_all(p->small, in, out, stream, nullptr, batch, work, fz, -1, nullptr, nullptr);
+    if (p->aliased && in == out) {
+        if (ev || only >= 0) return fail(MFFT_ERR_INVALID, "timing this plan's passes needs out != in");
+        return exec_all(p->aliased, in, out, stream, nullptr, batch, work);
+    }
     if (p->out_mid && in == out)
         for (const PassSpec &ps : p->passes) {
             // a pass that reads the input (not a fused real source) and writes the output in

@@ -1,6 +1,6 @@
 """GPU tests of plans on the mixed-radix kernels beside other plans and at their limits: two plans that
-share a kernel and take different amounts of LDS, and batches of more workgroups than one launch may
-have."""
+share a kernel and take different amounts of LDS, batches of more workgroups than one launch may
+have, and transforms in place that change the element size."""
 import numpy as np
 import pytest
 
@@ -45,3 +45,24 @@ def test_more_workgroups_than_a_launch_takes(dev):
     whole = batch // 1024 * 1024
     assert torch.equal(y[:whole].view(-1, 1024, 48, 2, 2), want.expand(whole // 1024, 1024, 48, 2, 2))
     assert torch.equal(y[whole:], want[:batch - whole])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,batch", [(480, 3000), (1152, 901), (2304, 5), (3840, 300)])
+@pytest.mark.parametrize("inf,outf", [("c16", "c32"), ("c32", "c16")])
+def test_in_place_with_another_element_size(dev, n, batch, inf, outf):
+    import torch
+
+    import fft_demo_amd as F
+
+    dt = {"c16": torch.float16, "c32": torch.float32}
+    x = complex_input((batch, n), n)
+    with F.Plan((n,), batch, precision="split_fp16", in_fmt=inf, out_fmt=outf) as plan:
+        xd = to_device(x, dt[inf], dev)
+        buf = torch.empty(batch * n * 8, dtype=torch.uint8, device=dev)  # holds either format
+        buf[:xd.numel() * xd.element_size()] = xd.view(-1).view(torch.uint8)
+        plan.exec_ptr(buf.data_ptr(), buf.data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
+        y = buf.view(dt[outf])[:2 * batch * n].view(batch, n, 2)
+        scale = plan.out_scale
+    l2, mx = rel_errors(from_device(y) / scale, oracle.fft(x))
+    assert l2 <= 1e-3 and mx <= 4e-3, (l2, mx)
