@@ -949,6 +949,15 @@ static int finalize_plan(mfft_plan_s *p)
     return build_tables(p);
 }
 
+// Lines per tile of a strided mixed-radix pass, of c0 lines per transform: fewer when the launch would
+// leave compute units without a tile.
+static int mixed_col_tile(const PassSpec &ps, long long c0, long long transforms)
+{
+    int T = ps.T;
+    while (T > 8 && (c0 + T - 1) / T * transforms < ps.max_grid / 2) T /= 2;
+    return T;
+}
+
 static int check_desc(const mfft_desc *d)
 {
     if (d->precision < 0 || d->precision > 3) return fail(MFFT_ERR_INVALID, "precision %d", d->precision);
@@ -975,6 +984,7 @@ static void trace_pass(const mfft_plan_s *p, const PassSpec &ps, const TileArgs 
                        hipStream_t s)
 {
     const char *fam = ps.small ? "stream"
+                      : ps.mixed ? (ps.mixed_cap ? "mixed_cols" : "mixed_rows")
                       : ps.fast_kind == KIND_ROWS ? "fast_rows"
                       : ps.fast_kind == KIND_ROWS_TR ? "fast_rows_tr"
                       : ps.fast_kind == KIND_COLS ? "fast_cols"
@@ -998,7 +1008,8 @@ static void trace_pass(const mfft_plan_s *p, const PassSpec &ps, const TileArgs 
     }
     if (a.in_mul) rd += std::min(pts, a.in_mul_period) * 8;
     char name[64];
-    snprintf(name, sizeof name, "%s R%d %s%s>%s", fam, ps.R, src, a.in_mul ? "*H" : "", fmt_name(a.out_fmt));
+    snprintf(name, sizeof name, "%s R%d %s%s>%s%s", fam, ps.R, src, a.in_mul ? "*H" : "",
+             a.crop_out ? "real32" : fmt_name(a.out_fmt), a.merge ? " merged" : "");
     (void)p;
     long long wr = pts * fmt_bytes(a.out_fmt);
     if (a.crop_out)  // the planes of the chunk's transforms (2 per transform, or 1)
@@ -1219,9 +1230,7 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
             m.dft_ops = p->ops;
             m.sign = p->d.direction;
             m.c0 = a.c0;
-            // fewer lines per tile when the launch would leave compute units without one
-            m.T = ps.T;
-            while (m.T > 8 && (long long)((a.c0 + m.T - 1) / m.T) * a.c1 < ps.max_grid / 2) m.T /= 2;
+            m.T = mixed_col_tile(ps, a.c0, a.c1);
             m.tiles0 = (a.c0 + m.T - 1) / m.T;
             m.ps_in = (int)a.in_ps;
             m.ps_out = (int)a.out_ps;
@@ -1569,12 +1578,21 @@ int mfft_plan_info(mfft_plan p, mfft_info *info)
         long long lines = 1;
         for (auto &l : ps.lines) lines *= l.batch ? p->chunk : l.count;
         long long c0 = ps.lines[ps.l0].batch ? p->chunk : ps.lines[ps.l0].count;
-        pi.tiles = (lines / c0) * ((c0 + ps.T - 1) / ps.T);
+        int T = ps.T;
+        if (ps.mixed && ps.mixed_cap) {
+            T = mixed_col_tile(ps, c0, lines / c0);
+        } else if (ps.mixed) {  // dense lines: tiled through all levels
+            c0 = lines;
+            T = mixed_tile_lines(ps.R, lines, ps.max_grid);
+        }
+        pi.lines_per_tile = T;
+        pi.tiles = (lines / c0) * ((c0 + T - 1) / T);
         pi.generic = ps.generic;
         pi.in_elem_bytes = fmt_bytes(src_fmt(p, ps));
         pi.out_elem_bytes = fmt_bytes(dst_fmt(p, ps));
         pi.points = lines * ps.R;
         pi.kernel = ps.small ? MFFT_KERNEL_STREAM
+                    : ps.mixed ? (ps.mixed_cap ? MFFT_KERNEL_MIXED_COLS : MFFT_KERNEL_MIXED_ROWS)
                     : ps.fast_kind == KIND_ROWS ? MFFT_KERNEL_ROWS
                     : ps.fast_kind == KIND_ROWS_TR ? MFFT_KERNEL_ROWS_TR
                     : ps.fast_kind == KIND_COLS ? MFFT_KERNEL_COLS

@@ -100,7 +100,9 @@ enum {
     MFFT_KERNEL_COLS = 4,      /* matrix-core kernel, strided 256-point lines (fft_fast) */
     MFFT_KERNEL_STREAM = 5,    /* streaming short-DFT kernel, one thread per line (small_cols) */
     MFFT_KERNEL_ONCHIP = 6,    /* one workgroup per 65536-point line, the intermediate on chip (fft_onchip) */
-    MFFT_KERNEL_ONCHIP_COLS = 7 /* 32 strided 2048-point columns per workgroup, on chip (fft_onchip_cols) */
+    MFFT_KERNEL_ONCHIP_COLS = 7, /* 32 strided 2048-point columns per workgroup, on chip (fft_onchip_cols) */
+    MFFT_KERNEL_MIXED_ROWS = 8, /* contiguous lines of 2^a 3^b 5^c 17^d points, whole in LDS (fft_mixed) */
+    MFFT_KERNEL_MIXED_COLS = 9  /* the same for strided lines (fft_mixed_cols) */
 };
 
 typedef struct mfft_info {
@@ -146,8 +148,8 @@ int mfft_exec_events(mfft_plan plan, const void *in, void *out, void *stream, vo
 int mfft_exec_pass(mfft_plan plan, int pass, const void *in, void *out, void *stream, void *start_event,
                    void *stop_event);
 
-/* Work-queue batching: many transforms of uneven length (n <= 4096, radices
- * {16, 8, 4, 2, 3, 5, 17}) and batch count in ONE launch of a persistent kernel that takes
+/* Work-queue batching: many transforms of uneven length (n <= 4096, a product of powers
+ * of 2, 3, 5 and 17) and batch count in ONE launch of a persistent kernel that takes
  * tiles from a device-side counter. Items are contiguous batches in the batcher's formats. */
 typedef struct mfft_batch_item {
     const void *in;

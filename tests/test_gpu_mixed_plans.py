@@ -1,6 +1,6 @@
 """GPU tests of plans on the mixed-radix kernels beside other plans and at their limits: two plans that
 share a kernel and take different amounts of LDS, batches of more workgroups than one launch may
-have, and transforms in place that change the element size."""
+have, transforms in place that change the element size, and what a plan reports of them."""
 import numpy as np
 import pytest
 
@@ -66,3 +66,16 @@ def test_in_place_with_another_element_size(dev, n, batch, inf, outf):
         scale = plan.out_scale
     l2, mx = rel_errors(from_device(y) / scale, oracle.fft(x))
     assert l2 <= 1e-3 and mx <= 4e-3, (l2, mx)
+
+
+@pytest.mark.gpu
+def test_reported_passes(dev):
+    import fft_demo_amd as F
+
+    with F.Plan((1200,), 3001, precision="split_fp16") as plan:
+        (p,) = plan.info["passes"]
+        assert p["kernel"] == "mixed_rows" and p["lines_per_tile"] == 3 and p["tiles"] == 1001
+    with F.Plan((48, 300), 5, precision="split_fp16") as plan:  # 5 x 48 rows, 5 x 300 columns
+        rows, cols = plan.info["passes"]
+        assert rows["kernel"] == "mixed_rows" and rows["lines_per_tile"] * rows["tiles"] >= 240
+        assert cols["kernel"] == "mixed_cols" and cols["lines_per_tile"] == 8 and cols["tiles"] == 5 * 38
