@@ -1023,7 +1023,11 @@ static void trace_pass(const mfft_plan_s *p, const PassSpec &ps, const TileArgs 
 // fast tile's 32 lines, 15 x 32 15 of a tile kernel's 128 (2176 points x 8704 lines, 16-bit words:
 // 39.2 -> 32.1 us; 480 x 15360, fp32: 113 -> 37.6). Not where the groups' own tiles all run at once:
 // fewer, fuller tiles then leave compute units idle (conv 183 x 657 x 2, 240 groups of 3 lines: 36
-// us, merged into 45 tiles 42).
+// us, merged into 45 tiles 42), nor up to four tiles a compute unit of the tile kernel's longer lines,
+// which has no small tiles for them, or where those are over 60% full: a merged store walks the output
+// value by value (whole set_filters calls of an fp16 operator, groups of 3 lines of 64 points: 768 of
+// them 27.9 us, merged into 36 tiles 31.6; 2048 of them 33.6, merged 29.8; 2048 groups of 3 x 1024
+// points 86 and 93).
 static void merge_line_groups(const PassSpec &ps, TileArgs &a)
 {
     const bool fast = ps.fast_kind == KIND_ROWS_TR;
@@ -1032,7 +1036,9 @@ static void merge_line_groups(const PassSpec &ps, TileArgs &a)
         a.c1 * (long long)a.c2 == 1)
         return;
     const long long m = a.c0, groups = (long long)a.c1 * a.c2;
-    if ((m + a.T - 1) / a.T * groups <= (fast ? ps.max_grid : 2 * device_cus())) return;
+    const long long own = (m + a.T - 1) / a.T * groups;
+    if (own <= (fast ? ps.max_grid : (a.R > 32 ? 4 : 2) * device_cus())) return;
+    if (tile && a.R > 32 && 5 * m * groups > 3 * own * a.T) return;
     const bool flat = a.c2 == 1 || (a.in_s2 == a.c1 * a.in_s1 && a.out_s2 == a.c1 * a.out_s1);
     if (a.in_s1 != m * a.in_s0 || (a.c2 > 1 && !flat) || m * groups >= (1LL << 31)) return;
     const unsigned mul = (65536u + (unsigned)m - 1) / (unsigned)m;
