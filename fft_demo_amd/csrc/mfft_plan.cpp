@@ -386,8 +386,10 @@ static int plan_axis(std::vector<PassSpec> &out, long long L, long long ps_in, l
     const bool odd_split = perm_axis < 0 && split_hint != 1 && odd > 1 && small_odd(odd) && L / odd >= 16 &&
                            L / odd <= kMaxTile;
     const bool fast_cols = (perm_axis < 0 || rev_cols) && split_hint <= 1;  // no split asked for
-    // 1088 = 17 * 64 columns of 16-bit words at a wide pitch keep their two passes (1088 x 2048 x 14
-    // with 16-bit intermediates: 146 us, in one 150)
+    // 1088 = 17 * 64 columns of 16-bit words at a wide pitch keep their two passes, for any batch (14
+    // transforms of 1088 x 2048, 3072 and 4096 with 16-bit intermediates: 133, 282 and 254 us, in one
+    // pass 142, 300 and 273; one and two of 1088 x 2048 30 and 37, in one 24 and 31; 3 of 1088 x 1024
+    // 37, in one 33)
     const bool wide = narrow && odd_split && L > 1024 && ps_in >= 2048;
     const bool one_mixed =
         mixed >= 0 && perm_axis < 0 && split_hint <= 1 && !wide && mixed_one_pass(mixed, L, ps_in, ps_out, lines);

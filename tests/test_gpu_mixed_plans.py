@@ -1,6 +1,7 @@
 """GPU tests of plans on the mixed-radix kernels beside other plans and at their limits: two plans that
 share a kernel and take different amounts of LDS, batches of more workgroups than one launch may
-have, transforms in place that change the element size, and what a plan reports of them."""
+have, transforms in place that change the element size, what a plan reports of them, and the columns
+whose number of passes depends on their pitch."""
 import numpy as np
 import pytest
 
@@ -79,3 +80,18 @@ def test_reported_passes(dev):
         rows, cols = plan.info["passes"]
         assert rows["kernel"] == "mixed_rows" and rows["lines_per_tile"] * rows["tiles"] >= 240
         assert cols["kernel"] == "mixed_cols" and cols["lines_per_tile"] == 8 and cols["tiles"] == 5 * 38
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ny,passes", [(1024, 2), (2048, 3)])  # one pass of columns; at a wide pitch two
+def test_columns_of_1088_points(dev, ny, passes):
+    import torch
+
+    import fft_demo_amd as F
+
+    x = complex_input((1, 1088, ny), ny)
+    with F.Plan((1088, ny), 1, precision="split_fp16", mid_fmt="c16") as plan:
+        assert len(plan.info["passes"]) == passes
+        y = from_device(plan.exec(to_device(x, torch.float16, dev))) / plan.out_scale
+    l2, mx = rel_errors(y, oracle.fft2d(x))
+    assert l2 <= 1e-3 and mx <= 4e-3, (l2, mx)
