@@ -39,10 +39,10 @@ __device__ __forceinline__ void spec_st(void *p, long long i, float2 v)
 
 // Row kernels: the elements of a launch are rows of `width` elements, V consecutive ones per
 // thread. A block of tx x ty threads covers ty rows, tx * V columns of each (xb blocks side by
-// side). tx is a multiple of 64, so a wave stays in one row, which it decodes once, in scalar
-// registers. Bound by
-// memory: 64 planes of 256 x 256 packed in 14.5 us, 3.3 TB/s (one element per thread, its index
-// divided down in 64 bits: 19.7 us).
+// side). Where tx is 64 or more, a wave stays in one row, which it decodes once, in scalar
+// registers; narrow rows share a wave (1024 planes of 64 x 64 packed in 10.9 us, with a wave for 32
+// pairs of columns 13.7). Bound by memory: 64 planes of 256 x 256 packed in 14.5 us, 3.3 TB/s (one
+// element per thread, its index divided down in 64 bits: 19.7 us).
 struct RowGrid {
     unsigned xb;
     dim3 grid, block;
@@ -53,7 +53,7 @@ static RowGrid row_grid(long long rows, int width, int V)
 {
     RowGrid g;
     const int per = (width + V - 1) / V;
-    unsigned tx = 64;
+    unsigned tx = 16;
     while (tx < 256 && tx < (unsigned)per) tx *= 2;
     const unsigned ty = 256 / tx;
     g.xb = (per + tx - 1) / tx;
@@ -64,16 +64,23 @@ static RowGrid row_grid(long long rows, int width, int V)
     return g;
 }
 
+// wave, narrow: the kernel for blocks whose rows are whole waves, and for others.
+template <typename... A, typename... B>
+static void launch_rows(void (*wave)(A...), void (*narrow)(A...), const RowGrid &g, hipStream_t s, B... args)
+{
+    hipLaunchKernelGGL(g.block.x >= 64 ? wave : narrow, g.grid, g.block, 0, s, static_cast<A>(args)...);
+}
+
 struct RowAt {
     unsigned row;
     int x;
 };
 
-template <int V>
+template <int V, bool WAVE>
 __device__ __forceinline__ RowAt row_at(unsigned xb)
 {
     const unsigned q = blockIdx.x / xb;
-    const unsigned ty = (unsigned)__builtin_amdgcn_readfirstlane((int)threadIdx.y);  // the wave's row
+    const unsigned ty = WAVE ? (unsigned)__builtin_amdgcn_readfirstlane((int)threadIdx.y) : threadIdx.y;  // WAVE: the wave's row
     return {q * blockDim.y + ty, (int)(((blockIdx.x - q * xb) * blockDim.x + threadIdx.x) * V)};
 }
 
@@ -90,11 +97,11 @@ __device__ __forceinline__ void spec_st2(void *p, long long i, float2 a, float2 
 // Two real images (batch items 2k and 2k+1, same channel) become the real and imaginary
 // parts of one complex image, zero-padded to Ph x Pw at the origin.
 // src: real [B][C][h][w] (fp32 or fp64); dst: complex [pairs][C][Ph][Pw] (FMT). V = 2: Pw even.
-template <typename T, int FMT, int V>
+template <typename T, int FMT, int V, bool WAVE>
 __global__ void pack_pairs_kernel(const T *src, void *dst, int B, int C, int h, int w, int Ph, int Pw, unsigned rows,
                                   unsigned xb)
 {
-    const RowAt at = row_at<V>(xb);
+    const RowAt at = row_at<V, WAVE>(xb);
     if (at.row >= rows || at.x >= Pw) return;
     const unsigned plane = at.row / (unsigned)Ph, y = at.row - plane * (unsigned)Ph;
     const unsigned k = plane / (unsigned)C, c = plane - k * (unsigned)C;
@@ -121,11 +128,11 @@ __global__ void pack_pairs_kernel(const T *src, void *dst, int B, int C, int h, 
 
 // Filter [F][C][fh][fw] real -> complex fp32 [F][C][Ph][Pw], optionally rotated by 180
 // degrees (convolution by the rotated filter = cross-correlation). V = 2: Pw even.
-template <typename T, int V>
+template <typename T, int V, bool WAVE>
 __global__ void pack_filters_kernel(const T *src, float2 *dst, int fh, int fw, int Ph, int Pw, int rotate, unsigned rows,
                                     unsigned xb)
 {
-    const RowAt at = row_at<V>(xb);
+    const RowAt at = row_at<V, WAVE>(xb);
     if (at.row >= rows || at.x >= Pw) return;
     const unsigned fc = at.row / (unsigned)Ph;
     const int y = (int)(at.row - fc * (unsigned)Ph);
@@ -285,11 +292,11 @@ __global__ void quant_apply_kernel(const float2 *R, uint32_t *Q, const float *pa
 // (each spectrum value is read once for both images; rows: pairs x F x oh). A thread takes V
 // consecutive columns (V = 4: one 16-byte store per image, for fp32 output rows whose width is a
 // multiple of 4 on a 16-byte aligned buffer).
-template <typename T, int FMT, int V>
+template <typename T, int FMT, int V, bool WAVE>
 __global__ void crop_unpack_kernel(const void *Y, T *out, int B, int F, int oh, int ow, int Ph, int Pw, int oy,
                                    int ox, float scale, unsigned rows, unsigned xb, const float *map_scale)
 {
-    const RowAt at = row_at<V>(xb);
+    const RowAt at = row_at<V, WAVE>(xb);
     if (at.row >= rows || at.x >= ow) return;
     const int x = at.x;
     const unsigned kf = at.row / (unsigned)oh;
@@ -611,11 +618,11 @@ __global__ void gen_dft_rows_kernel(float2 *out, int n, int pitch, long long cou
 
 // out[b][c][y][x] = scale * (Re or Im) Y[b/2][c][(y + oy) mod Ph][(x + ox) mod Pw], oy < Ph and
 // ox < Pw; both images of a pair from one read (rows: pairs x C x oh).
-template <typename T>
+template <typename T, bool WAVE>
 __global__ void crop_cyclic_kernel(const float2 *Y, T *out, int B, int C, int oh, int ow, int Ph, int Pw, int oy, int ox,
                                    float scale, unsigned rows, unsigned xb)
 {
-    const RowAt at = row_at<1>(xb);
+    const RowAt at = row_at<1, WAVE>(xb);
     if (at.row >= rows || at.x >= ow) return;
     const unsigned plane = at.row / (unsigned)oh, y = at.row - plane * (unsigned)oh;
     const unsigned k = plane / (unsigned)C, c = plane - k * (unsigned)C;
@@ -651,9 +658,9 @@ static hipError_t launch_pack_pairs(const T *src, void *dst, int B, int C, int h
     const RowGrid g = row_grid(rows, Pw, V);
     if (!g.ok) return hipErrorInvalidValue;
     if (V == 2)
-        hipLaunchKernelGGL((pack_pairs_kernel<T, FMT, 2>), g.grid, g.block, 0, s, src, dst, B, C, h, w, Ph, Pw, (unsigned)rows, g.xb);
+        launch_rows(pack_pairs_kernel<T, FMT, 2, true>, pack_pairs_kernel<T, FMT, 2, false>, g, s, src, dst, B, C, h, w, Ph, Pw, (unsigned)rows, g.xb);
     else
-        hipLaunchKernelGGL((pack_pairs_kernel<T, FMT, 1>), g.grid, g.block, 0, s, src, dst, B, C, h, w, Ph, Pw, (unsigned)rows, g.xb);
+        launch_rows(pack_pairs_kernel<T, FMT, 1, true>, pack_pairs_kernel<T, FMT, 1, false>, g, s, src, dst, B, C, h, w, Ph, Pw, (unsigned)rows, g.xb);
     return hipGetLastError();
 }
 
@@ -675,9 +682,9 @@ static hipError_t launch_pack_filters(const T *src, float2 *dst, int FC, int fh,
     const RowGrid g = row_grid(rows, Pw, V);
     if (!g.ok) return hipErrorInvalidValue;
     if (V == 2)
-        hipLaunchKernelGGL((pack_filters_kernel<T, 2>), g.grid, g.block, 0, s, src, dst, fh, fw, Ph, Pw, rotate, (unsigned)rows, g.xb);
+        launch_rows(pack_filters_kernel<T, 2, true>, pack_filters_kernel<T, 2, false>, g, s, src, dst, fh, fw, Ph, Pw, rotate, (unsigned)rows, g.xb);
     else
-        hipLaunchKernelGGL((pack_filters_kernel<T, 1>), g.grid, g.block, 0, s, src, dst, fh, fw, Ph, Pw, rotate, (unsigned)rows, g.xb);
+        launch_rows(pack_filters_kernel<T, 1, true>, pack_filters_kernel<T, 1, false>, g, s, src, dst, fh, fw, Ph, Pw, rotate, (unsigned)rows, g.xb);
     return hipGetLastError();
 }
 
@@ -744,13 +751,13 @@ static hipError_t launch_crop(const void *Y, void *out, int f64, int B, int F, i
     const RowGrid g = row_grid(rows, ow, vec ? 4 : 1);
     if (!g.ok) return hipErrorInvalidValue;
     if (f64)
-        hipLaunchKernelGGL((crop_unpack_kernel<double, FMT, 1>), g.grid, g.block, 0, s, Y, (double *)out, B, F, oh, ow, Ph, Pw,
+        launch_rows(crop_unpack_kernel<double, FMT, 1, true>, crop_unpack_kernel<double, FMT, 1, false>, g, s, Y, (double *)out, B, F, oh, ow, Ph, Pw,
                            oy, ox, scale, (unsigned)rows, g.xb, map_scale);
     else if (vec)
-        hipLaunchKernelGGL((crop_unpack_kernel<float, FMT, 4>), g.grid, g.block, 0, s, Y, (float *)out, B, F, oh, ow, Ph, Pw,
+        launch_rows(crop_unpack_kernel<float, FMT, 4, true>, crop_unpack_kernel<float, FMT, 4, false>, g, s, Y, (float *)out, B, F, oh, ow, Ph, Pw,
                            oy, ox, scale, (unsigned)rows, g.xb, map_scale);
     else
-        hipLaunchKernelGGL((crop_unpack_kernel<float, FMT, 1>), g.grid, g.block, 0, s, Y, (float *)out, B, F, oh, ow, Ph, Pw,
+        launch_rows(crop_unpack_kernel<float, FMT, 1, true>, crop_unpack_kernel<float, FMT, 1, false>, g, s, Y, (float *)out, B, F, oh, ow, Ph, Pw,
                            oy, ox, scale, (unsigned)rows, g.xb, map_scale);
     return hipGetLastError();
 }
@@ -878,10 +885,10 @@ hipError_t conv_crop_cyclic(const float2 *Y, void *out, int f64, int B, int C, i
     oy %= Ph;
     ox %= Pw;
     if (f64)
-        hipLaunchKernelGGL(crop_cyclic_kernel<double>, g.grid, g.block, 0, s, Y, (double *)out, B, C, oh, ow, Ph, Pw, oy, ox,
+        launch_rows(crop_cyclic_kernel<double, true>, crop_cyclic_kernel<double, false>, g, s, Y, (double *)out, B, C, oh, ow, Ph, Pw, oy, ox,
                            scale, (unsigned)rows, g.xb);
     else
-        hipLaunchKernelGGL(crop_cyclic_kernel<float>, g.grid, g.block, 0, s, Y, (float *)out, B, C, oh, ow, Ph, Pw, oy, ox,
+        launch_rows(crop_cyclic_kernel<float, true>, crop_cyclic_kernel<float, false>, g, s, Y, (float *)out, B, C, oh, ow, Ph, Pw, oy, ox,
                            scale, (unsigned)rows, g.xb);
     return hipGetLastError();
 }
