@@ -237,6 +237,7 @@ struct mfft_plan_s {
     long long work_bytes = 0;
     long long chunk = 1;
     double out_scale = 1.0;
+    long long cus = 256;      // compute units, asked for once (at every pass: 2 us of a 16 x 16 conv's 23)
     std::vector<void *> allocs;
     std::vector<int> rev_axis[2];
     std::vector<int> rev_list_axis[2];  // the radix lists rev_axis was generated from
@@ -664,6 +665,7 @@ static MixOrder mixed_order(const mfft_desc &d, int in_fmt, int R, bool cols)
 // Choose tile geometry and kernel for every pass.
 static int finish_passes(mfft_plan_s *p)
 {
+    p->cus = device_cus();
     for (auto &ps : p->passes) {
         if (ps.onchip_cols) {
             ps.radix = {16, 16, 8};
@@ -795,7 +797,7 @@ static int finish_passes(mfft_plan_s *p)
                 ps.radix.assign(ps.mix.radix, ps.mix.radix + ps.mix.nst);
                 long long nl = 1;
                 for (auto &l : ps.lines) nl *= l.count;
-                ps.max_grid = 2 * device_cus();
+                ps.max_grid = 2 * p->cus;
                 ps.TL = 1;
                 ps.l0 = 0;
                 if (mixed_cols) {
@@ -1030,7 +1032,7 @@ static void trace_pass(const mfft_plan_s *p, const PassSpec &ps, const TileArgs 
 // value by value (whole set_filters calls of an fp16 operator, groups of 3 lines of 64 points: 768 of
 // them 27.9 us, merged into 36 tiles 31.6; 2048 of them 33.6, merged 29.8; 2048 groups of 3 x 1024
 // points 86 and 93).
-static void merge_line_groups(const PassSpec &ps, TileArgs &a)
+static void merge_line_groups(const PassSpec &ps, long long cus, TileArgs &a)
 {
     const bool fast = ps.fast_kind == KIND_ROWS_TR;
     const bool tile = ps.fast_kind < 0 && !ps.small && !ps.mixed && !ps.generic && ps.TL == 1 && ps.ps_in == 1 && ps.ps_out != 1;
@@ -1039,7 +1041,7 @@ static void merge_line_groups(const PassSpec &ps, TileArgs &a)
         return;
     const long long m = a.c0, groups = (long long)a.c1 * a.c2;
     const long long own = (m + a.T - 1) / a.T * groups;
-    if (own <= (fast ? ps.max_grid : (a.R > 32 ? 4 : 2) * device_cus())) return;
+    if (own <= (fast ? ps.max_grid : (a.R > 32 ? 4 : 2) * cus)) return;
     if (tile && a.R > 32 && 5 * m * groups > 3 * own * a.T) return;
     const bool flat = a.c2 == 1 || (a.in_s2 == a.c1 * a.in_s1 && a.out_s2 == a.c1 * a.out_s1);
     if (a.in_s1 != m * a.in_s0 || (a.c2 > 1 && !flat) || m * groups >= (1LL << 31)) return;
@@ -1161,7 +1163,7 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
         a.in_rev = ps.rev_q;
         a.tw_rev = ps.rev_tw;
         memcpy(a.w16, g_w16, sizeof a.w16);
-        merge_line_groups(ps, a);
+        merge_line_groups(ps, p->cus, a);
         long long ntiles = ((a.c0 + a.T - 1) / a.T) * (long long)a.c1 * a.c2;
         if (a.merge && ps.fast_kind < 0 && ntiles < 4 * device_cus())
             // a full tile takes this kernel 11 us whatever the launch, a small one 6 (48 x 1680):
@@ -1834,7 +1836,7 @@ static int batch_exec_mixed(mfft_batcher b, const mfft_batch_item *items, int ni
     long long points = 0;
     for (int i = 0; i < nitems; ++i) points += items[i].count * items[i].n;
     // points per tile: kMaxTile, less when that would leave compute units without a tile
-    const long long cap = std::min<long long>(kMaxTile, std::max<long long>(kMixThreads, points / (2 * device_cus())));
+    const long long cap = std::min<long long>(kMaxTile, std::max<long long>(kMixThreads, points / (b->grid / 2)));
     MixQueueArgs q;
     q.lens = b->lens;
     q.dft_ops = b->ops;
