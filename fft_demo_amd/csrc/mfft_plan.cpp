@@ -33,7 +33,7 @@ hipError_t gen_dft_ops(DftOps *ops, int sign, hipStream_t s);
 hipError_t gen_w16(float *host3);
 typedef void (*tile_fn)(TileArgs);
 tile_fn find_tile_kernel(int prec, int R, int TL, bool generic);
-tile_fn find_small_tile_kernel(int prec, int R);
+tile_fn find_merged_tile_kernel(int prec, int R, bool small);
 int pow2_tile_lines(int R, int TL);
 hipError_t launch_tile(const void *fn, const TileArgs &a, long long ntiles, hipStream_t stream, hipEvent_t start = nullptr,
                        hipEvent_t stop = nullptr);
@@ -1035,7 +1035,7 @@ static void trace_pass(const mfft_plan_s *p, const PassSpec &ps, const TileArgs 
 static void merge_line_groups(const PassSpec &ps, long long cus, TileArgs &a)
 {
     const bool fast = ps.fast_kind == KIND_ROWS_TR;
-    const bool tile = ps.fast_kind < 0 && !ps.small && !ps.mixed && !ps.generic && ps.TL == 1 && ps.ps_in == 1 && ps.ps_out != 1;
+    const bool tile = ps.fast_kind < 0 && !ps.small && !ps.mixed && !ps.generic && ps.TL == 1 && ps.R <= 512 && ps.ps_in == 1 && ps.ps_out != 1;
     if ((!fast && !tile) || ps.tw_N || !ps.rev_list.empty() || a.in_perm || a.c0 % a.T == 0 || a.out_s0 != 1 ||
         a.c1 * (long long)a.c2 == 1)
         return;
@@ -1165,14 +1165,16 @@ static int exec_chunk(mfft_plan_s *p, const char *in, char *out, long long nb, h
         memcpy(a.w16, g_w16, sizeof a.w16);
         merge_line_groups(ps, p->cus, a);
         long long ntiles = ((a.c0 + a.T - 1) / a.T) * (long long)a.c1 * a.c2;
-        if (a.merge && ps.fast_kind < 0 && ntiles < 4 * device_cus())
+        if (a.merge && ps.fast_kind < 0) {
             // a full tile takes this kernel 11 us whatever the launch, a small one 6 (48 x 1680):
             // small ones until every compute unit has four full ones
-            if (const void *small = (const void *)find_small_tile_kernel(p->d.precision, ps.R)) {
-                fn = small;
+            const void *small = ntiles < 4 * p->cus ? (const void *)find_merged_tile_kernel(p->d.precision, ps.R, true) : nullptr;
+            fn = small ? small : (const void *)find_merged_tile_kernel(p->d.precision, ps.R, false);
+            if (small) {
                 a.T = kSmallTile / ps.R;
                 ntiles = ((a.c0 + a.T - 1) / a.T) * (long long)a.c1 * a.c2;
             }
+        }
         if (ntiles <= 0) continue;
         if (ntiles >= (1LL << 31)) return fail(MFFT_ERR_UNSUPPORTED, "grid too large");
         if (trace_active()) trace_pass(p, ps, a, nb, b0, s);
