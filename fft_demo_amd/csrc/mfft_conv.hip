@@ -381,7 +381,7 @@ __global__ void crop_two_kernel(const void *Y, T *out0, T *out1, int oh, int ow,
 // Its inverse is sum_b in[b][c] (correlated with) delta[b][f], which is real: G(-p) = conj G(p),
 // so a thread computes a tile of TF filters x TC channels at one point of the upper half plane
 // and stores both. Per-map threads over the whole plane re-read X and D for every map (4
-// pairs, 3 channels, 16 filters of 256 x 256: 27.2 us, 2 x 2 tiles 18.6).
+// pairs, 3 channels, 16 filters of 256 x 256: 27.3 us, 2 x 4 tiles 17.3).
 template <int TF, int TC>
 __global__ void __launch_bounds__(256) pointwise_gw_kernel(const float2 *X, const float2 *D, float2 *G, int pairs, int C, int F,
                                                            int Ph, int Pw)
@@ -704,12 +704,13 @@ static bool flat_fits(long long P, long long na, long long nb) { return map_bloc
 template <int XFMT, int YFMT>
 static hipError_t launch_pointwise(const void *X, const float2 *H, void *Y, int pairs, int C, int F, long long P, hipStream_t s)
 {
-    // Tiles where both map axes have something to share and the launch fills the device; a tile's
-    // thread waits as long for each channel's loads, so with fewer blocks one map a thread is faster
+    // Tiles where both map axes have something to share (one filter shares its spectrum, but with more
+    // than one channel to wait for that is not enough) and the launch fills the device; a tile's thread
+    // waits as long for each channel's loads, so with fewer blocks one map a thread is faster
     // (us, tiles / one map: 1 pair, 128 channels, 16 filters of 64 x 64 59 / 37; 8 x 64 x 64 of 16 x 16,
     // 32 blocks, 22 / 11; 2 x 8 x 8 of 192 x 192, 288 blocks, 7.9 / 7.0; 4 x 8 x 16 of 160 x 160, 400
     // blocks, 12 / 17).
-    const int T = flat_fits(P, pairs, F) && (map_blocks(P, pairs, F) < 300 || pairs == 1 || F == 1) ? 1 : kMapTile;
+    const int T = flat_fits(P, pairs, F) && (map_blocks(P, pairs, F) < 300 || pairs == 1 || (F == 1 && C > 1)) ? 1 : kMapTile;
     const long long blocks = map_blocks(P, pairs, F, T, T);
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)blocks), block(256);
@@ -775,19 +776,23 @@ hipError_t conv_pointwise_gw(const float2 *X, const float2 *D, float2 *G, int pa
     const long long P = (long long)(Ph / 2 + 1) * Pw;
     if ((long long)Ph * Pw > 0x7fffffffLL) return hipErrorInvalidValue;
     // Tiles by the blocks that the largest would give; a tile's thread walks the pairs one after the
-    // other, so a launch of few blocks takes the time of one thread's walk (us, 4 x 4 / 2 x 2 / 1 x 1:
-    // 64 pairs, 3 channels, 8 filters of 16 x 16, 2 blocks, 80 / 17 / 11; 16 x 16 x 32 of 40 x 40, 128
-    // blocks, 39 / 12 / 20; 16 x 16 x 32 of 128 x 128, 1056 blocks, 62 / 84 / 211). 4 x 4 tiles of one
-    // filter or channel repeat loads (32 x 1 x 64 of 128 x 128: 121, 2 x 2 54).
+    // other, so a launch of few blocks takes the time of one thread's walk (us, 4 x 4 / 2 x 4 / 2 x 2 /
+    // 1 x 1: 64 pairs, 3 channels, 8 filters of 16 x 16, 2 blocks, 80 / 57 / 17 / 11; 16 x 16 x 32 of 40 x
+    // 40, 128 blocks, 39 / 28 / 12 / 20; of 96 x 96, 608 blocks, 53 / 43 / 52 / 134; of 128 x 128, 1056
+    // blocks, 62 / 80 / 84 / 211). Tiles of four repeat loads along an axis of one map (32 x 1 x 64 of 128 x
+    // 128: 121 / 98 / 54 / 62).
     const long long full = map_blocks(P, F, C);
-    const int T = full < 128 && flat_fits(P, F, C) ? 1 : full < kFillBlocks || F == 1 || C == 1 ? 2 : kMapTile;
-    const long long blocks = map_blocks(P, F, C, T, T);
+    const int tf = full < 128 && flat_fits(P, F, C) ? 1 : full < kFillBlocks || F == 1 || C == 1 ? 2 : kMapTile;
+    const int tc = tf == 2 && full >= kFillBlocks / 2 && C >= 3 && F > 1 ? kMapTile : tf;
+    const long long blocks = map_blocks(P, F, C, tf, tc);
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)blocks), block(256);
-    if (T == 1)
+    if (tf == 1)
         hipLaunchKernelGGL((pointwise_gw_kernel<1, 1>), grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
-    else if (T == 2)
+    else if (tc == 2)
         hipLaunchKernelGGL((pointwise_gw_kernel<2, 2>), grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
+    else if (tf == 2)
+        hipLaunchKernelGGL((pointwise_gw_kernel<2, kMapTile>), grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
     else
         hipLaunchKernelGGL((pointwise_gw_kernel<kMapTile, kMapTile>), grid, block, 0, s, X, D, G, pairs, C, F, Ph, Pw);
     return hipGetLastError();
@@ -800,7 +805,7 @@ hipError_t conv_pointwise_gi(const float2 *D, const float2 *H, float2 *R, long l
     // One map a thread where tiles would leave the device idle or share nothing along an axis (us,
     // one map / tiles: 64 pairs, 3 channels, 8 filters of 16 x 16, 16 blocks, 3.1 / 4.1; 1 x 32 x 32 of
     // 128 x 128 21 / 26; 16 x 16 x 32 of 64 x 64, 256 blocks, 34 / 18); many filters gain from the split.
-    if (flat_fits(P, pairs, C) && F <= 32 && (full < 32 || ((pairs == 1 || C == 1) && full < kFillBlocks))) {
+    if (flat_fits(P, pairs, C) && F <= 32 && (full < 32 || ((pairs == 1 || (C == 1 && F > 1)) && full < kFillBlocks))) {
         const dim3 flat((unsigned)map_blocks(P, pairs, C, 1, 1));
         hipLaunchKernelGGL((pointwise_gi_kernel<1, 1>), flat, dim3(256), 0, s, D, H, R, (int)pairs, C, F, P);
         return hipGetLastError();
