@@ -7,7 +7,9 @@ intermediates between the two passes. One step = one exec of the whole batch wit
 input already resident in HBM; `value` is GFLOP/s = 5 N log2(N) batch / t over exactly
 --steps execs after --warmup untimed ones.
 
-The one JSON line also carries (all measured in the same run):
+--report FILE writes all of the following, measured in the same run, as one JSON object; the
+JSON line that is printed is its short form (under 6 KB: readers keep the last 8 KB of the
+output), with each object's values and without launch lists, schedules and texts:
   * rel-L2 / rel-max against the FP64 oracle; the fp32 (plain GPU FFT of this library,
     the ratio's denominator), fp16, bf16 and fp32-intermediate variants, torch.fft
     (rocFFT) as a labelled external point;
@@ -28,7 +30,7 @@ The one JSON line also carries (all measured in the same run):
     for --serve-seconds, default the full 30 s): p50/p99, throughput, the same trace in
     plain per-request fp32 mode, saturation and the equal-p99 ratio.
 
-python bench.py [--gpus 1] [--steps K] [--warmup W] [--config c1|c2|c3|c4|c5]
+python bench.py [--gpus 1] [--steps K] [--warmup W] [--config c1|c2|c3|c4|c5] [--report FILE]
 """
 from __future__ import annotations
 
@@ -1039,6 +1041,73 @@ def headline_line(cfg, args, dev, stream):
     return line
 
 
+def _pick(d, *keys):
+    return {k: d[k] for k in keys if k in d}
+
+
+def _short_roofline(r):
+    return _pick(r, "bound", "achieved", "peak", "unit", "frac", "traffic", "kernel", "algorithmic_bytes_per_launch",
+                 "avg_launch_ms", "copy_gbs", "frac_of_copy", "frac_of_same_size_copy")
+
+
+def _short_config(c):
+    out = _pick(c, "workload", "value", "unit", "ms_per_exec", "ms_per_batch", "steps", "precision", "rel_l2",
+                "rel_max", "pass_avg_ms", "plain_fp32", "ratio_vs_plain_fp32")
+    if "roofline" in c:
+        out["roofline"] = _short_roofline(c["roofline"])
+    if "cpu_baseline" in c:
+        out["cpu_baseline"] = _pick(c["cpu_baseline"], "value", "unit", "cores", "kind")
+    return out
+
+
+def _short_serve(s):
+    out = _pick(s, "workload", "requests", "saturation_ratio_vs_plain_fp32", "saturation_ratio_vs_plain_rocfft")
+    for mode in ("split", "plain_fp32"):
+        if mode in s:
+            out[mode] = _pick(s[mode], "p50_ms", "p99_ms", "req_per_s", "saturation_req_per_s", "launches",
+                              "coalesced", "paired", "peak_bytes")
+    if "equal_p99" in s:
+        out["equal_p99"] = _pick(s["equal_p99"], "p99_bound_ms", "sustained_req_per_s", "ratio")
+    return out
+
+
+def _round(o, digits=8):
+    """Floats to `digits` significant digits, at any depth."""
+    if isinstance(o, float):
+        return float(f"{o:.{digits}g}") if math.isfinite(o) else o
+    if isinstance(o, dict):
+        return {k: _round(v, digits) for k, v in o.items()}
+    return [_round(v, digits) for v in o] if isinstance(o, list) else o
+
+
+def short_line(report):
+    """The report without its launch lists, schedules and explanations: what is printed."""
+    line = {k: v for k, v in report.items() if k not in (
+        "passes", "pass_timing", "pass_check", "schedule", "settle", "comparators", "reference_api", "conv")}
+    if "roofline" in line:
+        line["roofline"] = _short_roofline(line["roofline"])
+    if "comparators" in report:
+        line["comparators"] = {k: _pick(v, "gflops", "ms_per_exec", "rel_l2")
+                               for k, v in report["comparators"].items()}
+    if "reference_api" in report:
+        line["reference_api"] = {k: _pick(report["reference_api"][k], "ms_per_exec", "gflops", "rel_l2", "ok")
+                                 for k in ("tcfftExec", "doit") if k in report["reference_api"]}
+    if "configs" in report:
+        line["configs"] = {k: _short_config(v) for k, v in report["configs"].items()}
+    if "conv" in report:
+        line["conv"] = _short_config(report["conv"])
+    if "serve" in report:
+        line["serve"] = _short_serve(report["serve"])
+    return _round(line)
+
+
+def emit(report, path):
+    if path:
+        with open(path, "w") as f:
+            json.dump(report, f, indent=1)
+    print(json.dumps(short_line(report)))
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -1060,6 +1129,7 @@ def main():
                          "scales rocprofv3 FETCH_SIZE / WRITE_SIZE readings)")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-compare", action="store_true", help="headline precision only")
+    ap.add_argument("--report", metavar="FILE", help="write the whole report (launch lists, schedules) here as JSON")
     args = ap.parse_args()
     if args.steps is None:
         args.steps = 1000 if args.config == "c1" else 200
@@ -1088,18 +1158,17 @@ def main():
         return
     if args.config == "c4":
         cv = conv_config(args.steps, args.warmup, with_cpu=not args.no_cpu)
-        print(json.dumps({"metric": METRIC, "value": cv["value"], "unit": "images/s", "n_gpus": 1,
-                          "steps": args.steps, "warmup": args.warmup, "ms_per_step": cv["ms_per_batch"],
-                          "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "fp16",
-                          "data": "synthetic", "config": {"workload": cv["workload"]}, "roofline": cv["roofline"],
-                          "cpu_baseline": cv.get("cpu_baseline"), "conv": cv}))
+        emit({"metric": METRIC, "value": cv["value"], "unit": "images/s", "n_gpus": 1, "steps": args.steps,
+              "warmup": args.warmup, "ms_per_step": cv["ms_per_batch"], "higher_is_better": True, "scaling": "weak",
+              "vs_baseline": None, "dtype": "fp16", "data": "synthetic", "config": {"workload": cv["workload"]},
+              "roofline": cv["roofline"], "cpu_baseline": cv.get("cpu_baseline"), "conv": cv}, args.report)
         return
     if args.config == "c5":
         sv = serve_section(args.serve_seconds, p99_bound_ms=args.serve_p99_ms)
-        print(json.dumps({"metric": METRIC, "value": sv["split"]["p99_ms"], "unit": "ms (p99)", "n_gpus": 1,
-                          "steps": sv["requests"], "warmup": 0, "ms_per_step": None, "higher_is_better": False,
-                          "scaling": "weak", "vs_baseline": None, "dtype": "fp16", "data": "synthetic",
-                          "config": {"workload": sv["workload"]}, "serve": sv}))
+        emit({"metric": METRIC, "value": sv["split"]["p99_ms"], "unit": "ms (p99)", "n_gpus": 1,
+              "steps": sv["requests"], "warmup": 0, "ms_per_step": None, "higher_is_better": False,
+              "scaling": "weak", "vs_baseline": None, "dtype": "fp16", "data": "synthetic",
+              "config": {"workload": sv["workload"]}, "serve": sv}, args.report)
         return
     line = headline_line(args.config, args, dev, stream)
     print(f"[bench] {args.config}: {line['value']} GFLOP/s", file=sys.stderr, flush=True)
@@ -1119,7 +1188,7 @@ def main():
     if not args.no_serve:
         torch.cuda.empty_cache()
         line["serve"] = serve_section(args.serve_seconds, p99_bound_ms=args.serve_p99_ms)
-    print(json.dumps(line))
+    emit(line, args.report)
 
 
 if __name__ == "__main__":
