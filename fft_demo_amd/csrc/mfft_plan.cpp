@@ -1628,8 +1628,15 @@ static int exec_all(mfft_plan p, const void *in, void *out, void *stream, hipEve
         (!fz || !fz->input() || (p->small->passes.front().small && p->small->passes.front().src == BUF_IN)))
         return exec_all(p->small, in, out, stream, nullptr, batch, work, fz, -1, nullptr, nullptr);
     if (p->aliased && in == out) {
-        if (ev || only >= 0) return fail(MFFT_ERR_INVALID, "timing this plan's passes needs out != in");
-        return exec_all(p->aliased, in, out, stream, nullptr, batch, work);
+        // timed as the plan's one pass: all of the other plan's lies between the events
+        const long long launches = ev ? ((batch < 0 ? p->batch : batch) + p->chunk - 1) / p->chunk : 0;
+        if (ev) HIP_TRY(hipEventRecord(ev[0], (hipStream_t)stream));
+        if (kstart) HIP_TRY(hipEventRecord(kstart, (hipStream_t)stream));
+        const int rc = exec_all(p->aliased, in, out, stream, nullptr, batch, work);
+        if (rc) return rc;
+        if (kstop) HIP_TRY(hipEventRecord(kstop, (hipStream_t)stream));
+        for (long long i = 1; i <= launches; ++i) HIP_TRY(hipEventRecord(ev[i], (hipStream_t)stream));
+        return MFFT_OK;
     }
     if (p->out_mid && in == out)
         for (const PassSpec &ps : p->passes) {

@@ -70,6 +70,32 @@ def test_in_place_with_another_element_size(dev, n, batch, inf, outf):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("timed", ["events", "pass"])
+def test_in_place_with_another_element_size_timed(dev, timed):
+    import torch
+
+    import fft_demo_amd as F
+    from fft_demo_amd import _lib, hiptime
+
+    lib = _lib.load()
+    n, batch = 480, 3000
+    x = complex_input((batch, n), n)
+    with F.Plan((n,), batch, precision="split_fp16", in_fmt="c32", out_fmt="c16") as plan:
+        want = from_device(plan.exec(to_device(x, torch.float32, dev)))
+        buf = to_device(x, torch.float32, dev)
+        s, ptr, pool = torch.cuda.current_stream(dev).cuda_stream, buf.data_ptr(), hiptime.EventPool(2)
+        if timed == "events":
+            assert lib.mfft_exec_events(plan._h, ptr, ptr, s, pool.slice(0), 2) == 0
+        else:
+            assert lib.mfft_exec_pass(plan._h, 0, ptr, ptr, s, pool.arr[0], pool.arr[1]) == 0
+        assert pool.elapsed_ms(0, 1) > 0
+        y = from_device(buf.view(torch.float16).view(-1)[:2 * batch * n].view(batch, n, 2))
+        pool.close()
+    l2, mx = rel_errors(y, want)
+    assert l2 <= 1e-3 and mx <= 4e-3, (l2, mx)
+
+
+@pytest.mark.gpu
 def test_reported_passes(dev):
     import fft_demo_amd as F
 
