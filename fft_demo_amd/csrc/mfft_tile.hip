@@ -175,11 +175,15 @@ __device__ __forceinline__ void dft16_mfma(const float2 x[4], const DftOps *ops,
     }
 }
 
+// The stages and copies below are inlined by force: called by two kernels of a size each, they
+// otherwise become functions, 140 registers for every kernel that calls one (32 points x 131072, split
+// fp16, 20.2 us; inlined, 104 registers, 15.5).
+
 // One radix-16 Stockham stage on the matrix cores, in place in LDS.
 // Stage with stride s (product of earlier radices): column col = q + s*p reads points
 // col + j*R/16 (j = 0..15) and writes point q + s*(16p + t) scaled by W_{R/s}^{p*t}.
 template <int PREC, class Geo>
-__device__ void stage16_mfma(float2 *lds, const Geo &G, int s, float mul, const TileArgs &a)
+__device__ __forceinline__ void stage16_mfma(float2 *lds, const Geo &G, int s, float mul, const TileArgs &a)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, c = lane & 15;
@@ -331,7 +335,7 @@ __device__ __forceinline__ void dft_odd(float2 *v, const float2 *tw, int Rdiv)
 
 // One radix-RADIX Stockham stage on the vector ALUs (fp32), in place in LDS.
 template <int RADIX, class Geo>
-__device__ void stage_valu(float2 *lds, const Geo &G, int s, float mul, const TileArgs &a)
+__device__ __forceinline__ void stage_valu(float2 *lds, const Geo &G, int s, float mul, const TileArgs &a)
 {
     const int R = G.R, TL = G.TL;
     const int cols = R / RADIX;
@@ -396,7 +400,7 @@ __device__ __forceinline__ TileOrigin tile_origin(const TileArgs &a, long long t
 }
 
 template <class Geo>
-__device__ void copy_in(float2 *lds, const Geo &G, const TileArgs &a, const TileOrigin &o)
+__device__ __forceinline__ void copy_in(float2 *lds, const Geo &G, const TileArgs &a, const TileOrigin &o)
 {
     const int R = G.R, T = G.T;
     const int *perm = a.in_perm;
@@ -491,7 +495,7 @@ __device__ __forceinline__ float2 out_value(const float2 *lds, const Geo &G, con
 // MERGE: for launches of merged line groups, in kernels of their own: with both ways in one kernel a
 // launch of one tile takes 5.4 us instead of 4.6 (16 x 16 plane, fp32).
 template <bool MERGE, class Geo>
-__device__ void copy_out(const float2 *lds, const Geo &G, const TileArgs &a, const TileOrigin &o)
+__device__ __forceinline__ void copy_out(const float2 *lds, const Geo &G, const TileArgs &a, const TileOrigin &o)
 {
     const int R = G.R;
     const int nv = o.nvalid;
