@@ -7,8 +7,8 @@
 namespace mfft {
 
 constexpr int kMixThreads = 512;
-constexpr int kMixColSmall = 8192, kMixColLarge = 17408;  // points per tile of the strided kernels
-constexpr int mix_col_threads(int cap) { return cap == kMixColSmall ? 512 : 1024; }
+constexpr int kMixColTiny = 2048, kMixColSmall = 8192, kMixColLarge = 17408;  // points per tile of the strided kernels
+constexpr int mix_col_threads(int cap) { return cap == kMixColTiny ? 256 : cap == kMixColSmall ? 512 : 1024; }
 constexpr int kMixStages = 8;
 constexpr int kMixInline = 64;  // work-queue items that travel in the kernel's arguments
 
@@ -85,13 +85,13 @@ bool mix_radices(int n, std::vector<int> &out, MixOrder order = MIX_16_LAST);
 bool mix_schedule(int n, int prec, bool scale, MixOrder order, MixSched &sc);
 inline size_t mix_lds_bytes(int tile_points, int R) { return sizeof(float2) * ((size_t)tile_points + R); }
 // The most that a launch of a kernel takes (cap as find_mixed_kernel's): its largest tile beside the
-// longest line that comes in such tiles, 16 lines of 512 points or 8 of 2176.
+// longest line that comes in such tiles, 16 lines of 512 points or 8 of 2176, or a single one.
 constexpr int mix_lds_max(int cap)
 {
-    return (int)sizeof(float2) * (!cap ? 2 * kMaxTile : cap + (cap == kMixColSmall ? kMixColSmall / 16 : kMixColLarge / 8));
+    return (int)sizeof(float2) * (!cap ? 2 * kMaxTile : cap + (cap == kMixColTiny ? kMixColTiny : cap == kMixColSmall ? kMixColSmall / 16 : kMixColLarge / 8));
 }
 
-// cap: 0 = contiguous lines, kMixColSmall or kMixColLarge = strided lines
+// cap: 0 = contiguous lines, kMixColTiny, kMixColSmall or kMixColLarge = strided lines
 const void *find_mixed_kernel(int prec, int in_fmt, int out_fmt, int cap = 0);
 const void *find_mixed_queue_kernel(int prec, int in_fmt, int out_fmt);
 

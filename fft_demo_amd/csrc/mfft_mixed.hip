@@ -20,6 +20,7 @@ static const void *pick_mixed(int what)
     switch (what) {
     case 0: return (const void *)mixed::fft_mixed<PREC, INF, OUTF>;
     case kMixQueue: return (const void *)mixed::fft_mixed_queue<PREC, INF, OUTF>;
+    case kMixColTiny: return (const void *)mixed::fft_mixed_cols<kMixColTiny, PREC, INF, OUTF>;
     case kMixColSmall: return (const void *)mixed::fft_mixed_cols<kMixColSmall, PREC, INF, OUTF>;
     case kMixColLarge: return (const void *)mixed::fft_mixed_cols<kMixColLarge, PREC, INF, OUTF>;
     default: return nullptr;

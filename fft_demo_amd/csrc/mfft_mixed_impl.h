@@ -10,8 +10,8 @@
 // between the barriers of a stage (81-100 registers, 2-4 workgroups per compute unit by LDS);
 // the geometry is runtime, so every index is a product with a reciprocal instead of a division,
 // and a stage's item decodes its line and column once for all of its points. 1200 points x 3001
-// (16 x 15 x 5, split fp16, 16-bit words): 14.2 us, 2.0 TB/s; the tile kernel with integer
-// divisions per element, copies in and out of LDS and radices 3 and 5 apart took 87.3 us.
+// (16 x 15 x 5, split fp16, 16-bit words; a call on new inputs): 13.9 us, 2.1 TB/s; the tile kernel with
+// integer divisions per element, copies in and out of LDS and radices 3 and 5 apart took 87.5 us.
 #pragma once
 #include "mfft_butterfly.h"
 #include "mfft_fast_impl.h"
@@ -411,9 +411,13 @@ __global__ void __launch_bounds__(kMixThreads, row_waves<PREC>()) fft_mixed(MixA
 // Bound: instruction issue, and segment length (16 lines of 16-bit words are 64 bytes). Tiles
 // of up to 8192 points run 512 threads at 16 points each, two workgroups per compute unit (480
 // x 640 x 18 2D split fp16 39.9 us; 256 threads 44.4, 1024 threads 42.1); longer lines fill the
-// LDS with one workgroup of 1024. 2D execs with both axes on the mixed-radix kernels against an
-// odd pass and a power-of-two pass per axis (us): 480 x 640 x 18 fp32 90 -> 41, split fp16 86 ->
-// 40, 960 x 960 x 16 fp32 177 -> 100, 96 x 96 x 100 split fp16 90 -> 15.
+// LDS with one workgroup of 1024, and tiles of up to 2048 points (narrow transforms, short lines) run
+// 256 threads, more of which are busy (2D, 16-bit intermediates, in us, 512 / 256 threads: 5461 x 48 x
+// 16 54 / 41, in two passes of columns 46; 1000 x 24 x 24 11.1 / 9.2; 5461 x 1000 x 2 104 / 47; 500 x 96
+// x 16 11.2 / 11.0, with 128 threads 11.6). 2D execs with both axes on the mixed-radix kernels against an
+// odd pass and a power-of-two pass per axis (us), execs repeated on the same buffers: 480 x 640 x 18
+// fp32 89 -> 40, split fp16 86 -> 40, 960 x 960 x 16 fp32 164 -> 96, 96 x 96 x 100 split fp16 90 ->
+// 14. On new inputs at every call, which come from memory: 480 x 640 x 18 fp32 95.6 -> 47.4.
 template <int CAP, int PREC, int INF, int OUTF>
 __global__ void __launch_bounds__(mix_col_threads(CAP), 4) fft_mixed_cols(MixColArgs a)
 {
@@ -442,7 +446,7 @@ __global__ void __launch_bounds__(mix_col_threads(CAP), 4) fft_mixed_cols(MixCol
 // Many transforms of uneven length and count in one launch: workgroup b takes tile b, then
 // further tiles from the device-side counter until every tile is handed out. The last
 // workgroup to finish leaves the counter at zero for the next launch. 48 items of 16..4096
-// points (0.33 M points): 9.1 us per call, one launch; copying the job records, resetting the
+// points (0.33 M points): 9.5 us per call, one launch; copying the job records, resetting the
 // counter and 4096-point tiles on the tile kernel took 58 us.
 template <int PREC, int INF, int OUTF>
 __global__ void __launch_bounds__(kMixThreads, 4) fft_mixed_queue(MixQueueArgs a)

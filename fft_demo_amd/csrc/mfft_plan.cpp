@@ -789,7 +789,11 @@ static int finish_passes(mfft_plan_s *p)
         const bool mixed_cols = !is_pow2(ps.R) && ps.ps_in != 1 && mixed_one_pass(p->d.precision, ps.R, ps.ps_in, ps.ps_out, ps.lines);
         if (!p->conv && !ps.small && ps.fast_kind < 0 && !rev && !ps.tw_N && (mixed_cols || (ps.generic && dense_rows(ps)))) {
             const int T = mixed_cols ? mixed_col_lines(ps.R) : 0;
-            ps.mixed_cap = !mixed_cols ? 0 : ps.R * T <= kMixColSmall ? kMixColSmall : kMixColLarge;
+            long long most = T;  // lines a tile has: a narrow transform has fewer
+            if (mixed_cols)
+                for (auto &l : ps.lines)
+                    if (l.in_stride == 1 && l.out_stride == 1 && !l.batch) most = std::min<long long>(T, l.count);
+            ps.mixed_cap = !mixed_cols ? 0 : ps.R * most <= kMixColTiny ? kMixColTiny : ps.R * T <= kMixColSmall ? kMixColSmall : kMixColLarge;
             const void *fn = find_mixed_kernel(p->d.precision, in_fmt, out_fmt, ps.mixed_cap);
             if (fn && mix_schedule(ps.R, p->d.precision, p->d.scale == MFFT_SCALE_STAGE, mixed_order(p->d, in_fmt, ps.R, mixed_cols), ps.mix)) {
                 ps.mixed = true;

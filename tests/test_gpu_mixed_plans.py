@@ -32,12 +32,12 @@ def test_more_workgroups_than_a_launch_takes(dev):
 
     import fft_demo_amd as F
 
-    # one workgroup of 512 threads per transform's columns: 2^23 of them are 2^32 threads; the workspace
+    # one workgroup of 256 threads per transform's columns: 2^24 of them are 2^32 threads; the workspace
     # holds all, so that the batch is not cut into chunks before
-    batch = (1 << 23) + 3
+    batch = (1 << 24) + 3
     base = to_device(complex_input((1024, 48, 2), 5), torch.float16, dev)
     x = base.repeat(batch // 1024 + 1, 1, 1, 1)[:batch].contiguous()
-    with F.Plan((48, 2), batch, precision="split_fp16", workspace_limit=8 << 30) as plan, \
+    with F.Plan((48, 2), batch, precision="split_fp16", workspace_limit=16 << 30) as plan, \
             F.Plan((48, 2), 1024, precision="split_fp16") as one:
         assert plan.info["batch_chunk"] == batch
         y = plan.exec(x)
@@ -106,6 +106,25 @@ def test_reported_passes(dev):
         rows, cols = plan.info["passes"]
         assert rows["kernel"] == "mixed_rows" and rows["lines_per_tile"] * rows["tiles"] >= 240
         assert cols["kernel"] == "mixed_cols" and cols["lines_per_tile"] == 8 and cols["tiles"] == 5 * 38
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp32", "split_fp16", "bf16"])
+@pytest.mark.parametrize("nx,ny,batch", [(48, 16, 1), (48, 16, 700), (60, 32, 3), (60, 34, 3), (68, 32, 3), (1020, 2, 5),
+                                         (1020, 3, 2), (24, 2, 33)])
+def test_columns_of_small_tiles(dev, prec, nx, ny, batch):
+    import torch
+
+    import fft_demo_amd as F
+
+    fmt = {"fp32": "c32", "split_fp16": "c16", "bf16": "cbf16"}[prec]
+    x = complex_input((batch, nx, ny), nx + ny, fmt)
+    with F.Plan((nx, ny), batch, precision=prec) as plan:
+        assert plan.info["passes"][-1]["kernel"] == "mixed_cols"
+        y = from_device(plan.exec(to_device(x, plan.in_dtype(), dev))) / plan.out_scale
+    l2, mx = rel_errors(y, oracle.fft2d(x))
+    tol = {"fp32": (1e-5, 4e-5), "split_fp16": (1e-3, 4e-3), "bf16": (1e-2, 4e-2)}[prec]
+    assert l2 <= tol[0] and mx <= tol[1], (l2, mx)
 
 
 @pytest.mark.gpu
