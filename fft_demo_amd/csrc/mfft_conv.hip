@@ -518,7 +518,7 @@ __global__ void __launch_bounds__(256) pointwise_gi_kernel(const float2 *D, cons
 // ---------------------------------------------------------------- short filters
 // A filter of fh x fw taps, fh far below Ph: its Ph x Pw spectrum is a product of two small DFT
 // matrices, H = Ey w Ex, which one kernel computes straight from the taps instead of a padded
-// plane going through a whole 2D transform. 48 filters of 13 x 13 on 256 x 256: 12.3 us, 2 TB/s of
+// plane going through a whole 2D transform. 48 filters of 13 x 13 on 256 x 256: 12.8 us, 2 TB/s of
 // spectra written (packing, rows and columns took 30.6 us). Up to 32 taps the 2 x 32 products a
 // point stay below the transform's passes over memory. The matrices are tables: ty[ky][y] = W_Ph^(ky y) (rows
 // of NR entries, ky <= Ph / 2) and tx[x][kx] = W_Pw^(x kx), evaluated in FP64 and rounded once.
